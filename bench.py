@@ -253,7 +253,7 @@ def decode_kernel_label(nsplit):
     INT8K_DECODE_BLOCK=0 turns that off."""
     if nsplit <= 16 and os.environ.get("INT8K_DECODE_BLOCK", "1") != "0":
         return "decode_block_kernel (one launch per step)"
-    return "decode_split_kernel + decode_combine_kernel (one step)"
+    return "decode_block_kernel + decode_combine_kernel (one step)"
 
 
 def measure_decode(B, H, D, S, outlier_frac, args, dev, stream, keep_host=False,

@@ -68,7 +68,8 @@ const char* int8k_last_error(void);
 /*                                                                          */
 /* The workspace holds split partials.  Plans of at most 16 chunks per (b,h) */
 /* merge their chunks on chip and need none: the query returns 0 and the    */
-/* call accepts a null workspace for them.                                  */
+/* call accepts a null workspace for them.  Automatic plans above 16 chunks  */
+/* whose (b,h) would also fit that way fall back to it without a workspace.  */
 /* ------------------------------------------------------------------------ */
 size_t int8k_decode_attention_workspace_bytes(int BH, int S, int head_dim, int nsplit);
 
@@ -155,8 +156,8 @@ size_t int8k_decode_attention_paged_workspace_bytes(int B, int H, int max_contex
                                                     int head_dim, int nsplit);
 
 /* Chunks per (b, h) the paged call plans for these arguments (0 if they are
- * invalid).  Plans of up to 8 chunks whose page-id table fits 48 KiB run as
- * one launch; larger ones as a split kernel plus a combine kernel. */
+ * invalid).  They run on blocks of up to 8 waves, one block per (b, h) as one
+ * launch, or several that each leave a partial for a combine kernel. */
 int int8k_decode_attention_paged_num_splits(int B, int H, int max_context, int head_dim,
                                             int nsplit);
 
@@ -170,9 +171,9 @@ int int8k_decode_attention_forward_paged(
 /* Diagnostics of the paged calls: *count receives how many work units, on the
  * current device since the library was loaded, met a page id outside
  * [0, num_pages) among the table entries their positions use (entries past a
- * sequence's length are never read and never counted).  A unit is a (b, h) for
- * plans of up to 8 chunks and a (b, h, chunk) for larger ones, so one bad entry
- * counts at least once per head of its sequence.  Synchronises with the device.
+ * sequence's length are never read and never counted).  A unit is a (b, h), or the
+ * part of one that a block takes, so one bad entry counts at least once per head
+ * of its sequence.  Synchronises with the device.
  * No counterpart in the reference, whose decode has no page table. */
 int int8k_decode_paged_bad_page_ids(unsigned int* count);
 

@@ -21,9 +21,11 @@
 //    row is half a 128-byte line, so groups 2h and 2h+1 take the even and the
 //    odd rows of block rows 8h..8h+7 (slot t: row 8h + o + 2t) and every load
 //    instruction covers whole lines.  That makes non-temporal K/V loads pay
-//    at D=64 too; with half lines per instruction they cost 20-100%.  Each
-//    lane then loads one of its group's four scales and the group reads them
-//    with a DPP quad broadcast.
+//    at D=64 too; with half lines per instruction they cost 20-100%.
+//  * Scales: lane s of a group loads the scales of slots s % 4 (+ 4), one dword
+//    each, and the quad reads them with a DPP broadcast folded into the multiply:
+//    a wave's scale load is 256 contiguous bytes with no alignment beyond a
+//    dword, so odd row strides cost nothing.
 //  * QK: 4 v_dot4_i32_i8 per slot per lane (exact int32), then a DPP sum over
 //    the LPR lanes of the group (no LDS).  The group's lanes all hold the score.
 //  * Softmax: every row-group keeps its own online-softmax state (m, l) in the
@@ -32,10 +34,10 @@
 //    a wave are merged once, at the end of the wave's KV chunk.
 //  * PV: each V byte is converted with one SDWA v_cvt_f32_i32 and folded in
 //    with one FMA: acc += (p_j * sV_j) * v_j.
-//  * Split-KV: a work unit = one wave = one (bh, chunk).  The split count is
-//    chosen on the host so that BH*nsplit waves fill 256 CUs several times
-//    over; partial states (m, l, acc[D]) go to the workspace and a combine
-//    kernel merges them with the log-sum-exp rule into fp16.
+//  * Split-KV: a wave walks one chunk of one (b,h), the up to 8 waves of a block
+//    merge on chip, and where one block per (b,h) would leave CUs idle several
+//    blocks share it: their partial states (m, l, acc[D]) go to the workspace and
+//    a combine kernel merges them with the log-sum-exp rule (plan_groups).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -92,10 +94,14 @@ struct DecodeTuning {
 struct SplitPlan {
     int nsplit;
     int chunk;
+    bool forced;  // the caller's split count
 };
 
+// Most waves (chunks) per block of the one-launch and grouped kernels' fast instance.
+constexpr int kGroupWaves = 8;
+
 // Most chunks per (b,h) that run as one launch (decode_block_kernel: one wave
-// per chunk, merged in LDS); larger plans run the split + combine pair.
+// per chunk, merged in LDS); larger plans run several blocks and the combine.
 constexpr int kMaxBlockSplits = 16;
 // The automatic plan never picks 9..16 chunks: those would run the 16-wave
 // instance (one register set), and 8 chunks on the 8-wave instance (two
@@ -108,11 +114,11 @@ constexpr int kMaxAutoBlockSplits = 8;
 __device__ unsigned int g_paged_bad_ids;
 
 // Largest page-id table the paged one-launch kernel stages in LDS (12288 ids);
-// longer tables run the paged split + combine pair.
+// a block whose rows need more runs decode_paged_kernel + the combine.
 constexpr long long kPagedLdsTableBytes = 48 << 10;
 
 // Plans of at most kMaxBlockSplits chunks run as one launch (decode_block_kernel);
-// INT8K_DECODE_BLOCK=0 keeps them on the split + combine pair (read once).
+// INT8K_DECODE_BLOCK=0 makes them leave partials for the combine kernel (read once).
 bool use_block_kernel() {
     static const bool on = [] {
         const char* e = std::getenv("INT8K_DECODE_BLOCK");
@@ -152,10 +158,48 @@ DecodeTuning tuning_for(int D) {
     return t;
 }
 
+// How the chunks of a (b,h) are laid out on blocks: `blocks` blocks of `waves`
+// waves, each wave `chunk` rows.  The states of a block's waves merge on chip;
+// with more than one block per (b,h) each leaves a partial for
+// decode_combine_kernel.
+struct GroupPlan {
+    int blocks, waves, chunk;
+};
+constexpr int kNumCus = 256;
+
+// Automatic plans of the 8-wave kernels take the blocks per (b,h) (at most `most`)
+// with the smallest cost in wave iterations: a round is one block on each CU,
+// a block costs its waves' iterations plus about 2 for its first loads and its
+// merge, and the second launch about 6 at D = 64 and 2.5 at D = 128 (a CU streams
+// one block at ~55 GB/s: 1.27 and 2.5 us per iteration).  So short sequences stay
+// on one block (paged B4 H16 D64 4000 rows: 15.7 us, 16.4 on four and a combine)
+// and longer ones spread (B1 H12 D64 4096 rows: 13.2 -> 12.3 us on 8 blocks,
+// B1 H8 D128 3000 rows 19.6 -> 12.2, B4 H12 D128 2500 rows 18.4 -> 12.3).
+// Sweeps of 1..32 blocks at 8 to 64 (b,h) put the best time at one full round or
+// within 3% of it (B2 H8 D128 60013 rows: 53.2 / 44.1 / 46.0 us at 8 / 16 / 32
+// blocks; B1 H32 D64 128K: 103 / 87 / 88 us at 4 / 8 / 16): a partial extra round
+// leaves CUs idle, and fewer blocks than CUs read at a CU's ~55 GB/s each.
+GroupPlan plan_groups(int BH, int S, int D, int slots, long long most) {
+    const int R = rows_per_iter(D, slots);
+    const long long iters = ceil_div(S, R);
+    most = std::max(1LL, std::min({most, ceil_div(iters, kGroupWaves),
+                                   std::max(8LL, (long long)kNumCus / BH)}));
+    long long best = -1, per_wave = 0, blocks = 1;
+    for (long long nb = 1; nb <= most; ++nb) {
+        const long long pw = ceil_div(iters, nb * kGroupWaves);
+        const long long bl = ceil_div(iters, pw * kGroupWaves);
+        const long long rounds = ceil_div(BH * bl, kNumCus);
+        const long long cost = 2 * rounds * (pw + 2) + (bl > 1 ? (D == 128 ? 5 : 12) : 0);
+        if (best < 0 || cost < best) best = cost, per_wave = pw, blocks = bl;
+    }
+    const int waves = (int)std::min<long long>(kGroupWaves, ceil_div(iters, per_wave));
+    return GroupPlan{(int)blocks, waves, (int)(per_wave * R)};
+}
+
 // Split-count choice: a unit is one wave over one KV chunk of one (b,h);
 // aim for tuning.target_units units in total, each chunk a multiple of the
 // rows one wave iteration covers.
-SplitPlan plan_splits(int BH, int S, int D, int nsplit_req) {
+SplitPlan plan_splits(int BH, int S, int D, int nsplit_req, bool on_chip = false) {
     const DecodeTuning tn = tuning_for(D);
     const int R = rows_per_iter(D, tn.slots);
     const long long max_split = ceil_div(S, R);
@@ -171,11 +215,26 @@ SplitPlan plan_splits(int BH, int S, int D, int nsplit_req) {
             1, std::max(ceil_div(S, 4LL * R), std::min<long long>(kMaxAutoBlockSplits, ceil_div(S, R))));
         ns = std::min(ns, by_len);
         if (ns > kMaxAutoBlockSplits && ns <= kMaxBlockSplits) ns = kMaxAutoBlockSplits;
+        // Few (b,h): several blocks each, where that pays for the second launch.  nsplit
+        // then only sizes the workspace (above kMaxBlockSplits, so that it is one).
+        if (ns == kMaxAutoBlockSplits && !on_chip && max_split > kMaxBlockSplits) {
+            const GroupPlan g = plan_groups(BH, S, D, tn.slots, max_split);
+            if (g.blocks > 1)
+                ns = std::min(max_split, std::max(3LL, (long long)g.blocks) * kGroupWaves);
+            if (ns > kMaxBlockSplits)
+                return SplitPlan{(int)ns, (int)round_up((size_t)ceil_div(S, ns), (size_t)R), false};
+        }
     }
     ns = std::max<long long>(1, std::min(ns, max_split));
     long long chunk = round_up((size_t)ceil_div(S, ns), (size_t)R);
     ns = ceil_div(S, chunk);
-    return SplitPlan{(int)ns, (int)chunk};
+    return SplitPlan{(int)ns, (int)chunk, nsplit_req > 0};
+}
+
+// A forced plan keeps its chunks, up to kGroupWaves to a block.
+inline GroupPlan forced_groups(const SplitPlan& plan) {
+    const int blocks = (int)ceil_div(plan.nsplit, kGroupWaves);
+    return GroupPlan{blocks, (int)ceil_div(plan.nsplit, blocks), plan.chunk};
 }
 
 struct Int4 {
@@ -230,16 +289,16 @@ __device__ __forceinline__ float quad_bcast(float x, int t) {
 }
 
 // QK^T, online softmax and PV for one wave iteration whose NSLOT rows per
-// group are loaded (kv, vv, sk, sv).  MASKED: rows >= j1 get score -inf and
-// weight 0 (their loads point at some valid row).  RS: rows between slots
-// (2 for paired rows).  QB: sk[0]/sv[0] hold the scale of the lane's own slot
-// (lane s of the 4-lane group: slot s), read by the group with quad_bcast.
-template <int D, int NS, bool MASKED, int RS = 1, bool QB = false>
+// group are loaded (kv, vv, sk, sv).  MASKED: rows outside [jlo, j1) get score -inf
+// and weight 0 (their loads point at some valid row), and sk[t] / sv[t] are slot t's
+// scales.  Otherwise lane s of a quad holds those of slots s, s + 4 in sk[0],
+// sk[1] and the quad reads them with quad_bcast.  RS: rows between slots (2 for
+// paired rows).
+template <int D, int NS, bool MASKED, int RS = 1>
 __device__ __forceinline__ void decode_math(const Int4 (&kv)[NS], const Int4 (&vv)[NS],
                                             const float (&sk)[NS], const float (&sv)[NS],
                                             int row0, int j1, const Int4& q, float qscale,
-                                            float& m, float& l, float* acc) {
-    static_assert(!QB || (NS == 4 && D == 64), "quad broadcast: one scale per lane of a group");
+                                            float& m, float& l, float* acc, int jlo = 0) {
     // QK^T: exact int32 dot per row, summed over the LPR lanes of the group.
     float sc[NS];
 #pragma unroll
@@ -249,10 +308,10 @@ __device__ __forceinline__ void decode_math(const Int4 (&kv)[NS], const Int4 (&v
         d = __builtin_amdgcn_sdot4(q.z, kv[t].z, d, false);
         d = __builtin_amdgcn_sdot4(q.w, kv[t].w, d, false);
         d = group_sum<D>(d);
-        const float skt = QB ? quad_bcast(sk[0], t) : sk[t];
+        const float skt = MASKED ? sk[t] : quad_bcast(sk[t >> 2], t & 3);
         sc[t] = static_cast<float>(d) * qscale * skt;
         if constexpr (MASKED) {
-            if (row0 + t * RS >= j1) sc[t] = -INFINITY;
+            if (row0 + t * RS >= j1 || row0 + t * RS < jlo) sc[t] = -INFINITY;
         }
     }
 
@@ -270,9 +329,9 @@ __device__ __forceinline__ void decode_math(const Int4 (&kv)[NS], const Int4 (&v
     for (int t = 0; t < NS; ++t) {
         const float p = fast_exp2(sc[t] - m_use);
         l += p;
-        float w = p * (QB ? quad_bcast(sv[0], t) : sv[t]);
+        float w = p * (MASKED ? sv[t] : quad_bcast(sv[t >> 2], t & 3));
         if constexpr (MASKED) {
-            if (row0 + t * RS >= j1) w = 0.f;
+            if (row0 + t * RS >= j1 || row0 + t * RS < jlo) w = 0.f;
         }
         fma_bytes(acc + 0, vv[t].x, w);
         fma_bytes(acc + 4, vv[t].y, w);
@@ -282,7 +341,8 @@ __device__ __forceinline__ void decode_math(const Int4 (&kv)[NS], const Int4 (&v
     m = m_new;
 }
 
-// The registers of one wave iteration: NSLOT rows per group of K, V and scales.
+// The registers of one wave iteration: NSLOT rows per group of K, V and scales
+// (the scales of this lane's slots; see decode_math).
 template <int NS>
 struct IterBuf {
     Int4 kv[NS], vv[NS];
@@ -290,9 +350,8 @@ struct IterBuf {
 };
 
 // The loads of an unmasked wave iteration whose group rows start at row0 and
-// lie RS rows apart.  Paired rows with vector-capable scales (RS == 2 and
-// VEC_SCALES) load one scale per lane, slot `sub` (decode_math's QB).
-template <int D, int NS, bool VEC_SCALES, int FL, int RS = 1>
+// lie RS rows apart.
+template <int D, int NS, int FL, int RS = 1>
 __device__ __forceinline__ void load_iter(IterBuf<NS>& b, const int8_t* __restrict__ Kbh,
                                           const int8_t* __restrict__ Vbh,
                                           const float* __restrict__ sKbh,
@@ -303,58 +362,33 @@ __device__ __forceinline__ void load_iter(IterBuf<NS>& b, const int8_t* __restri
     for (int t = 0; t < NS; ++t) b.kv[t] = load_kv16<(FL & kNtKV) != 0>(kp + t * RS * D);
 #pragma unroll
     for (int t = 0; t < NS; ++t) b.vv[t] = load_kv16<(FL & kNtKV) != 0>(vp + t * RS * D);
-    if constexpr (VEC_SCALES && RS == 2) {
-        b.sk[0] = load_f32<(FL & kNtScales) != 0>(sKbh + row0 + 2 * sub);
-        b.sv[0] = load_f32<(FL & kNtScales) != 0>(sVbh + row0 + 2 * sub);
-    } else if constexpr (VEC_SCALES) {
 #pragma unroll
-        for (int t = 0; t < NS; t += 4) {
-            typedef float v4f __attribute__((ext_vector_type(4)));
-            v4f a, c;
-            if constexpr ((FL & kNtScales) != 0) {
-                a = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(sKbh + row0 + t));
-                c = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(sVbh + row0 + t));
-            } else {
-                a = *reinterpret_cast<const v4f*>(sKbh + row0 + t);
-                c = *reinterpret_cast<const v4f*>(sVbh + row0 + t);
-            }
-            b.sk[t] = a.x; b.sk[t + 1] = a.y; b.sk[t + 2] = a.z; b.sk[t + 3] = a.w;
-            b.sv[t] = c.x; b.sv[t + 1] = c.y; b.sv[t + 2] = c.z; b.sv[t + 3] = c.w;
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < NS; ++t) {
-            b.sk[t] = load_f32<(FL & kNtScales) != 0>(sKbh + row0 + t * RS);
-            b.sv[t] = load_f32<(FL & kNtScales) != 0>(sVbh + row0 + t * RS);
-        }
+    for (int i = 0; i < NS / 4; ++i) {
+        const size_t r = row0 + RS * ((sub & 3) + 4 * i);
+        b.sk[i] = load_f32<(FL & kNtScales) != 0>(sKbh + r);
+        b.sv[i] = load_f32<(FL & kNtScales) != 0>(sVbh + r);
     }
 }
 
-// One wave iteration over NSLOT rows per group.  MASKED handles the last
-// partial block of a chunk: rows >= j1 get score -inf and weight 0 (their
-// loads are redirected to row j1-1, which is in bounds).  RS: rows between
-// slots (2 for paired rows).
-template <int D, int NS, bool MASKED, bool VEC_SCALES, int FL, int RS = 1>
-__device__ __forceinline__ void decode_iter(
+// A partial wave iteration: rows outside [jlo, j1) get score -inf and weight 0
+// (their loads are redirected to a row inside).  RS: rows between slots (2 for
+// paired rows).
+template <int D, int NS, int FL, int RS = 1>
+__device__ __forceinline__ void decode_tail(
     const int8_t* __restrict__ Kbh, const int8_t* __restrict__ Vbh,
     const float* __restrict__ sKbh, const float* __restrict__ sVbh,
-    int row0, int j1, int sub, const Int4& q, float qscale,
+    int row0, int jlo, int j1, int sub, const Int4& q, float qscale,
     float& m, float& l, float* acc) {
     IterBuf<NS> b;
-    if constexpr (!MASKED) {
-        load_iter<D, NS, VEC_SCALES, FL, RS>(b, Kbh, Vbh, sKbh, sVbh, row0, sub);
-    } else {
 #pragma unroll
-        for (int t = 0; t < NS; ++t) {
-            const int r = min(row0 + t * RS, j1 - 1);
-            b.kv[t] = load_kv16<(FL & kNtKV) != 0>(Kbh + (size_t)r * D + sub * 16);
-            b.vv[t] = load_kv16<(FL & kNtKV) != 0>(Vbh + (size_t)r * D + sub * 16);
-            b.sk[t] = load_f32<(FL & kNtScales) != 0>(sKbh + r);
-            b.sv[t] = load_f32<(FL & kNtScales) != 0>(sVbh + r);
-        }
+    for (int t = 0; t < NS; ++t) {
+        const int r = max(min(row0 + t * RS, j1 - 1), jlo);
+        b.kv[t] = load_kv16<(FL & kNtKV) != 0>(Kbh + (size_t)r * D + sub * 16);
+        b.vv[t] = load_kv16<(FL & kNtKV) != 0>(Vbh + (size_t)r * D + sub * 16);
+        b.sk[t] = load_f32<(FL & kNtScales) != 0>(sKbh + r);
+        b.sv[t] = load_f32<(FL & kNtScales) != 0>(sVbh + r);
     }
-    decode_math<D, NS, MASKED, RS, (!MASKED && VEC_SCALES && RS == 2)>(
-        b.kv, b.vv, b.sk, b.sv, row0, j1, q, qscale, m, l, acc);
+    decode_math<D, NS, true, RS>(b.kv, b.vv, b.sk, b.sv, row0, j1, q, qscale, m, l, acc, jlo);
 }
 
 // Merges the G row-group states of a wave (lanes with equal `sub`) and writes
@@ -406,59 +440,6 @@ __device__ __forceinline__ void finish_unit(float m, float l, float* acc, int gr
     }
 }
 
-// Pass 1: one wave per (bh, split); writes the unnormalised partial state,
-// or — when the KV sequence is not split (FINAL) — the fp16 output itself.
-template <int D, int NS, bool VEC_SCALES, bool FINAL, int FL>
-__global__ __launch_bounds__(kBlockThreads) void decode_split_kernel(
-    const int8_t* __restrict__ Q, const int8_t* __restrict__ K,
-    const int8_t* __restrict__ V, const float* __restrict__ sQ,
-    const float* __restrict__ sK, const float* __restrict__ sV,
-    float* __restrict__ part_ml, float* __restrict__ part_acc, uint16_t* __restrict__ out,
-    int S, int S_cap, int nsplit, int chunk, int units, float qk_scale_log2, int stagger) {
-    using G = DecodeGeom<D, NS>;
-    const int lane = threadIdx.x & 63;
-    const int unit = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-    if (unit >= units) return;  // whole wave exits; no block barrier below
-    const int bh = unit / nsplit;
-    const int sp = unit - bh * nsplit;
-    const int j0 = sp * chunk;
-    const int j1 = min(S, j0 + chunk);
-
-    const int sub = lane % G::kLanesPerRow;
-    const int grp = lane / G::kLanesPerRow;
-
-    const Int4 q = load16(Q + (size_t)bh * D + sub * 16);
-    const float qscale = sQ[bh] * qk_scale_log2;
-
-    // (b,h) rows sit S_cap apart (the cache capacity); the first S are valid
-    const int8_t* Kbh = K + (size_t)bh * S_cap * D;
-    const int8_t* Vbh = V + (size_t)bh * S_cap * D;
-    const float* sKbh = sK + (size_t)bh * S_cap;
-    const float* sVbh = sV + (size_t)bh * S_cap;
-
-    float m = -INFINITY, l = 0.f;
-    float acc[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-
-    // Full iterations, optionally started at a unit-dependent rotation so that
-    // concurrent waves do not walk identical address offsets in lockstep.
-    const int n_full = (j1 - j0) / G::kRowsPerIter;
-    int it = stagger ? (int)(((unsigned)unit * 2654435761u) >> 16) % max(n_full, 1) : 0;
-    for (int k = 0; k < n_full; ++k) {
-        decode_iter<D, NS, false, VEC_SCALES, FL>(Kbh, Vbh, sKbh, sVbh,
-                                                  j0 + it * G::kRowsPerIter + grp * NS, j1, sub,
-                                                  q, qscale, m, l, acc);
-        it = (it + 1 == n_full) ? 0 : it + 1;
-    }
-    const int base = j0 + n_full * G::kRowsPerIter;
-    if (base < j1)
-        decode_iter<D, NS, true, VEC_SCALES, FL>(Kbh, Vbh, sKbh, sVbh, base + grp * NS, j1, sub,
-                                                 q, qscale, m, l, acc);
-
-    finish_unit<D, FINAL>(m, l, acc, grp, sub, unit, part_ml, part_acc, out);
-}
-
 // The output row of one (b,h) from the merged accumulator (dims lane*D/64 ..
 // +D/64 of this lane) and the merged sum L: the fp16 row, or with qout set the
 // per-token int8 quantization of that fp16 row (codes and scale as
@@ -490,41 +471,50 @@ __device__ __forceinline__ void emit_row(const float (&acc)[D / 64], float L, in
         out[(size_t)bh * D + lane * DPL + i] = __half_as_ushort(__float2half_rn(y[i]));
 }
 
-// Pass 2: one wave per bh merges its nsplit partial states into the output row.
+// Pass 2: one block per bh merges its n partial states into the output row.
+// The partials come from other XCDs' writes (a full memory round trip each), so
+// the block's 4 waves take every fourth partial, 8 loads in flight per wave, and
+// merge in LDS: at n = 235 one wave alone took 15.2 us.
 template <int D>
 __global__ __launch_bounds__(kBlockThreads) void decode_combine_kernel(
     const float* __restrict__ part_ml, const float* __restrict__ part_acc,
-    uint16_t* __restrict__ out, int8_t* __restrict__ qout, float* __restrict__ qscale, int BH,
-    int nsplit) {
+    uint16_t* __restrict__ out, int8_t* __restrict__ qout, float* __restrict__ qscale, int n) {
     constexpr int DPL = D / 64;  // dims per lane
+    __shared__ float s_acc[kWavesPerBlock][D];
     const int lane = threadIdx.x & 63;
-    const int bh = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-    if (bh >= BH) return;
-    const float* ml = part_ml + 2 * (size_t)bh * nsplit;
+    const int w = threadIdx.x >> 6;
+    const int bh = blockIdx.x;
+    const float2* ml = reinterpret_cast<const float2*>(part_ml) + (size_t)bh * n;
 
     float M = -INFINITY;
-    for (int s = lane; s < nsplit; s += 64) M = fmaxf(M, ml[2 * s]);
+    for (int s = lane; s < n; s += 64) M = fmaxf(M, ml[s].x);
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
     const float M_use = (M == -INFINITY) ? 0.f : M;
 
     float L = 0.f;
-    for (int s = lane; s < nsplit; s += 64) L += ml[2 * s + 1] * fast_exp2(ml[2 * s] - M_use);
+    for (int s = lane; s < n; s += 64) L += ml[s].y * fast_exp2(ml[s].x - M_use);
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) L += __shfl_xor(L, off);
 
     float acc[DPL];
 #pragma unroll
     for (int i = 0; i < DPL; ++i) acc[i] = 0.f;
-    const float* pa = part_acc + (size_t)bh * nsplit * D + lane * DPL;
-    // unrolled so the partial rows of several splits are loaded together (they
-    // come from other XCDs' writes, a full memory round trip each)
+    const float* pa = part_acc + (size_t)bh * n * D + lane * DPL;
 #pragma unroll 8
-    for (int s = 0; s < nsplit; ++s) {
-        const float w = fast_exp2(ml[2 * s] - M_use);
+    for (int s = w; s < n; s += kWavesPerBlock) {
+        const float wt = fast_exp2(ml[s].x - M_use);
 #pragma unroll
-        for (int i = 0; i < DPL; ++i) acc[i] = fmaf(pa[(size_t)s * D + i], w, acc[i]);
+        for (int i = 0; i < DPL; ++i) acc[i] = fmaf(pa[(size_t)s * D + i], wt, acc[i]);
     }
+#pragma unroll
+    for (int i = 0; i < DPL; ++i) s_acc[w][lane * DPL + i] = acc[i];
+    __syncthreads();
+    if (w != 0) return;
+#pragma unroll
+    for (int i = 0; i < DPL; ++i)
+#pragma unroll
+        for (int v = 1; v < kWavesPerBlock; ++v) acc[i] += s_acc[v][lane * DPL + i];
     emit_row<D>(acc, L, lane, bh, out, qout, qscale);
 }
 
@@ -533,20 +523,19 @@ __global__ __launch_bounds__(kBlockThreads) void decode_combine_kernel(
 // group's first row in iteration i; RS: rows between its slots.  PIPE: two
 // register sets, iteration k+1's loads issued before iteration k is computed
 // (the fences keep the compiler from sinking them).
-template <int D, int NS, bool VEC_SCALES, int FL, bool PIPE, int RS, typename RowOff>
+template <int D, int NS, int FL, bool PIPE, int RS, typename RowOff>
 __device__ __forceinline__ void walk_iters(const int8_t* __restrict__ K,
                                            const int8_t* __restrict__ V,
                                            const float* __restrict__ sK,
                                            const float* __restrict__ sV, RowOff roff, int n_full,
                                            int it, int sub, const Int4& q, float qscale, float& m,
                                            float& l, float* acc) {
-    constexpr bool QB = VEC_SCALES && RS == 2;
     auto nxt = [&](int i) { return (i + 1 == n_full) ? 0 : i + 1; };
     auto load = [&](IterBuf<NS>& b, int i) {
-        load_iter<D, NS, VEC_SCALES, FL, RS>(b, K, V, sK, sV, roff(i), sub);
+        load_iter<D, NS, FL, RS>(b, K, V, sK, sV, roff(i), sub);
     };
     auto math = [&](const IterBuf<NS>& b) {
-        decode_math<D, NS, false, RS, QB>(b.kv, b.vv, b.sk, b.sv, 0, 0, q, qscale, m, l, acc);
+        decode_math<D, NS, false, RS>(b.kv, b.vv, b.sk, b.sv, 0, 0, q, qscale, m, l, acc);
     };
     if constexpr (PIPE) {
         IterBuf<NS> ba, bb;
@@ -582,15 +571,18 @@ __device__ __forceinline__ void walk_iters(const int8_t* __restrict__ K,
 
 // The end of a one-launch block: each wave merges its row groups (lanes with
 // equal `sub`) and leaves (M, L, acc[D]) in LDS; wave 0 merges the nw chunk
-// states with the log-sum-exp rule, as decode_combine_kernel, and writes the
-// row.  Every wave of the block calls it (it holds the block's barrier).
+// states with the log-sum-exp rule, as decode_combine_kernel, and writes row
+// `bh`, or with part_ml set the merged state as partial `bh`.  Every wave of
+// the block calls it (it holds the block's barrier).
 template <int D, int MAXW>
 __device__ __forceinline__ void merge_block(float m, float l, float* acc, int lane, int grp,
                                             int sub, int w, int nw, int bh,
                                             float (&s_ml)[MAXW][2], float (&s_acc)[MAXW][D],
                                             uint16_t* __restrict__ out,
                                             int8_t* __restrict__ qout,
-                                            float* __restrict__ qscale) {
+                                            float* __restrict__ qscale,
+                                            float* __restrict__ part_ml = nullptr,
+                                            float* __restrict__ part_acc = nullptr) {
     constexpr int LPR = D / 16;
     float M = m;
 #pragma unroll
@@ -632,28 +624,45 @@ __device__ __forceinline__ void merge_block(float m, float l, float* acc, int la
 #pragma unroll
         for (int i = 0; i < DPL; ++i) o[i] = fmaf(s_acc[c][lane * DPL + i], wt, o[i]);
     }
+    if (part_ml != nullptr) {
+#pragma unroll
+        for (int i = 0; i < DPL; ++i) part_acc[(size_t)bh * D + lane * DPL + i] = o[i];
+        if (lane == 0) {
+            part_ml[2 * (size_t)bh] = Mall;
+            part_ml[2 * (size_t)bh + 1] = L;
+        }
+        return;
+    }
     emit_row<D>(o, L, lane, bh, out, qout, qscale);
 }
 
 // One launch for plans of at most kMaxBlockSplits chunks per (b,h): block bh
 // runs one wave per chunk (blockDim.x / 64 waves), each wave walks its chunk as
-// the split kernel does, merges its row groups and leaves (m, l, acc[D]) in
+// above, merges its row groups and leaves (m, l, acc[D]) in
 // LDS; wave 0 then merges the chunks with the log-sum-exp rule and writes the
 // row.  No partial state leaves the chip and there is no second launch.
 // MAXW: the most waves the instance is launched with (8 or kMaxBlockSplits).
 // The 8-wave instance has twice the registers per wave, which lets it keep the
 // next iteration's loads in flight (a second register set, two_sets) while the
 // current one computes: at 4 slots a short chunk is only a few dependent load
-// rounds, so their latency would show; at D = 128 with 8 slots (204 VGPRs, two
+// rounds, so their latency would show; at D = 128 with 8 slots (184 VGPRs, two
 // waves per SIMD) the stream then runs at fewer waves per CU with the same
 // bytes in flight, which the HBM read rate prefers.
-template <int D, int NS, bool VEC_SCALES, int FL, int MAXW>
+//
+// GROUP (plans of more than kMaxBlockSplits chunks): nb blocks per (b,h), block
+// bh * nb + g taking chunks g * waves .. of the (b,h) and leaving their merged
+// state as one partial for decode_combine_kernel.  Few (b,h) with long contexts
+// run here: against one wave per partial (one register set, grouped rows, 235
+// partials per (b,h)) B2 H8 D128 60013 rows of a 64K cache took 60.4 ->
+// 43.8 us.
+template <int D, int NS, int FL, int MAXW, bool GROUP>
 __global__ __launch_bounds__(64 * MAXW) void decode_block_kernel(
     const int8_t* __restrict__ Q, const int8_t* __restrict__ K,
     const int8_t* __restrict__ V, const float* __restrict__ sQ,
     const float* __restrict__ sK, const float* __restrict__ sV, uint16_t* __restrict__ out,
     int8_t* __restrict__ qout, float* __restrict__ qscale, int S, int S_cap, int chunk,
-    float qk_scale_log2, int stagger) {
+    float qk_scale_log2, int stagger, int nb, float* __restrict__ part_ml,
+    float* __restrict__ part_acc) {
     using G = DecodeGeom<D, NS>;
     constexpr int LPR = D / 16;
     __shared__ float s_ml[MAXW][2];
@@ -661,53 +670,75 @@ __global__ __launch_bounds__(64 * MAXW) void decode_block_kernel(
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int nw = blockDim.x >> 6;
-    const int bh = blockIdx.x;
-    const int j0 = w * chunk;
-    const int j1 = min(S, j0 + chunk);
+    const int bh = GROUP ? (int)(blockIdx.x / (unsigned)nb) : (int)blockIdx.x;
+    const int c = GROUP ? ((int)blockIdx.x - bh * nb) * nw + w : w;  // chunk of this wave
     const int sub = lane % LPR;
     const int grp = lane / LPR;
+    constexpr bool PAIRED = paired_rows(D, NS, MAXW);
+    constexpr int RS = PAIRED ? 2 : 1;
 
     const Int4 q = load16(Q + (size_t)bh * D + sub * 16);
     const float qscale_l = sQ[bh] * qk_scale_log2;
-    const int8_t* Kbh = K + (size_t)bh * S_cap * D;
-    const int8_t* Vbh = V + (size_t)bh * S_cap * D;
-    const float* sKbh = sK + (size_t)bh * S_cap;
-    const float* sVbh = sV + (size_t)bh * S_cap;
+    // Paired rows need the block rows 8h.. to start on a 128-byte line.  Where an odd
+    // row stride puts the (b,h)'s first 64-byte row in the middle of one, rows are
+    // counted from the row before it (jlo = 1: that row, the last of the previous
+    // (b,h), is never used), and the last chunk may run one row past its length.
+    const size_t row_bh = (size_t)bh * S_cap;
+    const int jlo =
+        PAIRED && bh > 0 ? (int)((reinterpret_cast<uintptr_t>(K + row_bh * D) >> 6) & 1) : 0;
+    const int8_t* Kbh = K + (row_bh - jlo) * D;
+    const int8_t* Vbh = V + (row_bh - jlo) * D;
+    const float* sKbh = sK + (row_bh - jlo);
+    const float* sVbh = sV + (row_bh - jlo);
+    const int end = S + jlo;
+    const int j0 = (int)min((long long)c * chunk, (long long)end);
+    const bool last = c == nb * nw - 1;
+    const int j1 = last ? end : min(end - j0, chunk) + j0;
 
     float m = -INFINITY, l = 0.f;
     float acc[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    const int n_full = max(0, j1 - j0) / G::kRowsPerIter;
-    const unsigned unit = (unsigned)bh * (unsigned)nw + (unsigned)w;
-    const int it = stagger ? (int)((unit * 2654435761u) >> 16) % max(n_full, 1) : 0;
-    constexpr bool PAIRED = paired_rows(D, NS, MAXW);
-    constexpr int RS = PAIRED ? 2 : 1;
     const int g0 = group_row0<PAIRED, NS>(grp);
-    walk_iters<D, NS, VEC_SCALES, FL, two_sets(D, NS, MAXW), RS>(
-        Kbh, Vbh, sKbh, sVbh, [&](int i) { return (size_t)(j0 + i * G::kRowsPerIter + g0); },
+    // the first iteration of a (b,h) counted from the row before it is partial
+    const int head = (PAIRED && c == 0 && jlo != 0) ? min(G::kRowsPerIter, j1) : 0;
+    const int n_full = max(0, j1 - j0 - head) / G::kRowsPerIter;
+    const unsigned unit = blockIdx.x * (unsigned)nw + (unsigned)w;
+    const int it = stagger ? (int)((unit * 2654435761u) >> 16) % max(n_full, 1) : 0;
+    const int jf = j0 + head;
+    walk_iters<D, NS, FL, two_sets(D, NS, MAXW), RS>(
+        Kbh, Vbh, sKbh, sVbh, [&](int i) { return (size_t)(jf + i * G::kRowsPerIter + g0); },
         n_full, it, sub, q, qscale_l, m, l, acc);
-    const int base = j0 + n_full * G::kRowsPerIter;
-    if (base < j1)
-        decode_iter<D, NS, true, VEC_SCALES, FL, RS>(Kbh, Vbh, sKbh, sVbh, base + g0, j1, sub,
-                                                     q, qscale_l, m, l, acc);
-    merge_block<D, MAXW>(m, l, acc, lane, grp, sub, w, nw, bh, s_ml, s_acc, out, qout, qscale);
+    // partial iterations: the end of the chunk, and the head
+    int base = jf + n_full * G::kRowsPerIter, stop = j1;
+    for (int part = 0; part < 2; ++part) {
+        if (base < stop)
+            decode_tail<D, NS, FL, RS>(Kbh, Vbh, sKbh, sVbh, base + g0, jlo, stop, sub, q,
+                                       qscale_l, m, l, acc);
+        if (!PAIRED || head == 0) break;
+        base = 0;
+        stop = head;
+    }
+    merge_block<D, MAXW>(m, l, acc, lane, grp, sub, w, nw, GROUP ? (int)blockIdx.x : bh, s_ml,
+                         s_acc, out, qout, qscale, GROUP ? part_ml : nullptr, part_acc);
 }
 
-// Paged one-launch variant for plans of up to 8 chunks per (b,h): the block
-// of (b,h) first copies sequence b's page ids (the first n_tab, clamped to
-// [0, num_pages) as in decode_paged_kernel) into LDS, so that each
-// iteration's row offset is an LDS read instead of a global load in front of
-// its K/V loads; then it walks and merges its chunks as decode_block_kernel.
-template <int D, int NS, bool VEC_SCALES, int FL, int MAXW>
+// Paged variant of decode_block_kernel: a block first copies the page ids of
+// its rows (clamped to [0, num_pages)) into LDS, so that each iteration's row
+// offset is an LDS read instead of a global load in front of its K/V loads; then
+// it walks and merges its chunks as decode_block_kernel.  GROUP: nb blocks per
+// (b,h), the (b,h) index fastest in the grid; a block past the end of its
+// sequence leaves an empty partial.  n_tab: page ids a block's rows can span.
+template <int D, int NS, int FL, int MAXW, bool GROUP>
 __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
     const int8_t* __restrict__ Q, const int8_t* __restrict__ Kp,
     const int8_t* __restrict__ Vp, const float* __restrict__ sQ,
     const float* __restrict__ sKp, const float* __restrict__ sVp,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ context_lens,
-    uint16_t* __restrict__ out, int8_t* __restrict__ qout, float* __restrict__ qscale, int H,
-    int num_pages, int log2_page, int max_pages, int n_tab, int chunk, float qk_scale_log2,
-    int stagger) {
+    uint16_t* __restrict__ out, int8_t* __restrict__ qout, float* __restrict__ qscale, int BH,
+    int H, int num_pages, int log2_page, int max_pages, int n_tab, int chunk,
+    float qk_scale_log2, int stagger, int nb, float* __restrict__ part_ml,
+    float* __restrict__ part_acc) {
     using G = DecodeGeom<D, NS>;
     constexpr int LPR = D / 16;
     extern __shared__ int s_pages[];
@@ -716,13 +747,14 @@ __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int nw = blockDim.x >> 6;
+    const int g = GROUP ? (int)(blockIdx.x / (unsigned)BH) : 0;
+    int bh = (int)blockIdx.x - g * BH;
     // With 16-token pages a head's scales in a page are 64 bytes, and heads 2k
     // and 2k+1 share one 128-byte line.  Blocks go to the 8 XCDs in turn, so
-    // with 16 | gridDim.x block i of XCD x takes head pair 8 (i / 2) + x: the
+    // with 16 | BH block i of XCD x takes head pair 8 (i / 2) + x: the
     // pair's two heads run at adjacent slots of one XCD (one L2) and walk their
     // pages in the same order (one stagger), and the line is fetched once.
-    const bool pair = log2_page < 5 && (gridDim.x & 15) == 0;
-    int bh = blockIdx.x;
+    const bool pair = log2_page < 5 && (BH & 15) == 0;
     if (pair) {
         const int x = bh & 7, i = bh >> 3;
         bh = ((((i >> 1) << 3) + x) << 1) + (i & 1);
@@ -730,25 +762,31 @@ __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
     const int b = bh / H, hh = bh - b * H;
     const int page = 1 << log2_page;
     const int32_t* table = block_tables + (size_t)b * max_pages;
-    const int len = min(context_lens[b], n_tab << log2_page);
-    const int used = (len + page - 1) >> log2_page;  // entries past it are never read
-    bool bad = false;
-    for (int i = threadIdx.x; i < n_tab; i += blockDim.x) {
-        const int id = table[i];
-        bad |= i < used && (unsigned)id >= (unsigned)num_pages;
-        s_pages[i] = (int)min((unsigned)id, (unsigned)(num_pages - 1));
-    }
-    if (__syncthreads_or(bad) && threadIdx.x == 0)
-        __hip_atomic_fetch_add(&g_paged_bad_ids, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int j0 = w * chunk;
-    const int j1 = min(len, j0 + chunk);
+    const long long c0 = (long long)g * nw;  // first chunk of the block
+    const int p0 = GROUP ? (int)min(c0 * chunk >> log2_page, (long long)max_pages) : 0;
+    // the first id of every thread and the query go out beside the length's load
+    const int t = (int)threadIdx.x, nt = (int)blockDim.x;
+    int id = table[min(p0 + min(t, n_tab - 1), max_pages - 1)];
     const int sub = lane % LPR;
     const int grp = lane / LPR;
     const Int4 q = load16(Q + (size_t)bh * D + sub * 16);
     const float qscale_l = sQ[bh] * qk_scale_log2;
+    const int len =
+        (int)min((long long)context_lens[b], (long long)max_pages << log2_page);
+    const int used = min(((len + page - 1) >> log2_page) - p0, n_tab);  // entries past it: not used
+    bool bad = false;
+    for (int i = t; i < used; i += nt) {
+        if (i != t) id = table[p0 + i];
+        bad |= (unsigned)id >= (unsigned)num_pages;
+        s_pages[i] = (int)min((unsigned)id, (unsigned)(num_pages - 1));
+    }
+    if (__syncthreads_or(bad) && threadIdx.x == 0)
+        __hip_atomic_fetch_add(&g_paged_bad_ids, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int j0 = (int)min((c0 + w) * chunk, (long long)max(len, 0));
+    const int j1 = min(len - j0, chunk) + j0;
     // row offset (in rows of the page arrays) of position r of this head
     auto row_off = [&](int r) -> size_t {
-        return ((size_t)s_pages[r >> log2_page] * H + hh) * page + (r & (page - 1));
+        return ((size_t)s_pages[(r >> log2_page) - p0] * H + hh) * page + (r & (page - 1));
     };
 
     float m = -INFINITY, l = 0.f;
@@ -756,13 +794,15 @@ __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.f;
     const int n_full = max(0, j1 - j0) / G::kRowsPerIter;
-    const unsigned unit = (unsigned)(pair ? bh >> 1 : bh) * (unsigned)nw + (unsigned)w;
+    const unsigned unit =
+        ((unsigned)(pair ? bh >> 1 : bh) * (GROUP ? (unsigned)nb : 1u) + (unsigned)g) *
+            (unsigned)nw + (unsigned)w;
     const int it = stagger ? (int)((unit * 2654435761u) >> 16) % max(n_full, 1) : 0;
     // a group's rows (NS-aligned, or the 8-aligned pair block) share one page
     constexpr bool PAIRED = paired_rows(D, NS, MAXW);
     constexpr int RS = PAIRED ? 2 : 1;
     const int g0 = group_row0<PAIRED, NS>(grp);
-    walk_iters<D, NS, VEC_SCALES, FL, two_sets(D, NS, MAXW), RS>(
+    walk_iters<D, NS, FL, two_sets(D, NS, MAXW), RS>(
         Kp, Vp, sKp, sVp, [&](int i) { return row_off(j0 + i * G::kRowsPerIter + g0); },
         n_full, it, sub, q, qscale_l, m, l, acc);
     const int base = j0 + n_full * G::kRowsPerIter;
@@ -780,7 +820,8 @@ __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
         decode_math<D, NS, true, RS>(bt.kv, bt.vv, bt.sk, bt.sv, row0, j1, q, qscale_l, m, l,
                                      acc);
     }
-    merge_block<D, MAXW>(m, l, acc, lane, grp, sub, w, nw, bh, s_ml, s_acc, out, qout, qscale);
+    merge_block<D, MAXW>(m, l, acc, lane, grp, sub, w, nw, GROUP ? bh * nb + g : bh, s_ml, s_acc,
+                         out, qout, qscale, GROUP ? part_ml : nullptr, part_acc);
 }
 
 // Paged variant of pass 1.  Unit = (b, h, split) as above, over positions
@@ -790,9 +831,7 @@ __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
 // slot offsets as the contiguous kernel.  Page p of head h holds
 // K/V [p][h][page_size][D] and scales [p][h][page_size].  FL: the
 // non-temporal load flags of the contiguous kernel's tuning for this D.
-// VEC_SCALES: a group's NS scales load as 16-byte vectors (its rows are
-// NS-aligned inside one page; needs 16-byte aligned scale arrays).
-template <int D, int NS, bool FINAL, int FL, bool VEC_SCALES>
+template <int D, int NS, bool FINAL, int FL>
 __global__ __launch_bounds__(kBlockThreads) void decode_paged_kernel(
     const int8_t* __restrict__ Q, const int8_t* __restrict__ Kp,
     const int8_t* __restrict__ Vp, const float* __restrict__ sQ,
@@ -839,41 +878,12 @@ __global__ __launch_bounds__(kBlockThreads) void decode_paged_kernel(
     int it = stagger ? (int)(((unsigned)unit * 2654435761u) >> 16) % max(n_full, 1) : 0;
     size_t r_next = n_full > 0 ? row_off(j0 + it * G::kRowsPerIter + grp * NS) : 0;
     for (int k = 0; k < n_full; ++k) {
-        const int row0 = j0 + it * G::kRowsPerIter + grp * NS;
         const size_t r0 = r_next;
         it = (it + 1 == n_full) ? 0 : it + 1;
         if (k + 1 < n_full) r_next = row_off(j0 + it * G::kRowsPerIter + grp * NS);
-        const int8_t* kp = Kp + r0 * D + sub * 16;
-        const int8_t* vp = Vp + r0 * D + sub * 16;
-        Int4 kv[NS], vv[NS];
-        float sk[NS], sv[NS];
-#pragma unroll
-        for (int t = 0; t < NS; ++t) kv[t] = load_kv16<(FL & kNtKV) != 0>(kp + t * D);
-#pragma unroll
-        for (int t = 0; t < NS; ++t) vv[t] = load_kv16<(FL & kNtKV) != 0>(vp + t * D);
-        if constexpr (VEC_SCALES) {
-#pragma unroll
-            for (int t = 0; t < NS; t += 4) {
-                typedef float v4f __attribute__((ext_vector_type(4)));
-                v4f a, b;
-                if constexpr ((FL & kNtScales) != 0) {
-                    a = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(sKp + r0 + t));
-                    b = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(sVp + r0 + t));
-                } else {
-                    a = *reinterpret_cast<const v4f*>(sKp + r0 + t);
-                    b = *reinterpret_cast<const v4f*>(sVp + r0 + t);
-                }
-                sk[t] = a.x; sk[t + 1] = a.y; sk[t + 2] = a.z; sk[t + 3] = a.w;
-                sv[t] = b.x; sv[t + 1] = b.y; sv[t + 2] = b.z; sv[t + 3] = b.w;
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < NS; ++t) {
-                sk[t] = load_f32<(FL & kNtScales) != 0>(sKp + r0 + t);
-                sv[t] = load_f32<(FL & kNtScales) != 0>(sVp + r0 + t);
-            }
-        }
-        decode_math<D, NS, false>(kv, vv, sk, sv, row0, j1, q, qscale, m, l, acc);
+        IterBuf<NS> b;
+        load_iter<D, NS, FL>(b, Kp, Vp, sKp, sVp, r0, sub);
+        decode_math<D, NS, false>(b.kv, b.vv, b.sk, b.sv, 0, 0, q, qscale, m, l, acc);
     }
     const int base = j0 + n_full * G::kRowsPerIter;
     if (base < j1) {
@@ -909,41 +919,31 @@ DecodeWorkspace carve(void* ws, long long units, int D) {
                            ml_bytes + acc_bytes};
 }
 
-template <int D, int NS, bool VEC, bool FINAL>
-void launch_split(int flags, int stagger, dim3 grid, hipStream_t stream, const int8_t* Q,
-                  const int8_t* K, const int8_t* V, const float* sQ, const float* sK,
-                  const float* sV, const DecodeWorkspace& w, uint16_t* out, int S, int S_cap,
-                  const SplitPlan& plan, int units, float qk) {
-#define INT8K_SPLIT_LAUNCH(FLV)                                                      \
-    decode_split_kernel<D, NS, VEC, FINAL, FLV><<<grid, kBlockThreads, 0, stream>>>( \
-        Q, K, V, sQ, sK, sV, w.part_ml, w.part_acc, out, S, S_cap, plan.nsplit,      \
-        plan.chunk, units, qk, stagger)
-    switch (flags & 3) {
-        case 0: INT8K_SPLIT_LAUNCH(0); break;
-        case 1: INT8K_SPLIT_LAUNCH(1); break;
-        case 2: INT8K_SPLIT_LAUNCH(2); break;
-        default: INT8K_SPLIT_LAUNCH(3); break;
-    }
-#undef INT8K_SPLIT_LAUNCH
-}
+// Where a decode writes its rows: fp16 `f16`, or int8 `q` + per-row scale `qs`.
+struct DecodeOut {
+    uint16_t* f16;
+    int8_t* q;
+    float* qs;
+};
+
+// The arguments of a contiguous decode.
+struct DecodeArgs {
+    const int8_t *Q, *K, *V;
+    const float *sQ, *sK, *sV;
+    int BH, S, S_cap;
+    float qk;
+};
 
 // The 8-wave instance takes the paired-row load flags where it pairs rows.
-template <int D, int NS, bool VEC>
-void launch_block(const DecodeTuning& tn, int BH, hipStream_t stream, const int8_t* Q,
-                  const int8_t* K, const int8_t* V, const float* sQ, const float* sK,
-                  const float* sV, uint16_t* out, int8_t* qout, float* qs, int S, int S_cap,
-                  const SplitPlan& plan, float qk) {
-    const int stagger = tn.stagger;
-    const bool eight = plan.nsplit <= 8;
-    const int flags = (eight && paired_rows(D, NS, 8)) ? tn.pair_flags : tn.flags;
-#define INT8K_BLOCK_LAUNCH(FLV)                                                               \
-    if (eight)                                                                                \
-        decode_block_kernel<D, NS, VEC, FLV, 8><<<(unsigned)BH, 64 * plan.nsplit, 0, stream>>>(  \
-            Q, K, V, sQ, sK, sV, out, qout, qs, S, S_cap, plan.chunk, qk, stagger);           \
-    else                                                                                      \
-        decode_block_kernel<D, NS, VEC, FLV, kMaxBlockSplits>                                 \
-            <<<(unsigned)BH, 64 * plan.nsplit, 0, stream>>>(Q, K, V, sQ, sK, sV, out, qout, qs, \
-                                                            S, S_cap, plan.chunk, qk, stagger)
+template <int D, int NS, int MAXW, bool GROUP>
+void launch_block(const DecodeTuning& tn, const DecodeArgs& a, const DecodeOut& o,
+                  const GroupPlan& g, const DecodeWorkspace& w, hipStream_t stream) {
+    const int flags = paired_rows(D, NS, MAXW) ? tn.pair_flags : tn.flags;
+    const unsigned blocks = (unsigned)a.BH * (unsigned)g.blocks;
+#define INT8K_BLOCK_LAUNCH(FLV)                                                                 \
+    decode_block_kernel<D, NS, FLV, MAXW, GROUP><<<blocks, 64 * g.waves, 0, stream>>>(          \
+        a.Q, a.K, a.V, a.sQ, a.sK, a.sV, o.f16, o.q, o.qs, a.S, a.S_cap, g.chunk, a.qk,         \
+        tn.stagger, g.blocks, w.part_ml, w.part_acc)
     switch (flags & 3) {
         case 0: INT8K_BLOCK_LAUNCH(0); break;
         case 1: INT8K_BLOCK_LAUNCH(1); break;
@@ -953,67 +953,38 @@ void launch_block(const DecodeTuning& tn, int BH, hipStream_t stream, const int8
 #undef INT8K_BLOCK_LAUNCH
 }
 
-template <int D, bool VEC, bool FINAL>
-void launch_split_ns(int ns, int flags, int stagger, dim3 grid, hipStream_t stream,
-                     const int8_t* Q, const int8_t* K, const int8_t* V, const float* sQ,
-                     const float* sK, const float* sV, const DecodeWorkspace& w, uint16_t* out,
-                     int S, int S_cap, const SplitPlan& plan, int units, float qk) {
-    if (ns == 4)
-        launch_split<D, 4, VEC, FINAL>(flags, stagger, grid, stream, Q, K, V, sQ, sK, sV, w, out,
-                                       S, S_cap, plan, units, qk);
-    else
-        launch_split<D, 8, VEC, FINAL>(flags, stagger, grid, stream, Q, K, V, sQ, sK, sV, w, out,
-                                       S, S_cap, plan, units, qk);
-}
-
-// Where a decode writes its rows: fp16 `f16`, or int8 `q` + per-row scale `qs`.
-struct DecodeOut {
-    uint16_t* f16;
-    int8_t* q;
-    float* qs;
-};
-
 template <int D>
-int launch_decode(const int8_t* Q, const int8_t* K, const int8_t* V, const DecodeOut& o,
-                  const float* sQ, const float* sK, const float* sV, int BH, int S, int S_cap,
-                  const SplitPlan& plan, const DecodeWorkspace& w, hipStream_t stream) {
-    uint16_t* out = o.f16;
-    const long long units = (long long)BH * plan.nsplit;
-    const float qk_scale_log2 = (1.0f / std::sqrt((float)D)) * kLog2e;
-    const dim3 grid((unsigned)ceil_div(units, kWavesPerBlock));
-    const bool vec = (S_cap % 4 == 0) && aligned_to(sK, 16) && aligned_to(sV, 16);
+int launch_decode(const DecodeArgs& a, const DecodeOut& o, const SplitPlan& plan,
+                  const DecodeWorkspace& w, hipStream_t stream) {
     const DecodeTuning tn = tuning_for(D);
-    const int ns = tn.slots;
-    const int fl = tn.flags;
-    const int sg = tn.stagger;
-    const int u = (int)units;
-    const float qk = qk_scale_log2;
+    // f(slots) with the slot count as a compile-time constant
+    auto with_ns = [&](auto&& f) {
+        if (tn.slots == 4) f(std::integral_constant<int, 4>{});
+        else f(std::integral_constant<int, 8>{});
+    };
     if (plan.nsplit <= kMaxBlockSplits && use_block_kernel()) {
         // one launch: the chunks of a (b,h) are the waves of one block
-        if (ns == 4) {
-            if (vec) launch_block<D, 4, true>(tn, BH, stream, Q, K, V, sQ, sK, sV, out, o.q, o.qs, S, S_cap, plan, qk);
-            else launch_block<D, 4, false>(tn, BH, stream, Q, K, V, sQ, sK, sV, out, o.q, o.qs, S, S_cap, plan, qk);
-        } else {
-            if (vec) launch_block<D, 8, true>(tn, BH, stream, Q, K, V, sQ, sK, sV, out, o.q, o.qs, S, S_cap, plan, qk);
-            else launch_block<D, 8, false>(tn, BH, stream, Q, K, V, sQ, sK, sV, out, o.q, o.qs, S, S_cap, plan, qk);
-        }
+        const GroupPlan g{1, plan.nsplit, plan.chunk};
+        with_ns([&](auto ns) {
+            if (plan.nsplit <= kGroupWaves)
+                launch_block<D, ns.value, kGroupWaves, false>(tn, a, o, g, w, stream);
+            else
+                launch_block<D, ns.value, kMaxBlockSplits, false>(tn, a, o, g, w, stream);
+        });
         return check_launch("decode_block_kernel");
     }
-    // the in-kernel final write is fp16 only; int8 rows always go through the combine
-    const bool final_pass = plan.nsplit == 1 && out != nullptr && aligned_to(out, 16);
-    if (vec && final_pass)
-        launch_split_ns<D, true, true>(ns, fl, sg, grid, stream, Q, K, V, sQ, sK, sV, w, out, S, S_cap, plan, u, qk);
-    else if (vec)
-        launch_split_ns<D, true, false>(ns, fl, sg, grid, stream, Q, K, V, sQ, sK, sV, w, out, S, S_cap, plan, u, qk);
-    else if (final_pass)
-        launch_split_ns<D, false, true>(ns, fl, sg, grid, stream, Q, K, V, sQ, sK, sV, w, out, S, S_cap, plan, u, qk);
-    else
-        launch_split_ns<D, false, false>(ns, fl, sg, grid, stream, Q, K, V, sQ, sK, sV, w, out, S, S_cap, plan, u, qk);
-    int st = check_launch("decode_split_kernel");
-    if (st != INT8K_OK || final_pass) return st;
-    const dim3 gridc((unsigned)ceil_div(BH, kWavesPerBlock));
-    decode_combine_kernel<D><<<gridc, kBlockThreads, 0, stream>>>(w.part_ml, w.part_acc, out,
-                                                                  o.q, o.qs, BH, plan.nsplit);
+    const GroupPlan g = plan.forced || !use_block_kernel()
+                            ? forced_groups(plan)
+                            : plan_groups(a.BH, a.S, D, tn.slots, plan.nsplit);
+    const bool group = g.blocks > 1 || !use_block_kernel();
+    with_ns([&](auto ns) {
+        if (group) launch_block<D, ns.value, kGroupWaves, true>(tn, a, o, g, w, stream);
+        else launch_block<D, ns.value, kGroupWaves, false>(tn, a, o, g, w, stream);
+    });
+    int st = check_launch("decode_block_kernel");
+    if (st != INT8K_OK || !group) return st;
+    decode_combine_kernel<D><<<(unsigned)a.BH, kBlockThreads, 0, stream>>>(
+        w.part_ml, w.part_acc, o.f16, o.q, o.qs, g.blocks);
     return check_launch("decode_combine_kernel");
 }
 
@@ -1021,49 +992,54 @@ template <int D>
 int launch_decode_paged(const int8_t* Q, const int8_t* Kp, const int8_t* Vp, const DecodeOut& o,
                         const float* sQ, const float* sKp, const float* sVp,
                         const int32_t* tables, const int32_t* lens, int B, int H,
-                        int num_pages, int log2_page, int max_pages, const SplitPlan& plan,
-                        const DecodeWorkspace& w, hipStream_t stream) {
+                        int num_pages, int log2_page, int max_pages, int max_context,
+                        const SplitPlan& plan, const DecodeWorkspace& w, hipStream_t stream) {
     uint16_t* out = o.f16;
     const int BH = B * H;
     const long long units = (long long)BH * plan.nsplit;
     const float qk = (1.0f / std::sqrt((float)D)) * kLog2e;
     const dim3 grid((unsigned)ceil_div(units, kWavesPerBlock));
     constexpr int NS = D == 128 ? 8 : 4;
-    const bool vec = aligned_to(sKp, 16) && aligned_to(sVp, 16);
-    // page ids the chunks can reach, staged in LDS by the one-launch kernel
+    const DecodeTuning tn = tuning_for(D);
+    const bool one_launch = plan.nsplit <= kGroupWaves && use_block_kernel();
+    GroupPlan g;
+    if (plan.forced || !use_block_kernel())
+        g = one_launch ? GroupPlan{1, plan.nsplit, plan.chunk} : forced_groups(plan);
+    else
+        g = plan_groups(BH, max_context, D, NS, plan.nsplit);
+    // page ids the rows of a block can span, staged in LDS
+    const long long rows = (long long)g.waves * g.chunk;
     const long long n_tab = std::min<long long>(
-        max_pages, ceil_div((long long)plan.nsplit * plan.chunk, 1LL << log2_page));
-    if (plan.nsplit <= 8 && use_block_kernel() && n_tab * 4 <= kPagedLdsTableBytes) {
-        const int st = tuning_for(D).stagger;
+        max_pages, g.blocks == 1 ? ceil_div(rows, 1LL << log2_page) : ((rows - 1) >> log2_page) + 2);
+    if (n_tab * 4 <= kPagedLdsTableBytes && (long long)BH * g.blocks * g.waves < (1LL << 26)) {
         const size_t lds = (size_t)n_tab * 4;
-#define INT8K_PAGED_BLOCK(FLV)                                                                 \
-    if (vec)                                                                                   \
-        decode_paged_block_kernel<D, NS, true, FLV, 8>                                         \
-            <<<(unsigned)BH, 64 * plan.nsplit, lds, stream>>>(                                 \
-                Q, Kp, Vp, sQ, sKp, sVp, tables, lens, out, o.q, o.qs, H, num_pages, log2_page, \
-                max_pages, (int)n_tab, plan.chunk, qk, st);                                     \
-    else                                                                                       \
-        decode_paged_block_kernel<D, NS, false, FLV, 8>                                        \
-            <<<(unsigned)BH, 64 * plan.nsplit, lds, stream>>>(                                 \
-                Q, Kp, Vp, sQ, sKp, sVp, tables, lens, out, o.q, o.qs, H, num_pages, log2_page, \
-                max_pages, (int)n_tab, plan.chunk, qk, st)
-        const DecodeTuning tn = tuning_for(D);
+        const unsigned blocks = (unsigned)BH * (unsigned)g.blocks;
+        const bool group = !(g.blocks == 1 && use_block_kernel());
+#define INT8K_PAGED_BLOCK(FLV, GR)                                                          \
+    decode_paged_block_kernel<D, NS, FLV, 8, GR><<<blocks, 64 * g.waves, lds, stream>>>(    \
+        Q, Kp, Vp, sQ, sKp, sVp, tables, lens, out, o.q, o.qs, BH, H, num_pages, log2_page, \
+        max_pages, (int)n_tab, g.chunk, qk, tn.stagger, g.blocks, w.part_ml, w.part_acc)
+#define INT8K_PAGED_BLOCK2(FLV)             \
+    if (group) INT8K_PAGED_BLOCK(FLV, true); \
+    else INT8K_PAGED_BLOCK(FLV, false)
         switch ((paired_rows(D, NS, 8) ? tn.pair_flags : tn.flags) & 3) {
-            case 0: INT8K_PAGED_BLOCK(0); break;
-            case 1: INT8K_PAGED_BLOCK(1); break;
-            case 2: INT8K_PAGED_BLOCK(2); break;
-            default: INT8K_PAGED_BLOCK(3); break;
+            case 0: INT8K_PAGED_BLOCK2(0); break;
+            case 1: INT8K_PAGED_BLOCK2(1); break;
+            case 2: INT8K_PAGED_BLOCK2(2); break;
+            default: INT8K_PAGED_BLOCK2(3); break;
         }
+#undef INT8K_PAGED_BLOCK2
 #undef INT8K_PAGED_BLOCK
-        return check_launch("decode_paged_block_kernel");
+        int st = check_launch("decode_paged_block_kernel");
+        if (st != INT8K_OK || !group) return st;
+        decode_combine_kernel<D><<<(unsigned)BH, kBlockThreads, 0, stream>>>(
+            w.part_ml, w.part_acc, out, o.q, o.qs, g.blocks);
+        return check_launch("decode_combine_kernel");
     }
     const bool final_pass = plan.nsplit == 1 && out != nullptr && aligned_to(out, 16);
-#define INT8K_PAGED_LAUNCH(FIN, FLV)                                                         \
-    if (vec) decode_paged_kernel<D, NS, FIN, FLV, true><<<grid, kBlockThreads, 0, stream>>>( \
-        Q, Kp, Vp, sQ, sKp, sVp, tables, lens, w.part_ml, w.part_acc, out, H, num_pages,     \
-        log2_page, max_pages, plan.nsplit, plan.chunk, (int)units, qk, tuning_for(D).stagger); \
-    else decode_paged_kernel<D, NS, FIN, FLV, false><<<grid, kBlockThreads, 0, stream>>>(   \
-        Q, Kp, Vp, sQ, sKp, sVp, tables, lens, w.part_ml, w.part_acc, out, H, num_pages,     \
+#define INT8K_PAGED_LAUNCH(FIN, FLV)                                                     \
+    decode_paged_kernel<D, NS, FIN, FLV><<<grid, kBlockThreads, 0, stream>>>(            \
+        Q, Kp, Vp, sQ, sKp, sVp, tables, lens, w.part_ml, w.part_acc, out, H, num_pages, \
         log2_page, max_pages, plan.nsplit, plan.chunk, (int)units, qk, tuning_for(D).stagger)
 #define INT8K_PAGED_FLAGS(FIN)                          \
     switch (tuning_for(D).flags & 3) {                  \
@@ -1081,9 +1057,8 @@ int launch_decode_paged(const int8_t* Q, const int8_t* Kp, const int8_t* Vp, con
 #undef INT8K_PAGED_LAUNCH
     int st = check_launch("decode_paged_kernel");
     if (st != INT8K_OK || final_pass) return st;
-    const dim3 gridc((unsigned)ceil_div(BH, kWavesPerBlock));
-    decode_combine_kernel<D><<<gridc, kBlockThreads, 0, stream>>>(w.part_ml, w.part_acc, out,
-                                                                  o.q, o.qs, BH, plan.nsplit);
+    decode_combine_kernel<D><<<(unsigned)BH, kBlockThreads, 0, stream>>>(
+        w.part_ml, w.part_acc, out, o.q, o.qs, plan.nsplit);
     return check_launch("decode_combine_kernel");
 }
 
@@ -1128,7 +1103,14 @@ static int decode_impl(const int8_t* Q, const int8_t* K, const int8_t* V, const 
         !aligned_to(scale_Q, 4) || !aligned_to(scale_K, 4) || !aligned_to(scale_V, 4) ||
         !out_ok(out))
         return INT8K_ERR_MISALIGNED;
-    const SplitPlan plan = plan_splits(BH, S, head_dim, nsplit);
+    SplitPlan plan = plan_splits(BH, S, head_dim, nsplit);
+    // a short sequence spread over several blocks falls back to one block per (b,h) when
+    // the caller brings no workspace
+    if (!plan.forced && plan.nsplit > kMaxBlockSplits &&
+        (!workspace || workspace_bytes < decode_partial_bytes(plan, BH, head_dim))) {
+        const SplitPlan small = plan_splits(BH, S, head_dim, 0, true);
+        if (small.nsplit <= kMaxBlockSplits) plan = small;
+    }
     const long long units = (long long)BH * plan.nsplit;
     if (units >= (1LL << 26)) return INT8K_ERR_UNSUPPORTED;  // 64 work-items per unit, < 2^32
     // the one-launch path reads no workspace: a null or short one is accepted there
@@ -1138,11 +1120,10 @@ static int decode_impl(const int8_t* Q, const int8_t* K, const int8_t* V, const 
         if (!aligned_to(workspace, 16)) return INT8K_ERR_MISALIGNED;
     }
     const DecodeWorkspace w = carve(workspace, units, head_dim);
-    if (head_dim == 128)
-        return launch_decode<128>(Q, K, V, out, scale_Q, scale_K, scale_V, BH, S, S_cap, plan,
-                                  w, as_stream(stream));
-    return launch_decode<64>(Q, K, V, out, scale_Q, scale_K, scale_V, BH, S, S_cap, plan, w,
-                             as_stream(stream));
+    const DecodeArgs a{Q,  K, V,     scale_Q, scale_K, scale_V,
+                       BH, S, S_cap, (1.0f / std::sqrt((float)head_dim)) * kLog2e};
+    return head_dim == 128 ? launch_decode<128>(a, out, plan, w, as_stream(stream))
+                           : launch_decode<64>(a, out, plan, w, as_stream(stream));
 }
 
 extern "C" int int8k_decode_attention_forward(
@@ -1204,7 +1185,7 @@ static SplitPlan plan_paged(int BH, int max_context, int D, int nsplit_req) {
     ns = std::max<long long>(1, std::min(ns, max_split));
     const long long chunk = round_up((size_t)ceil_div(max_context, ns), (size_t)R);
     ns = ceil_div(max_context, chunk);
-    return SplitPlan{(int)ns, (int)chunk};
+    return SplitPlan{(int)ns, (int)chunk, nsplit_req > 0};
 }
 
 extern "C" size_t int8k_decode_attention_paged_workspace_bytes(int B, int H, int max_context,
@@ -1272,10 +1253,10 @@ static int paged_impl(
     if (head_dim == 128)
         return launch_decode_paged<128>(Q, K_pages, V_pages, out, scale_Q, sK_pages, sV_pages,
                                         block_tables, context_lens, B, H, num_pages, log2_page,
-                                        max_pages_per_seq, plan, w, as_stream(stream));
+                                        max_pages_per_seq, max_context, plan, w, as_stream(stream));
     return launch_decode_paged<64>(Q, K_pages, V_pages, out, scale_Q, sK_pages, sV_pages,
                                    block_tables, context_lens, B, H, num_pages, log2_page,
-                                   max_pages_per_seq, plan, w, as_stream(stream));
+                                   max_pages_per_seq, max_context, plan, w, as_stream(stream));
 }
 
 extern "C" int int8k_decode_attention_forward_paged(

@@ -1,0 +1,101 @@
+"""Decode plans of several blocks per (b,h): partials merged by the combine kernel.
+
+Shapes sit at the edges of the layout: one row past a whole wave iteration, odd row
+strides at D = 64 (the paired rows count from the row before a head that starts in the
+middle of a 128-byte line), a cache longer than the sequence, chunks that end inside an
+iteration, empty tail blocks, and the same calls without a workspace (one block per
+(b,h)).  Against float64 attention with fp32 sums' bound: the fp16 rounding of the
+output (2^-11 relative) plus the 2e-3 that the fp32 softmax over up to 2^15 rows moves.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import int8k_capi as capi
+import workloads
+from helpers import assert_attn_close
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(c, S):
+    q = c["Qi"].double() * c["sQ"].double().unsqueeze(-1)
+    k = c["Ki"][:, :, :S].double() * c["sK"][:, :, :S].double().unsqueeze(-1)
+    v = c["Vi"][:, :, :S].double() * c["sV"][:, :, :S].double().unsqueeze(-1)
+    s = (k * q.unsqueeze(2)).sum(-1) * q.shape[-1] ** -0.5
+    return (torch.softmax(s, -1).unsqueeze(-1) * v).sum(2).cpu().numpy()
+
+
+@pytest.mark.parametrize("B,H,D,S,cap", [
+    (1, 3, 64, 4097, 4097), (1, 5, 64, 8191, 8191), (2, 3, 64, 5000, 5001), (1, 2, 64, 33, 37),
+    (1, 3, 64, 2049, 2050), (3, 7, 64, 63, 63), (1, 3, 128, 2113, 2113), (2, 2, 128, 12001, 12288),
+    (1, 1, 128, 1600, 1601), (1, 300, 64, 515, 515), (5, 60, 128, 3001, 3001)])
+def test_grouped_plans_match_float64(gpu, B, H, D, S, cap):
+    c = workloads.decode_case(B, H, D, cap, seed=S, device=gpu, outlier_frac=0.01)
+    BH = B * H
+    out = torch.empty((BH, D), dtype=torch.float16, device=gpu)
+    n = capi.decode_workspace_bytes(BH, S, D)
+    ref = _ref(c, S)
+    for ws in ([torch.empty(max(n, 1), dtype=torch.uint8, device=gpu)] +
+               ([None] if capi.decode_num_splits(BH, S, D) * 64 <= 8 * 2048 else [])):
+        st = capi.load().int8k_decode_attention_forward_cache(
+            *(ctypes.c_void_p(t.data_ptr()) for t in (c["Qi"], c["Ki"], c["Vi"], out, c["sQ"],
+                                                      c["sK"], c["sV"])),
+            BH, S, cap, D, 0, ctypes.c_void_p(ws.data_ptr() if ws is not None else 0),
+            n if ws is not None else 0,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        if ws is None and st == capi.INT8K_ERR_WORKSPACE:
+            assert n > 0  # a plan that always leaves partials
+            continue
+        assert st == capi.INT8K_OK
+        assert_attn_close(out.float().reshape(B, H, D).cpu().numpy(), ref, f"{B} {H} {D} {S} {cap}")
+
+
+def test_short_sequences_without_workspace_stay_on_one_block(gpu):
+    # spread over more blocks with a workspace, one block per (b,h) without: both accepted
+    B, H, D, S = 1, 12, 64, 6000
+    c = workloads.decode_case(B, H, D, S, seed=5, device=gpu)
+    outs = []
+    for ws_bytes in (capi.decode_workspace_bytes(12, S, D), 0):
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=gpu)
+        out = torch.empty((B * H, D), dtype=torch.float16, device=gpu)
+        st = capi.load().int8k_decode_attention_forward(
+            *(ctypes.c_void_p(t.data_ptr()) for t in (c["Qi"], c["Ki"], c["Vi"], out, c["sQ"],
+                                                      c["sK"], c["sV"])),
+            B * H, S, D, 0, ctypes.c_void_p(ws.data_ptr() if ws_bytes else 0), ws_bytes,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        outs.append((st, out.float().cpu().numpy()))
+    ref = _ref(c, S).reshape(B * H, D)
+    for i, (st, o) in enumerate(outs):
+        if st != capi.INT8K_OK:
+            assert i == 1 and capi.decode_num_splits(12, S, D) > 16
+        else:
+            assert_attn_close(o, ref, f"workspace {i == 0}")
+    assert outs[0][0] == capi.INT8K_OK
+
+
+@pytest.mark.parametrize("D,page,lens", [(64, 16, [6000, 1, 17, 3000]), (128, 64, [9000, 65]),
+                                         (64, 1024, [5001, 0]), (128, 16, [20000])])
+def test_grouped_paged_plans_match_float64(gpu, D, page, lens):
+    H = 4
+    c = workloads.paged_case(len(lens), H, D, page, lens, seed=page + D, device=gpu)
+    out = capi.decode_attention_paged(c["Qi"], c["K_pages"], c["V_pages"], c["sQ"],
+                                      c["sK_pages"], c["sV_pages"], c["block_tables"],
+                                      c["context_lens"], c["max_context"])
+    torch.cuda.synchronize()
+    for b, n in enumerate(lens):
+        o = out[b].float().cpu().numpy()
+        if n == 0:
+            assert np.all(o == 0)
+            continue
+        t = c["block_tables"][b, :-(-n // page)].long()
+        flat = {k: c[k][t].transpose(0, 1).reshape(H, len(t) * page, -1)[:, :n]
+                for k in ("K_pages", "V_pages", "sK_pages", "sV_pages")}
+        ref = _ref(dict(Qi=c["Qi"][b:b + 1], sQ=c["sQ"].reshape(len(lens), H)[b:b + 1],
+                        Ki=flat["K_pages"][None], Vi=flat["V_pages"][None],
+                        sK=flat["sK_pages"][None, ..., 0], sV=flat["sV_pages"][None, ..., 0]), n)
+        assert_attn_close(o, ref[0], f"paged D{D} page{page} len{n}")
