@@ -71,6 +71,10 @@ constexpr long long kMaxBlocks = 1LL << 20;
 // blocks (about 8 resident blocks per CU of a 256-CU device, 4 rounds).
 constexpr long long kVecBlocks = 8192;
 
+// LayerNorm keeps gamma and beta in registers over a wave's rows: a grid of 4
+// blocks per CU, so that many rows share one read of them.
+constexpr long long kLnBlocks = 1024;
+
 template <typename Op>
 __device__ __forceinline__ float wave_reduce(float v, Op op) {
 #pragma unroll
@@ -177,98 +181,143 @@ __device__ __forceinline__ uint4 pack_chunk(const float (&y)[Vec<DT>::W]) {
     return make_uint4(d[0], d[1], d[2], d[3]);
 }
 
+// gamma or beta of the W columns from col0 (a multiple of W): as 16-byte vectors
+// where the array is aligned for them, else one by one.
+template <int W>
+__device__ __forceinline__ void load_affine(const float* p, int col0, bool vec, float (&v)[W]) {
+    if (vec) {
+#pragma unroll
+        for (int j = 0; j < W; j += 4) {
+            const float4 f = *reinterpret_cast<const float4*>(p + col0 + j);
+            v[j] = f.x, v[j + 1] = f.y, v[j + 2] = f.z, v[j + 3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < W; ++e) v[e] = p[col0 + e];
+    }
+}
+
 // LayerNorm + per-token quantizer with the row in registers: 1 << lg lanes per
-// row, NC 16-byte chunks per lane (chunk_slots).  One read of x; the passes of
-// the one-element-per-lane kernel above become register passes.
-template <int DT, int NC>
+// row, NC 16-byte chunks per lane.  One read of x; the passes of the
+// one-element-per-lane kernel above become register passes.  PAD: slots past the
+// row repeat its last chunk and count for nothing in the sums.  ROWBLOCK: the 256
+// threads of a block hold one row (rows of more than kWaveRowChunks chunks, where one
+// wave would need 8 or more chunks per lane: 150-280 registers, 1-3 waves per
+// SIMD), reduced across the four waves through LDS.
+// HBM-bound, and latency-bound for few rows.  us with gamma and beta, before (one
+// element per lane, or gamma and beta element by element) -> here: 4000 x 768 bf16
+// 18.2 -> 7.1 (kernel time), 16384 x 1024 fp16 66 -> 16.7, 4096 x 8192 bf16 155 -> 30,
+// 100000 x 80 fp16 155 -> 16.7.
+constexpr int kWaveRowChunks = 256;
+
+template <int DT, int NC, bool PAD, bool ROWBLOCK>
 __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
     const void* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
     float eps, int8_t* __restrict__ q, float* __restrict__ scales, void* __restrict__ y_out,
-    uint32_t rows, int lg, int nc) {
+    uint32_t rows, int lg, uint32_t cpr, int affine_vec) {
     constexpr int W = Vec<DT>::W;
-    constexpr int NCMAX = chunk_slots<NC>();
-    if (NC > 0) nc = NC;
+    __shared__ float red[3][kWaves];
     const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    if (ROWBLOCK) lg = 6;
     const uint32_t rpw = 64u >> lg;
-    const uint32_t c0 = lane & ((1u << lg) - 1);
-    const uint32_t cpr = (uint32_t)nc << lg;
+    const uint32_t c0 = ROWBLOCK ? threadIdx.x : lane & ((1u << lg) - 1);
+    const int slg = ROWBLOCK ? 8 : lg;  // chunks between a lane's slots, as a power of two
+    if (!PAD) cpr = (uint32_t)NC << slg;
+    auto real = [&](int i) { return !PAD || ((uint32_t)i << slg) + c0 < cpr; };
     const int cols = (int)cpr * W;
+    // 1 / cols is exact where the row fills every slot (a power of two)
     const float inv_cols = 1.f / (float)cols;
+    auto over_cols = [&](float v) { return PAD ? v / (float)cols : v * inv_cols; };
     const uint4* src = reinterpret_cast<const uint4*>(x);
     auto add = [](float a, float b) { return a + b; };
-    const uint32_t nw = gridDim.x * 4;
-    for (uint32_t rb = (blockIdx.x * 4 + (threadIdx.x >> 6)) * rpw; rb < rows; rb += nw * rpw) {
+    auto mx = [](float a, float b) { return fmaxf(a, b); };
+    auto reduce = [&](float v, int k, auto op) {
+        v = row_reduce(v, lg, op);
+        if constexpr (ROWBLOCK) {
+            if (lane == 0) red[k][wave] = v;
+            __syncthreads();
+            v = op(op(red[k][0], red[k][1]), op(red[k][2], red[k][3]));
+        }
+        return v;
+    };
+    // gamma and beta stay in registers over the rows of a wave: re-read per row they
+    // are up to 4x the bytes of x through L2
+    float eg[NC][W], eb[NC][W];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int col0 = (int)(slot_chunk<PAD>(i, slg, c0, cpr) * W);
+        if (gamma) load_affine<W>(gamma, col0, affine_vec, eg[i]);
+        if (beta) load_affine<W>(beta, col0, affine_vec, eb[i]);
+    }
+    const uint32_t step = gridDim.x * (ROWBLOCK ? 1u : 4u * rpw);
+    for (uint32_t rb = ROWBLOCK ? blockIdx.x : (blockIdx.x * 4 + wave) * rpw; rb < rows;
+         rb += step) {
         // rows past the end take the last row and store it again (the same bytes
         // its own lane stores): no divergent branch around loads or stores
-        const uint32_t r = min(rb + (lane >> lg), rows - 1);
-        uint4 w[NCMAX];
+        const uint32_t r = ROWBLOCK ? rb : min(rb + (lane >> lg), rows - 1);
+        uint4 w[NC];
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+            w[i] = src[(size_t)r * cpr + slot_chunk<PAD>(i, slg, c0, cpr)];
         float sum = 0.f;
 #pragma unroll
-        for (int i = 0; i < NCMAX; ++i) {
-            if (NC > 0 || i < nc) {
-                w[i] = src[(size_t)r * cpr + ((uint32_t)i << lg) + c0];
-                float v[W];
-                unpack_chunk<DT>(w[i], v);
+        for (int i = 0; i < NC; ++i) {
+            float v[W];
+            unpack_chunk<DT>(w[i], v);
 #pragma unroll
-                for (int e = 0; e < W; ++e) sum += v[e];
-            }
+            for (int e = 0; e < W; ++e) sum += real(i) ? v[e] : 0.f;
         }
-        const float mean = row_reduce(sum, lg, add) * inv_cols;
+        const float mean = over_cols(reduce(sum, 0, add));
 #pragma unroll
-        for (int i = 0; i < NCMAX; ++i) reload_barrier(w[i]);
+        for (int i = 0; i < NC; ++i) reload_barrier(w[i]);
         float var = 0.f;
 #pragma unroll
-        for (int i = 0; i < NCMAX; ++i) {
-            if (NC > 0 || i < nc) {
-                float v[W];
-                unpack_chunk<DT>(w[i], v);
+        for (int i = 0; i < NC; ++i) {
+            float v[W];
+            unpack_chunk<DT>(w[i], v);
 #pragma unroll
-                for (int e = 0; e < W; ++e) {
-                    const float d = v[e] - mean;
-                    var = fmaf(d, d, var);
-                }
+            for (int e = 0; e < W; ++e) {
+                const float d = real(i) ? v[e] - mean : 0.f;
+                var = fmaf(d, d, var);
             }
         }
-        const float rstd = 1.f / sqrtf(row_reduce(var, lg, add) * inv_cols + eps);
+        const float rstd = 1.f / sqrtf(over_cols(reduce(var, 1, add)) + eps);
 #pragma unroll
-        for (int i = 0; i < NCMAX; ++i) reload_barrier(w[i]);
+        for (int i = 0; i < NC; ++i) reload_barrier(w[i]);
         // y, rounded to the dtype, replaces x in the chunk registers (its storage
-        // bits: unpacking them gives the rounded values back exactly).  gamma and
-        // beta are re-read per row (cache hits) instead of being hoisted out of
-        // the row loop into registers.
-        const float* g = gamma;
-        const float* bt = beta;
-        asm volatile("" : "+s"(g), "+s"(bt));
+        // bits: unpacking them gives the rounded values back exactly)
         float m = 0.f;
 #pragma unroll
-        for (int i = 0; i < NCMAX; ++i) {
-            if (NC > 0 || i < nc) {
-                float y[W];
-                unpack_chunk<DT>(w[i], y);
-                const int col0 = (int)((((uint32_t)i << lg) + c0) * W);
+        for (int i = 0; i < NC; ++i) {
+            float y[W];
+            unpack_chunk<DT>(w[i], y);
 #pragma unroll
-                for (int e = 0; e < W; ++e) {
-                    float t = (y[e] - mean) * rstd;
-                    if (g) t *= g[col0 + e];
-                    if (bt) t += bt[col0 + e];
-                    y[e] = round_to(t, DT);
-                    m = fmaxf(m, fabsf(y[e]));
-                }
-                w[i] = pack_chunk<DT>(y);
+            for (int e = 0; e < W; ++e) y[e] = (y[e] - mean) * rstd;
+            if (gamma) {
+#pragma unroll
+                for (int e = 0; e < W; ++e) y[e] *= eg[i][e];
             }
+            if (beta) {
+#pragma unroll
+                for (int e = 0; e < W; ++e) y[e] += eb[i][e];
+            }
+#pragma unroll
+            for (int e = 0; e < W; ++e) {
+                y[e] = round_to(y[e], DT);
+                m = fmaxf(m, fabsf(y[e]));
+            }
+            w[i] = pack_chunk<DT>(y);
         }
-        const float sc = fmaxf(row_reduce(m, lg, [](float a, float b) { return fmaxf(a, b); }),
-                               1e-8f) / 127.f;
+        const float sc = fmaxf(reduce(m, 2, mx), 1e-8f) / 127.f;
         const float inv = 1.f / sc;
 #pragma unroll
-        for (int i = 0; i < NCMAX; ++i) {
-            if (NC > 0 || i < nc) {
-                float y[W];
-                unpack_chunk<DT>(w[i], y);
-                const size_t chunk = (size_t)r * cpr + ((uint32_t)i << lg) + c0;
-                store_codes<W>(y, sc, inv, q + chunk * W);
-                if (y_out) reinterpret_cast<uint4*>(y_out)[chunk] = w[i];
-            }
+        for (int i = 0; i < NC; ++i) {
+            float y[W];
+            unpack_chunk<DT>(w[i], y);
+            const size_t chunk = (size_t)r * cpr + slot_chunk<PAD>(i, slg, c0, cpr);
+            store_codes<W>(y, sc, inv, q + chunk * W);
+            if (y_out) reinterpret_cast<uint4*>(y_out)[chunk] = w[i];
         }
         if (c0 == 0) scales[r] = sc;
     }
@@ -280,17 +329,20 @@ __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
 // wave are consecutive tokens of one head: its codes and scales go out as one
 // contiguous run (not as 64-byte pieces of H different heads), while each row
 // is still read as one full source row.  Each wave takes U row groups of its
-// grid stride at a time (U loads per lane in flight).
-template <int DT, int U>
+// grid stride at a time (U loads per lane in flight).  PAD: rows of cpr chunks on
+// more lanes (head_dim 80: 10 chunks on 16 lanes), the spare ones repeating the last.
+template <int DT, bool PAD, int U>
 __global__ __launch_bounds__(256) void quant_heads_vec_kernel(
     const void* __restrict__ x, int8_t* __restrict__ q0, float* __restrict__ s0,
     int8_t* __restrict__ q1, float* __restrict__ s1, int8_t* __restrict__ q2,
-    float* __restrict__ s2, uint32_t rows, uint32_t S, uint32_t parts, uint32_t H, int lg) {
+    float* __restrict__ s2, uint32_t rows, uint32_t S, uint32_t parts, uint32_t H, int lg,
+    uint32_t cpr) {
     constexpr int W = Vec<DT>::W;
     const int lane = threadIdx.x & 63;
     const uint32_t rpw = 64u >> lg;
-    const uint32_t c0 = lane & ((1u << lg) - 1);
-    const int Dh = (1 << lg) * W;
+    if (!PAD) cpr = 1u << lg;
+    const uint32_t c0 = slot_chunk<PAD>(0, lg, lane & ((1u << lg) - 1), cpr);
+    const int Dh = (int)cpr * W;
     const uint4* src = reinterpret_cast<const uint4*>(x);
     const uint32_t stride = gridDim.x * 4 * rpw;
     const uint32_t part_rows = rows / parts;  // B H S rows per part
@@ -308,7 +360,7 @@ __global__ __launch_bounds__(256) void quant_heads_vec_kernel(
             const uint32_t bh = drow[u] / S, s = drow[u] - bh * S;
             const uint32_t b = bh / H, h = bh - b * H;
             const uint32_t r = ((b * S + s) * parts + pp[u]) * H + h;
-            w[u] = src[((size_t)r << lg) + c0];
+            w[u] = src[(size_t)r * cpr + c0];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -349,12 +401,30 @@ extern "C" int int8k_layernorm_quantize_per_token(const void* x, int dtype, cons
     if (sh.ok && rows < (1LL << 31) && aligned_to(x, 16) && aligned_to(q, w) &&
         (!y_out || aligned_to(y_out, 16))) {
         const long long waves = ceil_div(rows, 64 >> sh.lg);
-        const unsigned blocks = (unsigned)std::min(ceil_div(waves, 4), kVecBlocks);
+        const bool row_block = sh.cpr > kWaveRowChunks;
+        const unsigned blocks =
+            (unsigned)std::min(row_block ? rows : ceil_div(waves, 4), kLnBlocks);
+        const int affine_vec =
+            (!gamma || aligned_to(gamma, 16)) && (!beta || aligned_to(beta, 16));
+        auto launch = [&](auto dt, auto nc, auto pad, auto rbk) {
+            layernorm_quant_vec_kernel<decltype(dt)::value, decltype(nc)::value,
+                                       decltype(pad)::value, decltype(rbk)::value>
+                <<<blocks, 256, 0, st>>>(x, gamma, beta, eps, q, scales, y_out, (uint32_t)rows,
+                                         sh.lg, (uint32_t)sh.cpr, affine_vec);
+        };
         with_dtype(dtype, [&](auto dt) {
-            with_chunks(sh.nc, [&](auto ncc) {
-                layernorm_quant_vec_kernel<decltype(dt)::value, decltype(ncc)::value>
-                    <<<blocks, 256, 0, st>>>(x, gamma, beta, eps, q, scales, y_out,
-                                             (uint32_t)rows, sh.lg, sh.nc);
+            if (row_block) {
+                if (sh.cpr <= 512)
+                    launch(dt, std::integral_constant<int, 2>{}, std::true_type{}, std::true_type{});
+                else if (sh.cpr <= 768)
+                    launch(dt, std::integral_constant<int, 3>{}, std::true_type{}, std::true_type{});
+                else
+                    launch(dt, std::integral_constant<int, 4>{}, std::true_type{}, std::true_type{});
+                return;
+            }
+            with_chunks(sh, [&](auto ncc, auto pad) {
+                if constexpr (decltype(ncc)::value <= kWaveRowChunks / 64)
+                    launch(dt, ncc, pad, std::false_type{});
             });
         });
         return check_launch("layernorm_quant_vec_kernel");
@@ -387,9 +457,13 @@ extern "C" int int8k_quantize_heads(const void* x, int dtype, int parts, int8_t*
         const long long waves = ceil_div(rows, 64 >> sh.lg);
         const unsigned blocks = (unsigned)std::min(ceil_div(waves, 4 * U), kVecBlocks);
         with_dtype(dtype, [&](auto dt) {
-            quant_heads_vec_kernel<decltype(dt)::value, U><<<blocks, 256, 0, st>>>(
-                x, q0, s0, q1, s1, q2, s2, (uint32_t)rows, (uint32_t)S, (uint32_t)parts,
-                (uint32_t)H, sh.lg);
+            with_chunks(sh, [&](auto ncc, auto pad) {
+                if constexpr (decltype(ncc)::value == 1)
+                    quant_heads_vec_kernel<decltype(dt)::value, decltype(pad)::value, U>
+                        <<<blocks, 256, 0, st>>>(x, q0, s0, q1, s1, q2, s2, (uint32_t)rows,
+                                                 (uint32_t)S, (uint32_t)parts, (uint32_t)H, sh.lg,
+                                                 (uint32_t)sh.cpr);
+            });
         });
         return check_launch("quant_heads_vec_kernel");
     }

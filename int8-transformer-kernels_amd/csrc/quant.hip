@@ -134,24 +134,26 @@ struct RowDst {
 
 // Vectorised per-token quantizer (one 16-byte chunk per lane, see rows.h): the
 // row is loaded once, kept in registers for the quantize step, and written as
-// 4- or 8-byte code groups.  NC chunks per lane (chunk_slots).  Each wave takes
-// U row groups of its grid stride at a time, so short rows still keep several
-// loads per lane in flight.
-template <int DT, int NC, int U>
-__global__ __launch_bounds__(256) void quant_rows_vec_kernel(const void* __restrict__ x,
-                                                             uint32_t rows, int lg, int nc,
-                                                             RowDst dst) {
+// 4- or 8-byte code groups.  NC chunks per lane.  Each wave takes U row groups of
+// its grid stride at a time, so short rows still keep several loads per lane in
+// flight.  HBM-bound.  4000 x 768 bf16 (96 chunks, 2 per lane with a third of the
+// slots repeated): 11.5 us with one element per lane, 5.0 here; 100000 x 80 fp16: 33 ->
+// 11.5.  One launch takes gridDim.y sources (the K and V of a cache append).
+template <int DT, int NC, bool PAD, int U>
+__global__ __launch_bounds__(256) void quant_rows_vec_kernel(const void* __restrict__ x0,
+                                                             const void* __restrict__ x1,
+                                                             uint32_t rows, int lg, uint32_t cpr,
+                                                             RowDst dst0, RowDst dst1) {
     constexpr int W = Vec<DT>::W;
-    constexpr int SLOTS = chunk_slots<NC>();
-    if (NC > 0) nc = NC;
+    const RowDst& dst = blockIdx.y ? dst1 : dst0;
     const int lane = threadIdx.x & 63;
     const uint32_t rpw = 64u >> lg;  // rows per wave
     const uint32_t c0 = lane & ((1u << lg) - 1);
-    const uint32_t cpr = (uint32_t)nc << lg;  // chunks per row
-    const uint4* src = reinterpret_cast<const uint4*>(x);
+    if (!PAD) cpr = (uint32_t)NC << lg;  // chunks per row
+    const uint4* src = reinterpret_cast<const uint4*>(blockIdx.y ? x1 : x0);
     const uint32_t stride = gridDim.x * 4 * rpw;  // rows between a wave's row groups
     for (uint32_t rb = (blockIdx.x * 4 + (threadIdx.x >> 6)) * rpw; rb < rows; rb += U * stride) {
-        uint4 w[U][SLOTS];
+        uint4 w[U][NC];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             // rows past the end take the last row: they load, quantize and store
@@ -159,37 +161,33 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(const void* __restr
             // around the loads or the stores, which keeps them all in flight.
             const uint32_t r = min(rb + u * stride + (lane >> lg), rows - 1);
 #pragma unroll
-            for (int i = 0; i < SLOTS; ++i)
-                if (NC > 0 || i < nc) w[u][i] = src[(size_t)r * cpr + ((uint32_t)i << lg) + c0];
+            for (int i = 0; i < NC; ++i)
+                w[u][i] = src[(size_t)r * cpr + slot_chunk<PAD>(i, lg, c0, cpr)];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t r = min(rb + u * stride + (lane >> lg), rows - 1);
             float m = 0.f;
 #pragma unroll
-            for (int i = 0; i < SLOTS; ++i) {
-                if (NC > 0 || i < nc) {
-                    float v[W];
-                    unpack_chunk<DT>(w[u][i], v);
+            for (int i = 0; i < NC; ++i) {
+                float v[W];
+                unpack_chunk<DT>(w[u][i], v);
 #pragma unroll
-                    for (int e = 0; e < W; ++e) m = fmaxf(m, fabsf(v[e]));
-                }
+                for (int e = 0; e < W; ++e) m = fmaxf(m, fabsf(v[e]));
             }
             m = row_reduce(m, lg, [](float a, float b) { return fmaxf(a, b); });
             const float s = fmaxf(m, 1e-8f) / 127.f;
             const float inv = 1.f / s;
 #pragma unroll
-            for (int i = 0; i < SLOTS; ++i) reload_barrier(w[u][i]);
+            for (int i = 0; i < NC; ++i) reload_barrier(w[u][i]);
             int8_t* qrow;
             float* sp;
             dst(r, qrow, sp);
 #pragma unroll
-            for (int i = 0; i < SLOTS; ++i) {
-                if (NC > 0 || i < nc) {
-                    float v[W];
-                    unpack_chunk<DT>(w[u][i], v);
-                    store_codes<W>(v, s, inv, qrow + (size_t)(((uint32_t)i << lg) + c0) * W);
-                }
+            for (int i = 0; i < NC; ++i) {
+                float v[W];
+                unpack_chunk<DT>(w[u][i], v);
+                store_codes<W>(v, s, inv, qrow + (size_t)slot_chunk<PAD>(i, lg, c0, cpr) * W);
             }
             if (c0 == 0) *sp = s;
         }
@@ -307,30 +305,43 @@ constexpr long long kMaxRowBlocks = 1LL << 20;
 // blocks (about 8 resident blocks per CU of a 256-CU device, 4 rounds).
 constexpr long long kVecRowBlocks = 8192;
 
-int launch_quant_rows(const void* x, int dtype, int8_t* q, float* scales, long long rows,
-                      int cols, const RowMap& map, hipStream_t stream) {
+// Per-token quantization of n_src (1 or 2) tensors of one shape.
+int launch_quant_rows(int n_src, const void* const* x, int dtype, int8_t* const* q,
+                      float* const* scales, long long rows, int cols, const RowMap& map,
+                      hipStream_t stream) {
     if (rows <= 0) return INT8K_OK;
     const RowShape sh = row_shape(cols, dtype);
     const int w = dtype == INT8K_DTYPE_F32 ? 4 : 8;
-    if (sh.ok && rows < (1LL << 31) && map.rows_per_group < (1LL << 31) && aligned_to(x, 16) &&
-        aligned_to(q, w)) {
+    bool vec = sh.ok && rows < (1LL << 31) && map.rows_per_group < (1LL << 31);
+    for (int i = 0; i < n_src; ++i) vec = vec && aligned_to(x[i], 16) && aligned_to(q[i], w);
+    if (vec) {
         const long long waves = ceil_div(rows, 64 >> sh.lg);
-        const RowDst dst{q, scales, cols, (uint32_t)map.rows_per_group, map.dst_group_stride,
-                         map.dst_offset};
+        RowDst dst[2];
+        for (int i = 0; i < 2; ++i) {
+            const int k = i < n_src ? i : 0;
+            dst[i] = RowDst{q[k], scales[k], cols, (uint32_t)map.rows_per_group,
+                            map.dst_group_stride, map.dst_offset};
+        }
         with_dtype(dtype, [&](auto dt) {
-            with_chunks(sh.nc, [&](auto ncc) {
+            with_chunks(sh, [&](auto ncc, auto pad) {
                 constexpr int DT = decltype(dt)::value, NC = decltype(ncc)::value;
+                constexpr bool PAD = decltype(pad)::value;
                 constexpr int U = NC == 1 ? 4 : (NC == 2 ? 2 : 1);
                 const unsigned blocks = (unsigned)std::min(ceil_div(waves, 4 * U), kVecRowBlocks);
-                quant_rows_vec_kernel<DT, NC, U><<<blocks, 256, 0, stream>>>(
-                    x, (uint32_t)rows, sh.lg, sh.nc, dst);
+                quant_rows_vec_kernel<DT, NC, PAD, U><<<dim3(blocks, n_src), 256, 0, stream>>>(
+                    x[0], x[n_src - 1], (uint32_t)rows, sh.lg, (uint32_t)sh.cpr, dst[0], dst[1]);
             });
         });
         return check_launch("quant_rows_vec_kernel");
     }
     const long long blocks = std::min((rows + 3) / 4, kMaxRowBlocks);
-    quant_rows_kernel<<<(unsigned)blocks, 256, 0, stream>>>(x, dtype, q, scales, rows, cols, map);
-    return check_launch("quant_rows_kernel");
+    for (int i = 0; i < n_src; ++i) {
+        quant_rows_kernel<<<(unsigned)blocks, 256, 0, stream>>>(x[i], dtype, q[i], scales[i], rows,
+                                                                cols, map);
+        const int st = check_launch("quant_rows_kernel");
+        if (st != INT8K_OK) return st;
+    }
+    return INT8K_OK;
 }
 
 inline int grid_for(long long n) {
@@ -379,7 +390,7 @@ extern "C" int int8k_quantize_per_token(const void* x, int dtype, int8_t* q, flo
         return INT8K_ERR_INVALID_ARGUMENT;
     if (!aligned_to(x, dtype == INT8K_DTYPE_F32 ? 4 : 2) || !aligned_to(scales, 4))
         return INT8K_ERR_MISALIGNED;
-    return launch_quant_rows(x, dtype, q, scales, rows, cols, RowMap{rows, rows, 0},
+    return launch_quant_rows(1, &x, dtype, &q, &scales, rows, cols, RowMap{rows, rows, 0},
                              as_stream(stream));
 }
 
@@ -401,10 +412,10 @@ extern "C" int int8k_kv_cache_append(const void* k_new, const void* v_new, int d
         return INT8K_ERR_MISALIGNED;
     const RowMap map{n_new, capacity, pos};
     const long long rows = (long long)BH * n_new;
-    hipStream_t s = as_stream(stream);
-    int st = launch_quant_rows(k_new, dtype, K_cache, sK_cache, rows, head_dim, map, s);
-    if (st != INT8K_OK) return st;
-    return launch_quant_rows(v_new, dtype, V_cache, sV_cache, rows, head_dim, map, s);
+    const void* x[2] = {k_new, v_new};
+    int8_t* q[2] = {K_cache, V_cache};
+    float* sc[2] = {sK_cache, sV_cache};
+    return launch_quant_rows(2, x, dtype, q, sc, rows, head_dim, map, as_stream(stream));
 }
 
 extern "C" int int8k_dequantize_per_token(const int8_t* q, const float* scales, int dtype,

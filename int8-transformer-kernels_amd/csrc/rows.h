@@ -4,11 +4,14 @@
 // (producer.hip) all reduce one row to its absmax and then quantize it.  Rows
 // are short (a head of 64 or 128 elements, a model row of 1–8K), so one lane
 // per element leaves most of a wave's load slots empty.  Here each lane owns
-// 16-byte chunks of a row instead: a row of C chunks is spread over
-// L = min(C, 64) lanes (L a power of two) with C / L chunks per lane, so a
-// wave holds 64 / L rows, loads are 16 bytes per lane and the row reductions
-// are shuffles inside an aligned lane group.  Shapes that do not split this
-// way keep the one-element-per-lane kernels.
+// 16-byte chunks of a row instead: a row of C chunks is spread over L lanes (C
+// rounded up to a power of two, at most 64) with ceil(C / L) chunks per lane,
+// so a wave holds 64 / L rows, loads are 16 bytes per lane and the row
+// reductions are shuffles inside an aligned lane group.  Where C is not L times
+// a chunk count that has an instance, the slots past C repeat the row's last
+// chunk (PAD): the same loads, maxima and stored bytes again, and no branch.
+// Rows that are not whole chunks, or of more than 1024, keep the
+// one-element-per-lane kernels.
 #pragma once
 
 #include <type_traits>
@@ -26,9 +29,10 @@ struct Vec {
 // At most this many chunks per lane (a row of 64 * 16 chunks = 16 KiB).
 constexpr int kMaxChunksPerLane = 16;
 
-// How a row of `cols` elements maps onto lanes: 1 << lg lanes, nc chunks each.
+// How a row of `cols` elements maps onto lanes: cpr chunks on 1 << lg lanes, at
+// most nc each.
 struct RowShape {
-    int lg = 0, nc = 0;
+    int lg = 0, nc = 0, cpr = 0;
     bool ok = false;
 };
 
@@ -36,39 +40,45 @@ inline RowShape row_shape(int cols, int dtype) {
     RowShape r;
     const int w = dtype == INT8K_DTYPE_F32 ? 4 : 8;
     if (cols <= 0 || cols % w) return r;
-    const int c = cols / w;
-    if (c <= 64) {
-        if (c & (c - 1)) return r;
-        while ((1 << r.lg) < c) ++r.lg;
-        r.nc = 1;
-    } else {
-        if (c % 64 || c / 64 > kMaxChunksPerLane) return r;
-        r.lg = 6;
-        r.nc = c / 64;
-    }
-    r.ok = true;
+    r.cpr = cols / w;
+    while (r.lg < 6 && (1 << r.lg) < r.cpr) ++r.lg;
+    r.nc = (r.cpr + (1 << r.lg) - 1) >> r.lg;
+    r.ok = r.nc <= kMaxChunksPerLane;
     return r;
 }
 
-// Chunks per lane of a kernel instance: NC > 0 is a compile-time count (no
-// guards around the loads); NC = 0 means a runtime nc <= kMaxChunksPerLane.
-template <int NC>
-constexpr int chunk_slots() {
-    return NC > 0 ? NC : kMaxChunksPerLane;
+// Calls f(std::integral_constant<int, NC>, PAD as a bool constant) with the
+// smallest instance of at least sh.nc chunks per lane; PAD false when the row
+// fills every slot.  3, 6 and 12 beside the powers of two keep the repeated
+// chunks to a third of the row.
+template <typename F>
+inline void with_chunks(const RowShape& sh, F&& f) {
+    auto go = [&](auto nc, auto pow2) {
+        if constexpr (pow2.value) {
+            if (sh.cpr == (nc.value << sh.lg)) {
+                f(nc, std::false_type{});
+                return;
+            }
+        }
+        f(nc, std::true_type{});
+    };
+    using T = std::true_type;
+    using N = std::false_type;
+    if (sh.nc <= 1) go(std::integral_constant<int, 1>{}, T{});
+    else if (sh.nc <= 2) go(std::integral_constant<int, 2>{}, T{});
+    else if (sh.nc <= 3) go(std::integral_constant<int, 3>{}, N{});
+    else if (sh.nc <= 4) go(std::integral_constant<int, 4>{}, T{});
+    else if (sh.nc <= 6) go(std::integral_constant<int, 6>{}, N{});
+    else if (sh.nc <= 8) go(std::integral_constant<int, 8>{}, T{});
+    else if (sh.nc <= 12) go(std::integral_constant<int, 12>{}, N{});
+    else go(std::integral_constant<int, 16>{}, T{});
 }
 
-// Calls f(std::integral_constant<int, NC>) with NC = nc for the common counts
-// 1, 2, 4, 8, 16, and NC = 0 (runtime count) otherwise.
-template <typename F>
-inline void with_chunks(int nc, F&& f) {
-    switch (nc) {
-        case 1: f(std::integral_constant<int, 1>{}); break;
-        case 2: f(std::integral_constant<int, 2>{}); break;
-        case 4: f(std::integral_constant<int, 4>{}); break;
-        case 8: f(std::integral_constant<int, 8>{}); break;
-        case 16: f(std::integral_constant<int, 16>{}); break;
-        default: f(std::integral_constant<int, 0>{});
-    }
+// Chunk of slot i of the lane whose first chunk is c0, in a row of cpr chunks.
+template <bool PAD>
+__device__ __forceinline__ uint32_t slot_chunk(int i, int lg, uint32_t c0, uint32_t cpr) {
+    const uint32_t c = ((uint32_t)i << lg) + c0;
+    return PAD ? min(c, cpr - 1) : c;
 }
 
 // Calls f(std::integral_constant<int, DT>) for a dtype code.
@@ -106,12 +116,25 @@ __device__ __forceinline__ void unpack_chunk(const uint4& w, float (&v)[Vec<DT>:
 }
 
 // Reduction over the aligned group of 1 << lg lanes that holds one row; every
-// lane of the group gets the result.
+// lane of the group gets it.  On the VALU: DPP inside a 16-lane row (after the
+// xor 1 and xor 2 steps a quad's lanes agree, so the mirrors pair whole quads and
+// halves as xor 4 and xor 8 would), then the row and half swaps.
 template <typename Op>
 __device__ __forceinline__ float row_reduce(float v, int lg, Op op) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-        if (k < lg) v = op(v, __shfl_xor(v, 1 << k));
+    auto f = [](int x) { return __int_as_float(x); };
+    auto i = [](float x) { return __float_as_int(x); };
+    if (lg > 0) v = op(v, f(dpp_xor1(i(v))));
+    if (lg > 1) v = op(v, f(dpp_xor2(i(v))));
+    if (lg > 2) v = op(v, f(dpp_half_mirror(i(v))));
+    if (lg > 3) v = op(v, f(dpp_row_mirror(i(v))));
+    if (lg > 4) {
+        const auto r = __builtin_amdgcn_permlane16_swap(i(v), i(v), false, false);
+        v = op(f(r[0]), f(r[1]));
+    }
+    if (lg > 5) {
+        const auto r = __builtin_amdgcn_permlane32_swap(i(v), i(v), false, false);
+        v = op(f(r[0]), f(r[1]));
+    }
     return v;
 }
 
