@@ -27,16 +27,15 @@
 // row on load (no requant pass, no int8 hidden in memory); same bytes, slower
 // on MI355X, so it runs only when INT8K_MLP_GEMM2_FP16_HIDDEN=1.
 //
-// Few tokens (decode-time MLPs, T = B): 256 x 256 tiles leave most CUs idle
-// (T = 128 gives 16 blocks for GEMM1 and 4 for GEMM2).  When a GEMM has fewer
-// tiles than CUs it runs split-K instead: gemm_i8_splitk_kernel (128 x 128
-// output tiles, the K range split over blocks, exact int32 partials) and
-// splitk_epilogue_kernel<EPI> (sums the partials per row, then the same
-// epilogue math as gemm_i8_kernel, writing the same fp16 output and absmax
-// partials), so requant_rows_kernel and every result are the same on both
-// paths.  Above 512 rows, a GEMM whose 256 x 256 grid has at most 128 tiles runs
-// gemm_i8_mid_kernel<EPI> (128 x 128 tiles, two blocks per CU, the same
-// epilogue), e.g. GEMM2 at T = 4096, d_model 1024.
+// Few tokens (decode-time MLPs, T = B): the time is the read of the weights, and
+// gemm_i8_stream_kernel streams them in either layout over all CUs, the K range
+// split over waves and blocks; rows_epilogue_kernel<EPI> then sums the exact int32
+// partials of a row, applies the epilogue and requantizes it.  Small packed GEMMs run
+// gemm_i8_skinny_kernel (32 x 32 tiles).  Between those and 128 big tiles,
+// gemm_i8_mid_kernel<EPI> runs 128 x 128 tiles, two blocks per CU, with the fp16
+// epilogue or, where the grid leaves CUs idle, split over K into the same partials.
+// gemm_route and mid_plan choose.  The integer sums and the epilogue's expressions
+// are the same on every path.
 #include <algorithm>
 #include <cstdlib>
 
@@ -617,17 +616,25 @@ __global__ __launch_bounds__(256) void rq_clear_kernel(uint32_t* __restrict__ p,
 // bytes as gemm_i8_kernel, with one absmax partial per row and 128 columns.
 constexpr int kMidB = 128, kMidW = 64, kMidT = kMidW / 32;
 constexpr int kMidAStage = kMidB * LDS_STRIDE;
-constexpr int kMidStage = 2 * kMidAStage;
-constexpr int kMidLds = 2 * kMidStage;
-constexpr int kMidEpiLds = kMidLds + 3 * kMidB * 4;
 constexpr int kMidChunks = kMidB * kChunksPerRow / kThreads;
-static_assert(kMidChunks == 4 && 2 * kMidEpiLds <= 160 * 1024, "two blocks per CU");
+// BKN: B stored [K][N], staged as 128 rows of k and read with transposing LDS reads
+// (rows 160 bytes apart: the 8 rows of a read start 32 bytes apart in the banks)
+template <bool BKN>
+struct MidLds {
+    static constexpr int kBStride = BKN ? kMidB + 32 : LDS_STRIDE;
+    static constexpr int kStage = kMidAStage + 128 * kBStride;
+    static constexpr int kScales = 2 * kStage;  // the epilogue's scales lie past the stages
+    static constexpr int kBytes = kScales + 3 * kMidB * 4;
+};
+static_assert(kMidChunks == 4 && 2 * MidLds<true>::kBytes <= 160 * 1024, "two blocks per CU");
 
-template <bool EDGE>
+// The K range [kb, ke) of a tile (kb a multiple of 16).
+template <bool EDGE, bool BKN>
 __device__ __forceinline__ void mid_mainloop(v16i (&acc)[kMidT][kMidT],
                                              const int8_t* __restrict__ A,
                                              const int8_t* __restrict__ Bt, int M, int N, int K,
-                                             int m0, int n0, char* lds) {
+                                             int kb, int ke, int m0, int n0, char* lds) {
+    constexpr int kMidStage = MidLds<BKN>::kStage, kBStride = MidLds<BKN>::kBStride;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -637,35 +644,46 @@ __device__ __forceinline__ void mid_mainloop(v16i (&acc)[kMidT][kMidT],
         for (int j = 0; j < kMidT; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-    const int nk = (K + BK - 1) / BK;
+    const int nk = (ke - kb + BK - 1) / BK;
     const int a_off = (wm * kMidW + (lane & 31)) * LDS_STRIDE + (lane >> 5) * 16;
-    const int b_off = kMidAStage + (wn * kMidW + (lane & 31)) * LDS_STRIDE + (lane >> 5) * 16;
+    const int g16 = lane >> 4, s16 = lane & 15;
+    const int b_off =
+        kMidAStage + (BKN ? (16 * (g16 >> 1) + (s16 >> 1)) * kBStride + wn * kMidW + 16 * (g16 & 1) +
+                                8 * (s16 & 1)
+                          : (wn * kMidW + (lane & 31)) * kBStride + (lane >> 5) * 16);
     int4 fa[kMidChunks], fb[kMidChunks];
     // chunk c = t + 256 i of a 128 x 128-byte operand tile: row c / 8, bytes (c % 8) * 16;
     // rows past the matrix and K past the end load clamped addresses, zeroed on EDGE
-    auto load = [&](int k0) {
+    auto load = [&](int ks) {
+        const int k0 = kb + ks;
 #pragma unroll
         for (int i = 0; i < kMidChunks; ++i) {
             const int c = threadIdx.x + i * kThreads;
             const int row = c / kChunksPerRow, kc = (c % kChunksPerRow) * 16;
             const int gk = min(k0 + kc, K - 16);
             fa[i] = *reinterpret_cast<const int4*>(A + (size_t)min(m0 + row, M - 1) * K + gk);
-            fb[i] = *reinterpret_cast<const int4*>(Bt + (size_t)min(n0 + row, N - 1) * K + gk);
+            if constexpr (BKN)
+                fb[i] = *reinterpret_cast<const int4*>(Bt + (size_t)min(k0 + row, K - 1) * N +
+                                                       min(n0 + kc, N - 16));
+            else
+                fb[i] = *reinterpret_cast<const int4*>(Bt + (size_t)min(n0 + row, N - 1) * K + gk);
         }
     };
-    auto store = [&](char* stage, int k0) {
+    auto store = [&](char* stage, int ks) {
+        const int k0 = kb + ks;
 #pragma unroll
         for (int i = 0; i < kMidChunks; ++i) {
             const int c = threadIdx.x + i * kThreads;
             const int row = c / kChunksPerRow, kc = (c % kChunksPerRow) * 16;
             int4 va = fa[i], vb = fb[i];
             if constexpr (EDGE) {
-                const bool kok = k0 + kc < K;
+                const bool kok = k0 + kc < ke;
+                const bool bok = BKN ? k0 + row < ke && n0 + kc < N : kok && n0 + row < N;
                 if (!(kok && m0 + row < M)) va = make_int4(0, 0, 0, 0);
-                if (!(kok && n0 + row < N)) vb = make_int4(0, 0, 0, 0);
+                if (!bok) vb = make_int4(0, 0, 0, 0);
             }
             *reinterpret_cast<int4*>(stage + row * LDS_STRIDE + kc) = va;
-            *reinterpret_cast<int4*>(stage + kMidAStage + row * LDS_STRIDE + kc) = vb;
+            *reinterpret_cast<int4*>(stage + kMidAStage + row * kBStride + kc) = vb;
         }
     };
     // fragments of k-slice s of a stage: rows (l % 32) of the wave's two 32-row
@@ -675,8 +693,18 @@ __device__ __forceinline__ void mid_mainloop(v16i (&acc)[kMidT][kMidT],
         for (int i = 0; i < kMidT; ++i)
             a[i] = *reinterpret_cast<const v4i*>(stage + a_off + i * 32 * LDS_STRIDE + s * 32);
 #pragma unroll
-        for (int j = 0; j < kMidT; ++j)
-            b[j] = *reinterpret_cast<const v4i*>(stage + b_off + j * 32 * LDS_STRIDE + s * 32);
+        for (int j = 0; j < kMidT; ++j) {
+            if constexpr (BKN) {
+                typedef int v2i __attribute__((ext_vector_type(2)));
+                typedef __attribute__((address_space(3))) v2i lds_v2i;
+                const char* p = stage + b_off + s * 32 * kBStride + j * 32;
+                const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(p));
+                const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(p + 8 * kBStride));
+                b[j] = v4i{lo.x, lo.y, hi.x, hi.y};
+            } else {
+                b[j] = *reinterpret_cast<const v4i*>(stage + b_off + j * 32 * kBStride + s * 32);
+            }
+        }
     };
     auto mma = [&](const v4i (&a)[kMidT], const v4i (&b)[kMidT]) {
 #pragma unroll
@@ -713,28 +741,54 @@ __device__ __forceinline__ void mid_mainloop(v16i (&acc)[kMidT][kMidT],
     }
 }
 
-template <int EPI>
+// EPI_I32: blockIdx.y takes K range [y k_per_split, ..) and writes its exact int32
+// partials to c32 [split][M][ldc] (grids that leave CUs idle), else the whole K
+// and the fp16 epilogue.
+template <int EPI, bool BKN>
 __global__ __launch_bounds__(kThreads, 2) void gemm_i8_mid_kernel(
     const int8_t* __restrict__ A, const int8_t* __restrict__ Bt, int M, int N, int K,
-    int tiles_m, int tiles_n, EpiParams p) {
-    static_assert(EPI != EPI_I32, "fused epilogues only");
+    int k_per_split, int tiles_m, int tiles_n, EpiParams p) {
     extern __shared__ __align__(16) char lds[];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * kMidB, n0 = tn * kMidB;
+    const int kb = EPI == EPI_I32 ? (int)blockIdx.y * k_per_split : 0;
+    const int ke = EPI == EPI_I32 ? min(K - kb, k_per_split) + kb : K;
     // threads t and t + 128 load row / column t's scales (clamped, unconditional);
     // the epilogue keeps those of t < 128
     const int t = threadIdx.x & (kMidB - 1);
-    const float pre_sa = p.sa[(size_t)min(m0 + t, M - 1) * p.sa_stride];
-    const float pre_sb = p.sb[(size_t)min(n0 + t, N - 1) * p.sb_stride];
-    const float pre_b = p.bias != nullptr ? p.bias[min(n0 + t, N - 1)] : 0.f;
+    float pre_sa = 0.f, pre_sb = 0.f, pre_b = 0.f;
+    if constexpr (EPI != EPI_I32) {
+        pre_sa = p.sa[(size_t)min(m0 + t, M - 1) * p.sa_stride];
+        pre_sb = p.sb[(size_t)min(n0 + t, N - 1) * p.sb_stride];
+        if (p.bias != nullptr) pre_b = p.bias[min(n0 + t, N - 1)];
+    }
     v16i acc[kMidT][kMidT];
-    if (m0 + kMidB <= M && n0 + kMidB <= N && K % BK == 0)
-        mid_mainloop<false>(acc, A, Bt, M, N, K, m0, n0, lds);
+    if (m0 + kMidB <= M && n0 + kMidB <= N && (ke - kb) % BK == 0)
+        mid_mainloop<false, BKN>(acc, A, Bt, M, N, K, kb, ke, m0, n0, lds);
     else
-        mid_mainloop<true>(acc, A, Bt, M, N, K, m0, n0, lds);
-    epilogue_tile<EPI, kMidT, kMidT, kMidW, kMidW, kMidB, kMidLds>(acc, p, M, N, m0, n0, tn,
-                                                                   pre_sa, pre_sb, pre_b, lds);
+        mid_mainloop<true, BKN>(acc, A, Bt, M, N, K, kb, ke, m0, n0, lds);
+    if constexpr (EPI == EPI_I32) {
+        const int lane = threadIdx.x & 63;
+        const int wave = threadIdx.x >> 6;
+        const int rbase = m0 + (wave >> 1) * kMidW;
+        const int cbase = n0 + (wave & 1) * kMidW + (lane & 31);
+        int32_t* c = p.c32 + (size_t)blockIdx.y * M * p.ldc;
+#pragma unroll
+        for (int i = 0; i < kMidT; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = rbase + i * 32 + acc_row(r, lane);
+                if (row < M) {
+#pragma unroll
+                    for (int j = 0; j < kMidT; ++j)
+                        if (cbase + j * 32 < N) c[(size_t)row * p.ldc + cbase + j * 32] = acc[i][j][r];
+                }
+            }
+    } else {
+        epilogue_tile<EPI, kMidT, kMidT, kMidW, kMidW, kMidB, MidLds<BKN>::kScales>(
+            acc, p, M, N, m0, n0, tn, pre_sa, pre_sb, pre_b, lds);
+    }
 }
 
 // The MLP's GEMM2 over the fp16 hidden A16 [M][K] itself, with no
@@ -778,91 +832,245 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_i8_a16_kernel(
     epilogue_tile<EPI_F16>(acc, p, M, N, m0, n0, tn, pre_sa, pre_sb, 0.f, lds);
 }
 
-// ---------------------------------------------------------------- split-K path
+// ---------------------------------------------------------------- few tokens
+// gemm_i8_stream_kernel<MT, BKN>: a GEMM of up to 32 MT rows per row block, whose time
+// is the read of the weights (4096 -> 16384 as stored, 32 rows: 17.5 us per GEMM of 64
+// MiB, 3.8 TB/s, of which ~5 us are the first loads, the merge and the stores).  A wave owns 128 columns over its own range of K and
+// streams 128 x 128-byte weight tiles through its own piece of LDS: 16 loads of
+// 16 bytes per lane in flight, each covering whole 128-byte runs (8 weight rows
+// per instruction) for both layouts, the next tile's loads issued before the
+// current one's MFMAs, no block barrier in the loop.  Fragments come from LDS as
+// in the tiled kernels: 16-byte reads of [N][K] rows, or transposing reads of
+// [K][N] rows (BKN), so weights as stored need no transpose.  A's fragments are
+// read from global memory (L2) into registers one step ahead.  The waves of a
+// block meet in LDS, and the block writes exact int32 partials P[split][M][N],
+// which rows_epilogue_kernel sums.
+// MFMA operands are swapped, so a lane holds one row and 4 adjacent columns.
+// K past the end: A is zero there.  N past the end: those columns are not stored.
+constexpr int kStN = 128, kStK = 128;
+constexpr int kStMaxWaves = 8;
+template <bool BKN>
+struct StreamTile {
+    // bytes per LDS row: 16-byte fragment reads of consecutive [N][K] rows spread
+    // over the banks at 144; the 8 rows of a transposing read start 32 bytes apart
+    // (modulo the 256 of all banks) at 160
+    static constexpr int kStride = BKN ? kStN + 32 : kStK + 16;
+    static constexpr int kBytes = 128 * kStride;
+};
+constexpr int kStRedStride = kStN + 4;  // words per row of a wave's partial tile
+static_assert(32 * kStRedStride * 4 <= StreamTile<false>::kBytes, "a partial tile fits the stage");
 
-constexpr int kSkN = 128;       // output columns per block (4 waves x 32)
-constexpr int kSkM = 128;       // output rows per block (4 MFMA row tiles)
-constexpr int kSkK = 128;       // K bytes per step
-constexpr int kSkStride = kSkK + 16;  // padded LDS row of the A tile
-constexpr int kSkLds = 2 * kSkM * kSkStride;
-
-// P[split][M][N] (int32) = A[m0:m0+128, k range] . Bt[n0:n0+128, k range]^T.
-// grid = (N tiles, splits, M tiles); each wave owns 32 columns and all 128 rows
-// (4 x 32x32x32 MFMA tiles).  The A tile goes through LDS (shared by the four
-// waves); B fragments are loaded straight from global memory (each column is
-// used by one wave only).  K is a multiple of 32; rows >= M read as zero.
-__global__ __launch_bounds__(256) void gemm_i8_splitk_kernel(
-    const int8_t* __restrict__ A, const int8_t* __restrict__ Bt, int32_t* __restrict__ P,
-    int M, int N, int K, int k_per_split) {
+template <int MT, bool BKN>
+__global__ __launch_bounds__(64 * kStMaxWaves, 1) void gemm_i8_stream_kernel(
+    const int8_t* __restrict__ A, const int8_t* __restrict__ B, int32_t* __restrict__ P, int M,
+    int N, int K, int steps_per_wave) {
     extern __shared__ __align__(16) char lds[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n0 = blockIdx.x * kSkN, m0 = blockIdx.z * kSkM;
-    const int kb = blockIdx.y * k_per_split;
-    const int ke = min(K, kb + k_per_split);
-    const int ncol = n0 + wave * 32 + (lane & 31);
-    const int8_t* brow = Bt + (size_t)min(ncol, N - 1) * K;
-    v16i acc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][r] = 0;
+    using ST = StreamTile<BKN>;
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nw = blockDim.x >> 6;
+    const int n0 = blockIdx.x * kStN, m0 = blockIdx.z * 32 * MT;
+    const int kw = steps_per_wave * kStK;
+    const long long kb = ((long long)blockIdx.y * nw + wave) * kw;
+    const int k_begin = (int)min(kb, (long long)K);
+    const int k_end = min(K - k_begin, kw) + k_begin;
+    const int nsteps = (k_end - k_begin + kStK - 1) / kStK;
+    char* stage = lds + wave * ST::kBytes;
 
-    // A staging: 128 rows x 128 bytes = 1024 chunks of 16 B, 4 per thread
-    int4 ar[4];
-    auto load_a = [&](int k0) {
+    v16i acc[MT][4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = threadIdx.x + i * 256;
-            const int row = c >> 3, kc = (c & 7) * 16;
-            const int gk = min(k0 + kc, K - 16);
-            ar[i] = *reinterpret_cast<const int4*>(A + (size_t)min(m0 + row, M - 1) * K + gk);
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+
+    // weight tile: load i covers tile rows 8 i + lane / 8 (columns n of [N][K], or k of
+    // [K][N]), 16 bytes at 16 (lane % 8)
+    const uint32_t ldw = BKN ? (uint32_t)N : (uint32_t)K;
+    const uint32_t w_voff = (uint32_t)(lane >> 3) * ldw + (lane & 7) * 16;
+    v4u w[16];
+    auto load_w = [&](int k0) {
+        // the resource starts at the tile and ends with the matrix: rows past it read zero
+        const size_t off = BKN ? (size_t)k0 * N + n0 : (size_t)n0 * K + k0;
+        const size_t left = (size_t)N * K - off;
+        const __amdgpu_buffer_rsrc_t r = make_buffer(B + off, (uint32_t)min(left, (size_t)0xffffffffu));
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            w[i] = __builtin_amdgcn_raw_buffer_load_b128(r, w_voff, (uint32_t)(8 * i) * ldw, 0);
+    };
+    // A fragments of the step: rows 32 i + lane % 32, 16 bytes at k + 32 s + 16 (lane / 32)
+    const __amdgpu_buffer_rsrc_t ra =
+        make_buffer(A + (size_t)m0 * K, (uint32_t)min((size_t)(M - m0) * K, (size_t)0xffffffffu));
+    v4i a[MT][4];
+    auto load_a = [&](int k0, int s) {
+        const int k = k0 + 32 * s + 16 * (lane >> 5);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const uint32_t voff = (uint32_t)(32 * i + (lane & 31)) * (uint32_t)K + (uint32_t)k;
+            const v4u x = __builtin_amdgcn_raw_buffer_load_b128(ra, k < K ? voff : 0xffffffffu, 0, 0);
+            a[i][s] = __builtin_bit_cast(v4i, x);
         }
     };
-    auto store_a = [&](char* buf, int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = threadIdx.x + i * 256;
-            const int row = c >> 3, kc = (c & 7) * 16;
-            int4 v = ar[i];
-            if (!(m0 + row < M && k0 + kc < ke)) v = make_int4(0, 0, 0, 0);
-            *reinterpret_cast<int4*>(buf + row * kSkStride + kc) = v;
+    const int wr_off = (lane >> 3) * ST::kStride + (lane & 7) * 16;
+    const int g16 = lane >> 4, s16 = lane & 15;
+    const int rd_off = BKN ? (16 * (g16 >> 1) + (s16 >> 1)) * ST::kStride + 16 * (g16 & 1) + 8 * (s16 & 1)
+                           : (lane & 31) * ST::kStride + (lane >> 5) * 16;
+    auto read_b = [&](int j, int s) -> v4i {
+        if constexpr (BKN) {
+            typedef int v2i __attribute__((ext_vector_type(2)));
+            typedef __attribute__((address_space(3))) v2i lds_v2i;
+            const char* p = stage + rd_off + s * 32 * ST::kStride + j * 32;
+            const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(p));
+            const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(p + 8 * ST::kStride));
+            return v4i{lo.x, lo.y, hi.x, hi.y};
+        } else {
+            return *reinterpret_cast<const v4i*>(stage + rd_off + j * 32 * ST::kStride + s * 32);
         }
     };
-    const int nsteps = (ke - kb + kSkK - 1) / kSkK;
-    load_a(kb);
-    for (int st = 0; st < nsteps; ++st) {
-        const int k0 = kb + st * kSkK;
-        char* buf = lds + (st & 1) * (kSkM * kSkStride);
-        store_a(buf, k0);
-        // B fragments of this step: column ncol, bytes k0 + 32 s + 16 (lane / 32)
-        v4i bf[4];
+    if (nsteps > 0) {
+        load_w(k_begin);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int kk = k0 + 32 * s + 16 * (lane >> 5);
-            bf[s] = kk < ke ? *reinterpret_cast<const v4i*>(brow + kk) : v4i{0, 0, 0, 0};
-        }
-        if (st + 1 < nsteps) load_a(k0 + kSkK);
-        __syncthreads();
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (k0 + 32 * s >= ke) break;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const v4i af = *reinterpret_cast<const v4i*>(
-                    buf + (32 * i + (lane & 31)) * kSkStride + 32 * s + 16 * (lane >> 5));
-                acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf[s], acc[i], 0, 0, 0);
-            }
-        }
+        for (int s = 0; s < 4; ++s) load_a(k_begin, s);
     }
-    if (ncol >= N) return;
+    for (int st = 0; st < nsteps; ++st) {
+        const int k_next = k_begin + (st + 1) * kStK;
+        const bool more = st + 1 < nsteps;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            *reinterpret_cast<v4u*>(stage + wr_off + 8 * i * ST::kStride) = w[i];
+        // lanes read what other lanes of the wave wrote: keep the compiler from moving LDS
+        // accesses across (the wave's LDS operations complete in order)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (more) load_w(k_next);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            v4i b[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = read_b(j, s);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j], a[i][s], acc[i][j], 0, 0, 0);
+            if (more) load_a(k_next, s);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    // 32 rows at a time: each wave leaves its 32 x 128 partial tile in its own stage, the
+    // block sums the waves' tiles and stores them
     int32_t* Pp = P + (size_t)blockIdx.y * M * N;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MT; ++i) {
+        if (m0 + 32 * i >= M) break;
+        int* mine = reinterpret_cast<int*>(stage) + (lane & 31) * kStRedStride + 4 * (lane >> 5);
+        if (i > 0) __syncthreads();  // the previous rows have been read
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = m0 + 32 * i + acc_row(r, lane);
-            if (row < M) Pp[(size_t)row * N + ncol] = acc[i][r];
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<v4i*>(mine + 32 * j + 8 * q) =
+                    v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        __syncthreads();
+        for (int e = threadIdx.x; e < 32 * (kStN / 4); e += blockDim.x) {
+            const int row = e / (kStN / 4), c4 = e % (kStN / 4);
+            v4i sum = {0, 0, 0, 0};
+            for (int v = 0; v < nw; ++v)
+                sum += *reinterpret_cast<const v4i*>(lds + v * ST::kBytes +
+                                                     (row * kStRedStride + 4 * c4) * 4);
+            const int m = m0 + 32 * i + row, n = n0 + 4 * c4;
+            if (m < M && n < N) *reinterpret_cast<v4i*>(Pp + (size_t)m * N + n) = sum;
         }
+    }
+}
+
+// The row's value, requantization and scale from int32 partials: one block per row
+// sums the splits of its columns, applies the epilogue (same expressions as the
+// tiled kernels), keeps fp16(v) in registers, reduces the row's absmax and stores
+// the codes requant_rows_kernel would: no fp16 row, absmax partial or second
+// pass in memory.  NI groups of 4 columns per thread, blockDim.x * 4 * NI >= N.
+template <int EPI, int NI>
+__global__ __launch_bounds__(1024) void rows_epilogue_kernel(const int32_t* __restrict__ P,
+                                                             int splits, int M, int N,
+                                                             EpiParams p, int vec,
+                                                             int8_t* __restrict__ q,
+                                                             float* __restrict__ scales) {
+    __shared__ float red[16];
+    const int row = blockIdx.x, t = threadIdx.x;
+    const size_t plane = (size_t)M * N;
+    const int32_t* pr = P + (size_t)row * N;
+    const float sa = p.sa[(size_t)row * p.sa_stride];
+    // column scales and bias, in flight beside the partials (vec: 16-byte aligned arrays)
+    float4 sb[NI], bi[NI];
+    int nn[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int n = 4 * (t + i * (int)blockDim.x);
+        nn[i] = min(n, N - 4);  // groups past the row repeat the last one
+        if (vec) {
+            sb[i] = *reinterpret_cast<const float4*>(p.sb + nn[i]);
+            bi[i] = p.bias != nullptr ? *reinterpret_cast<const float4*>(p.bias + nn[i])
+                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+        } else {
+            const float* s = p.sb + (size_t)nn[i] * p.sb_stride;
+            const int d = p.sb_stride;
+            sb[i] = make_float4(s[0], s[d], s[2 * d], s[3 * d]);
+            const float* b = p.bias + nn[i];
+            bi[i] = p.bias != nullptr ? make_float4(b[0], b[1], b[2], b[3])
+                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    v4i sum[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) sum[i] = v4i{0, 0, 0, 0};
+    constexpr int kU = 8 / NI > 0 ? 8 / NI : 1;  // splits whose loads go out together
+    for (int sp = 0; sp < splits; sp += kU) {
+        v4i x[kU][NI];
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                x[u][i] = *reinterpret_cast<const v4i*>(pr + min(sp + u, splits - 1) * plane + nn[i]);
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                if (sp + u < splits) sum[i] += x[u][i];
+    }
+    uint16_t h[NI][4];
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const float sbe[4] = {sb[i].x, sb[i].y, sb[i].z, sb[i].w};
+        const float bie[4] = {bi[i].x, bi[i].y, bi[i].z, bi[i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = epi_value<EPI>(sum[i][e], sa, sbe[e], bie[e]);
+            m = fmaxf(m, fabsf(v));
+            h[i][e] = __half_as_ushort(f16_of_f32(v));
+        }
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
+    if ((t & 63) == 0) red[t >> 6] = m;
+    __syncthreads();
+    for (int v = 0; v < (int)blockDim.x >> 6; ++v) m = fmaxf(m, red[v]);
+    const float amax = fmaxf(m, 1e-8f);
+    const float inv = 127.f / amax;
+    if (t == 0) scales[row] = amax / 127.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float f = __half2float(__ushort_as_half(h[i][e])) * inv;
+            c |= ((uint32_t)(int)__builtin_rintf(fminf(fmaxf(f, -128.f), 127.f)) & 0xffu) << (8 * e);
+        }
+        *reinterpret_cast<uint32_t*>(q + (size_t)row * N + nn[i]) = c;
+    }
 }
 
 // acc = sum of the split partials (exact int32), then gemm_i8_kernel's
@@ -870,7 +1078,7 @@ __global__ __launch_bounds__(256) void gemm_i8_splitk_kernel(
 // covers columns [256 x, 256 x + 256) of row y and writes that chunk's absmax
 // to pmax[x][row], like one 256-column tile of gemm_i8_kernel.
 template <int EPI>
-__global__ __launch_bounds__(256) void splitk_epilogue_kernel(const int32_t* __restrict__ P,
+__global__ __launch_bounds__(256) void partial_epilogue_kernel(const int32_t* __restrict__ P,
                                                               int splits, int M, int N,
                                                               EpiParams p) {
     __shared__ float red[4];
@@ -888,7 +1096,7 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const int32_t* __r
         if constexpr (EPI == EPI_GELU_F16)
             v = gelu_tanh(v + (p.bias != nullptr ? p.bias[n] : 0.f));
         m = fabsf(v);
-        p.c16[(size_t)row * p.ldc + n] = f32_to_f16_bits(v);
+        p.c16[(size_t)row * p.ldc + n] = __half_as_ushort(f16_of_f32(v));
     }
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
@@ -908,23 +1116,126 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const int32_t* __r
 // writing one absmax partial per (32-column block, row).  No partial sums
 // leave the chip; split-K over blocks (above) would write them to memory.
 // Rows past M read row M-1 and are not stored.
-//
-//
 // It runs at ~3 us + 7 us per 2^30 multiply-adds on MI355X (latency-bound
-// loads; the tiles re-read A and Bt through L2, ~MNK/16 bytes).  Per GEMM,
-// measured against split-K and the 256 x 256 kernel at d_model 512..4096 and
-// T 1..2048, it wins up to M N K = 2^31, and up to 2^32 above 512 rows (no
-// split-K there) when the 256 x 256 grid would have fewer than 64 tiles.
+// loads; the tiles re-read A and Bt through L2, ~MNK/16 bytes); see gemm_route for
+// where it wins.
 constexpr int kSkinnyN = 32;
 constexpr int kSkinnyLds = 4 * 32 * kSkinnyN * 4 + 32 * 4;  // partials, row scales
 
-inline bool use_skinny(int M, int N, int K) {
-    if (N % kSkinnyN != 0 || K % 512 != 0) return false;
-    const long long mnk = (long long)M * N * K;
-    const long long big_tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    return mnk <= (1LL << 31) || (M > 4 * kSkM && big_tiles < 64 && mnk <= (1LL << 32));
+// Split of a few-token GEMM over waves and blocks: `waves` waves of `steps` 128-deep
+// K steps per block, `splits` blocks per column tile.
+struct StreamPlan {
+    int mt, waves, steps, splits, tiles_n, tiles_m;
+};
+constexpr int kRowsEpiMaxN = 32768;  // 1024 threads x 8 groups of 4 columns
+constexpr int kStWaves = 2048;       // 8 waves on each of 256 CUs
+
+inline StreamPlan stream_plan(int M, int N, int K) {
+    StreamPlan pl{};
+    pl.mt = M > 32 ? 2 : 1;
+    pl.tiles_n = (N + kStN - 1) / kStN;
+    pl.tiles_m = (M + 32 * pl.mt - 1) / (32 * pl.mt);
+    const int ksteps = (K + kStK - 1) / kStK;
+    const long long units = (long long)pl.tiles_n * pl.tiles_m * ksteps;
+    pl.steps = (int)std::max<long long>(1, units / kStWaves);
+    const int chain = (ksteps + pl.steps - 1) / pl.steps;  // waves per column tile
+    pl.waves = std::min(kStMaxWaves, chain);
+    pl.splits = (chain + pl.waves - 1) / pl.waves;
+    return pl;
 }
 
+// Split of a 128 x 128-tile GEMM over K (splits == 1: whole K, fp16 epilogue).
+struct MidPlan {
+    int tiles_m, tiles_n, splits, k_per_split;
+};
+
+// The split with the smallest time in units of 0.01 us: a K step of a block takes
+// about 0.6 us alone on its CU and 0.9 us beside a second block; the rows reach the
+// requantization as fp16 (written and read once) or as `splits` int32 partials, at
+// about 4.5 TB/s.  Measured, us per MLP with at most 512 / 256 blocks: T = 1024, 1024
+// -> 4096 48 / 34 (33 MB of partials for 4 K steps saved), T = 512, 2048 -> 8192
+// 53 / 45, T = 333, 4096 -> 16384 99 / 112 (GEMM2: 26 or 64 K steps per block).
+inline MidPlan mid_plan(int M, int N, int K) {
+    MidPlan pl{};
+    pl.tiles_m = (M + kMidB - 1) / kMidB;
+    pl.tiles_n = (N + kMidB - 1) / kMidB;
+    const long long tiles = (long long)pl.tiles_m * pl.tiles_n;
+    const long long ksteps = (K + BK - 1) / BK;
+    long long best = -1, steps = ksteps;
+    for (long long sp = 1; sp <= std::min(16LL, ksteps); ++sp) {
+        const long long st = ceil_div(ksteps, sp), n = ceil_div(ksteps, st);
+        const long long blocks = tiles * n;
+        const long long gemm = blocks <= 256 ? 60 * st : 90 * st * ceil_div(blocks, 512);
+        const long long rows = (n > 1 ? 8 * n : 4) * (long long)M * N / 45000;
+        if (best < 0 || gemm + rows < best) best = gemm + rows, steps = st;
+    }
+    pl.k_per_split = (int)(steps * BK);
+    pl.splits = (int)ceil_div(ksteps, steps);
+    return pl;
+}
+
+// The 128 x 128 kernel takes the GEMMs that the few-token paths leave and whose
+// 256 x 256 grid has at most 128 tiles: then its 4x as many tiles fit one round
+// of two blocks on each of the 256 CUs (before the split over K was added:).  Measured per MLP (d_model 1024, d_ff
+// 4096, prepacked): T = 2048 86 -> 57 us, T = 4096 99 -> 82 us, T = 8192 (128
+// big tiles in GEMM2) 145 -> 140 us; at 192 big tiles (T = 12288) it lost 11%.
+constexpr int kMidMaxBigTiles = 128;
+
+// The kernel of an M x N x K GEMM (packed: B is [N][K]).  Measured, us per MLP,
+// packed unless said, in turn:
+//  - up to 128 rows the weights' read is the time and the streaming kernel takes it:
+//    4096 -> 16384, T = 32: 62 (skinny) -> 48, as stored 109 (transposes + skinny) ->
+//    49; 2048 -> 8192, T = 64: 33 -> 28.5; with weights of at most 1 MiB up to 512
+//    rows (512 -> 2048, as stored);
+//  - packed weights of up to 4 MiB keep the skinny kernel to 2^30 multiply-adds, where
+//    a column tile of 128 leaves most CUs idle (1024 -> 4096, T = 64: 21 against 25);
+//  - then 128 x 128 tiles (split over K) to kMidMaxBigTiles: T = 333, 2048 -> 8192
+//    69 (split-K with a pass of its own for the epilogue and the requantization) ->
+//    45.6; T = 512, 1024 -> 4096 43 (skinny) -> 30; T = 512, 4096 -> 16384 172 -> 107.
+constexpr int kStreamRows = 128, kStreamRowsSmall = 512;
+constexpr long long kStreamSmallWeights = 1LL << 20, kSkinnyWeights = 1LL << 22;
+
+enum class Route { kStream, kSkinny, kMid, kTiled };
+
+Route gemm_route(int M, int N, int K, bool packed) {
+    const long long nk = (long long)N * K;
+    const long long big_tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    const bool skinny = packed && N % kSkinnyN == 0 && K % 512 == 0 && nk <= kSkinnyWeights &&
+                        M * nk <= (1LL << 30);
+    const int stream_rows = nk <= kStreamSmallWeights ? kStreamRowsSmall : kStreamRows;
+    if (M <= stream_rows && N <= kRowsEpiMaxN && K < (1 << 24) && !skinny) return Route::kStream;
+    if (skinny) return Route::kSkinny;
+    // (few rows of very wide weights: also operands of 4 GiB and more, see check_tiled_operands)
+    const bool few = M <= kStreamRowsSmall && big_tiles < 256;
+    return few || big_tiles <= kMidMaxBigTiles ? Route::kMid : Route::kTiled;
+}
+
+// How a GEMM's result reaches the requantization.
+struct GemmPlan {
+    Route route;
+    StreamPlan st;
+    MidPlan mid;
+    int splits;       // int32 partials to sum, 0: the GEMM applies its epilogue itself
+    int epi_tiles;    // absmax partials per row beside an fp16 output
+    size_t part_bytes(int M, int N) const { return (size_t)splits * M * N * 4; }
+};
+
+GemmPlan gemm_plan(int M, int N, int K, bool packed) {
+    GemmPlan g{};
+    g.route = gemm_route(M, N, K, packed);
+    g.epi_tiles = (N + BN - 1) / BN;
+    if (g.route == Route::kStream) {
+        g.st = stream_plan(M, N, K);
+        g.splits = g.st.splits;
+    } else if (g.route == Route::kSkinny) {
+        g.epi_tiles = N / kSkinnyN;
+    } else if (g.route == Route::kMid) {
+        g.mid = mid_plan(M, N, K);
+        if (g.mid.splits > 1) g.splits = g.mid.splits;
+        else g.epi_tiles = (N + kMidB - 1) / kMidB;
+    }
+    return g;
+}
 
 __device__ __forceinline__ void skinny_load(v4i (&b)[4], v4i (&a)[4], const int8_t* arow,
                                             const int8_t* brow, int k) {
@@ -945,7 +1256,7 @@ __global__ __launch_bounds__(256) void gemm_i8_skinny_kernel(const int8_t* __res
                                                              const int8_t* __restrict__ Bt,
                                                              int M, int N, int K, EpiParams p) {
     extern __shared__ __align__(16) char lds[];
-    (void)N;  // the grid covers the columns exactly: N % kSkinnyN == 0 (use_skinny)
+    (void)N;  // the grid covers the columns exactly: N % kSkinnyN == 0 (gemm_route)
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int n0 = blockIdx.x * kSkinnyN;
@@ -1025,65 +1336,41 @@ int launch_gemm_skinny(const int8_t* A, const int8_t* Bt, int M, int N, int K, c
     return check_launch("gemm_i8_skinny_kernel");
 }
 
-// Split plan for an M x N x K GEMM: run split-K when the 256 x 256 grid would
-// have fewer tiles than the device has CUs (256 on MI355X).
-struct SplitKPlan {
-    bool use;
-    int splits, k_per_split, tiles_n, tiles_m;
-};
-
-inline SplitKPlan splitk_plan(int M, int N, int K) {
-    SplitKPlan pl{};
-    const long long big_tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    if (big_tiles >= 256 || K % 32 != 0 || M > 4 * kSkM) return pl;
-    pl.tiles_n = (N + kSkN - 1) / kSkN;
-    pl.tiles_m = (M + kSkM - 1) / kSkM;
-    const int ksteps = (K + kSkK - 1) / kSkK;
-    const int want = (int)std::max<long long>(1, (512 + pl.tiles_n * pl.tiles_m - 1) /
-                                                     (pl.tiles_n * pl.tiles_m));
-    const int steps_per = (ksteps + std::min(want, ksteps) - 1) / std::min(want, ksteps);
-    pl.k_per_split = steps_per * kSkK;
-    pl.splits = (K + pl.k_per_split - 1) / pl.k_per_split;
-    pl.use = true;
-    return pl;
-}
-
-// The 128 x 128 kernel takes the GEMMs that the few-token paths leave and whose
-// 256 x 256 grid has at most 128 tiles: then its 4x as many tiles fit one round
-// of two blocks on each of the 256 CUs.  Measured per MLP (d_model 1024, d_ff
-// 4096, prepacked): T = 2048 86 -> 57 us, T = 4096 99 -> 82 us, T = 8192 (128
-// big tiles in GEMM2) 145 -> 140 us; at 192 big tiles (T = 12288) it lost 11%.
-constexpr int kMidMaxBigTiles = 128;
-
-inline bool use_mid(int M, int N, int K) {
-    if (use_skinny(M, N, K) || splitk_plan(M, N, K).use) return false;
-    const long long big_tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    return big_tiles <= kMidMaxBigTiles;
-}
-
-// Absmax partials per row that the GEMM's epilogue leaves (requant reads them).
-inline int epi_tiles(int M, int N, int K) {
-    if (use_skinny(M, N, K)) return N / kSkinnyN;
-    return use_mid(M, N, K) ? (N + kMidB - 1) / kMidB : (N + BN - 1) / BN;
-}
-
-inline size_t splitk_partial_bytes(int M, int N, int K) {
-    const SplitKPlan pl = splitk_plan(M, N, K);
-    return pl.use ? (size_t)pl.splits * M * N * 4 : 0;
-}
-
-template <int EPI>
-int launch_gemm_splitk(const int8_t* A, const int8_t* Bt, int M, int N, int K,
-                       const SplitKPlan& pl, int32_t* partial, const EpiParams& p,
-                       hipStream_t stream) {
+template <bool BKN>
+int launch_gemm_stream(const int8_t* A, const int8_t* B, int M, int N, int K,
+                       const StreamPlan& pl, int32_t* partial, hipStream_t stream) {
     const dim3 grid(pl.tiles_n, pl.splits, pl.tiles_m);
-    gemm_i8_splitk_kernel<<<grid, 256, kSkLds, stream>>>(A, Bt, partial, M, N, K,
-                                                         pl.k_per_split);
-    int st = check_launch("gemm_i8_splitk_kernel");
-    if (st != INT8K_OK) return st;
-    splitk_epilogue_kernel<EPI><<<dim3((N + 255) / 256, M), 256, 0, stream>>>(partial, pl.splits,
-                                                                              M, N, p);
-    return check_launch("splitk_epilogue_kernel");
+    const int lds = pl.waves * StreamTile<BKN>::kBytes;
+    if (pl.mt == 1)
+        gemm_i8_stream_kernel<1, BKN><<<grid, 64 * pl.waves, lds, stream>>>(A, B, partial, M, N, K,
+                                                                          pl.steps);
+    else
+        gemm_i8_stream_kernel<2, BKN><<<grid, 64 * pl.waves, lds, stream>>>(A, B, partial, M, N, K,
+                                                                          pl.steps);
+    return check_launch("gemm_i8_stream_kernel");
+}
+
+// The epilogue and requantization of M rows from `splits` int32 partials (N <= kRowsEpiMaxN).
+template <int EPI>
+int launch_rows_epilogue(const int32_t* partial, int splits, int M, int N, const EpiParams& p,
+                         int8_t* q, float* scales, hipStream_t stream) {
+    const int groups = (N + 3) / 4;
+    const int threads = std::min(1024, (groups + 63) / 64 * 64);
+    const int ni = (groups + threads - 1) / threads;
+    const int vec = p.sb_stride == 1 && aligned_to(p.sb, 16) && (!p.bias || aligned_to(p.bias, 16));
+    if (ni <= 1)
+        rows_epilogue_kernel<EPI, 1><<<M, threads, 0, stream>>>(partial, splits, M, N, p, vec, q,
+                                                              scales);
+    else if (ni <= 2)
+        rows_epilogue_kernel<EPI, 2><<<M, threads, 0, stream>>>(partial, splits, M, N, p, vec, q,
+                                                              scales);
+    else if (ni <= 4)
+        rows_epilogue_kernel<EPI, 4><<<M, threads, 0, stream>>>(partial, splits, M, N, p, vec, q,
+                                                              scales);
+    else
+        rows_epilogue_kernel<EPI, 8><<<M, threads, 0, stream>>>(partial, splits, M, N, p, vec, q,
+                                                              scales);
+    return check_launch("rows_epilogue_kernel");
 }
 
 // One block per row: reduce the row's absmax partials, then requantize the
@@ -1302,12 +1589,12 @@ int launch_gemm(const int8_t* A, const int8_t* Bt, int M, int N, int K, const Ep
     return check_launch("gemm_i8_kernel");
 }
 
-template <int EPI>
-int launch_gemm_mid(const int8_t* A, const int8_t* Bt, int M, int N, int K, const EpiParams& p,
-                    hipStream_t stream) {
-    const int tiles_m = (M + kMidB - 1) / kMidB, tiles_n = (N + kMidB - 1) / kMidB;
-    gemm_i8_mid_kernel<EPI><<<tiles_m * tiles_n, kThreads, kMidEpiLds, stream>>>(
-        A, Bt, M, N, K, tiles_m, tiles_n, p);
+template <int EPI, bool BKN>
+int launch_gemm_mid(const int8_t* A, const int8_t* B, int M, int N, int K, const MidPlan& pl,
+                    const EpiParams& p, hipStream_t stream) {
+    const dim3 grid(pl.tiles_m * pl.tiles_n, pl.splits);
+    gemm_i8_mid_kernel<EPI, BKN><<<grid, kThreads, MidLds<BKN>::kBytes, stream>>>(
+        A, B, M, N, K, pl.k_per_split, pl.tiles_m, pl.tiles_n, p);
     return check_launch("gemm_i8_mid_kernel");
 }
 
@@ -1386,67 +1673,62 @@ struct RqPlan {
     bool g1, g2;
 };
 
-inline bool rq_fusable(int M, int N, int K) {
-    if (use_skinny(M, N, K) || splitk_plan(M, N, K).use || use_mid(M, N, K)) return false;
-    return (N + BN - 1) / BN <= kRqMaxStripeTiles;
-}
+// The kernels of one MLP call.  Unpacked weights are read as the caller stores
+// them ([K][N]) by every GEMM but the fp16-hidden GEMM2, which reads a transposed
+// copy in the workspace.
+struct MlpPlan {
+    GemmPlan g1, g2;
+    RqPlan rq;
+    bool a16;       // GEMM2 reads the fp16 hidden (INT8K_MLP_GEMM2_FP16_HIDDEN=1)
+    bool kn1, kn2;
+    // no fp16 rows in memory: GEMM1 (GEMM2) requantizes in its epilogue, or
+    // rows_epilogue_kernel does from its partials (GEMM2: per-token output only)
+    bool direct1, direct2;
+};
 
-RqPlan rq_plan(int T, int dm, int dff, int flags) {
+MlpPlan mlp_plan(int T, int dm, int dff, int flags) {
     static const bool env_on = [] {
         const char* e = std::getenv("INT8K_MLP_FUSED_REQUANT");
         return !(e != nullptr && e[0] == '0');
     }();
-    const bool on = env_on && (flags & INT8K_MLP_SEPARATE_REQUANT) == 0;
-    RqPlan pl;
-    pl.g1 = on && !gemm2_reads_fp16_hidden() && rq_fusable(T, dff, dm);
-    pl.g2 = on && (flags & INT8K_MLP_OUT_PER_TENSOR) == 0 && rq_fusable(T, dm, dff);
-    return pl;
-}
-
-// Whether a GEMM runs on the 256 x 256 tiled kernels (gemm_i8_kernel, gemm_i8_rq_kernel).
-inline bool tiled_256(int M, int N, int K) {
-    return !use_skinny(M, N, K) && !splitk_plan(M, N, K).use && !use_mid(M, N, K);
-}
-
-// The kernels of one MLP call.  kn1 / kn2: the unpacked weights are read as the
-// caller stores them ([K][N]) by the tiled kernels, with no transpose; the other
-// tilings (and the fp16-hidden GEMM2) read transposed copies in the workspace.
-struct MlpPlan {
-    RqPlan rq;
-    bool a16;       // GEMM2 reads the fp16 hidden (INT8K_MLP_GEMM2_FP16_HIDDEN=1)
-    bool kn1, kn2;
-};
-
-MlpPlan mlp_plan(int T, int dm, int dff, int flags) {
+    const bool packed = (flags & INT8K_MLP_WEIGHTS_PREPACKED) != 0;
+    const bool per_token = (flags & INT8K_MLP_OUT_PER_TENSOR) == 0;
+    const bool fused = env_on && (flags & INT8K_MLP_SEPARATE_REQUANT) == 0;
     MlpPlan pl;
-    pl.rq = rq_plan(T, dm, dff, flags);
-    pl.a16 = !pl.rq.g1 && !use_skinny(T, dm, dff) && !splitk_plan(T, dm, dff).use &&
-             gemm2_reads_fp16_hidden();
-    const bool unpacked = (flags & INT8K_MLP_WEIGHTS_PREPACKED) == 0;
-    pl.kn1 = unpacked && tiled_256(T, dff, dm);
-    pl.kn2 = unpacked && !pl.a16 && tiled_256(T, dm, dff);
+    pl.g1 = gemm_plan(T, dff, dm, packed);
+    pl.g2 = gemm_plan(T, dm, dff, packed);
+    pl.a16 = gemm2_reads_fp16_hidden() &&
+             (pl.g2.route == Route::kMid || pl.g2.route == Route::kTiled);
+    auto fusable = [](const GemmPlan& g, int N) {
+        return g.route == Route::kTiled && (N + BN - 1) / BN <= kRqMaxStripeTiles;
+    };
+    pl.rq.g1 = fused && !pl.a16 && fusable(pl.g1, dff);
+    pl.rq.g2 = fused && per_token && !pl.a16 && fusable(pl.g2, dm);
+    pl.kn1 = !packed;
+    pl.kn2 = !packed && !pl.a16;
+    pl.direct1 = pl.rq.g1 || (!pl.a16 && pl.g1.splits > 0 && dff <= kRowsEpiMaxN);
+    pl.direct2 = pl.rq.g2 || (per_token && !pl.a16 && pl.g2.splits > 0 && dm <= kRowsEpiMaxN);
+    if (pl.a16) pl.g2.splits = 0, pl.g2.epi_tiles = (dm + BN - 1) / BN;
     return pl;
 }
 
 // Workspace layout of one MLP call (all offsets 256-byte aligned).
 struct MlpWorkspace {
-    int8_t* w1t;      // [d_ff][d_model]  (absent when prepacked)
-    int8_t* w2t;      // [d_model][d_ff]
-    uint16_t* h16;    // [T][d_ff]          (absent when GEMM1 requantizes)
+    int8_t* w2t;      // [d_model][d_ff]   (unpacked weights and the fp16-hidden GEMM2 only)
+    uint16_t* h16;    // [T][d_ff]          (absent with direct1)
     int8_t* hq;       // [T][d_ff]
     float* sh;        // [T]
-    float* p1;        // [tiles_n1][T]      (absent when GEMM1 requantizes)
-    uint16_t* o16;    // [T][d_model]       (absent when GEMM2 requantizes)
-    float* p2;        // [tiles_n2][T]      (absent when GEMM2 requantizes)
+    float* p1;        // [epi_tiles][T]     (absent with direct1)
+    uint16_t* o16;    // [T][d_model]       (absent with direct2)
+    float* p2;        // [epi_tiles][T]     (absent with direct2)
     float* tmax;      // [1]
     uint32_t* sync;   // fused requant: amax1 [T], amax2 [T], arrived1 [tiles_m], arrived2 [tiles_m]
     int sync_words;
-    int32_t* part;    // split-K partials (the larger GEMM's), when a GEMM runs split-K
+    int32_t* part;    // int32 partials (the larger GEMM's)
     size_t bytes;
 };
 
 MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const MlpPlan& pl) {
-    const RqPlan& rp = pl.rq;
     char* p = static_cast<char*>(base);
     size_t off = 0;
     auto take = [&](size_t n) {
@@ -1455,24 +1737,51 @@ MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const
         return r;
     };
     MlpWorkspace w{};
-    const size_t wbytes = prepacked ? 0 : (size_t)dm * dff;
-    w.w1t = reinterpret_cast<int8_t*>(take(pl.kn1 ? 0 : wbytes));
-    w.w2t = reinterpret_cast<int8_t*>(take(pl.kn2 ? 0 : wbytes));
-    w.h16 = reinterpret_cast<uint16_t*>(take(rp.g1 ? 0 : (size_t)T * dff * 2));
+    w.w2t = reinterpret_cast<int8_t*>(take(!prepacked && !pl.kn2 ? (size_t)dm * dff : 0));
+    w.h16 = reinterpret_cast<uint16_t*>(take(pl.direct1 ? 0 : (size_t)T * dff * 2));
     w.hq = reinterpret_cast<int8_t*>(take((size_t)T * dff));
     w.sh = reinterpret_cast<float*>(take((size_t)T * 4));
-    w.p1 = reinterpret_cast<float*>(take(rp.g1 ? 0 : (size_t)epi_tiles(T, dff, dm) * T * 4));
-    w.o16 = reinterpret_cast<uint16_t*>(take(rp.g2 ? 0 : (size_t)T * dm * 2));
-    w.p2 = reinterpret_cast<float*>(take(rp.g2 ? 0 : (size_t)epi_tiles(T, dm, dff) * T * 4));
+    w.p1 = reinterpret_cast<float*>(take(pl.direct1 ? 0 : (size_t)pl.g1.epi_tiles * T * 4));
+    w.o16 = reinterpret_cast<uint16_t*>(take(pl.direct2 ? 0 : (size_t)T * dm * 2));
+    w.p2 = reinterpret_cast<float*>(take(pl.direct2 ? 0 : (size_t)pl.g2.epi_tiles * T * 4));
     w.tmax = reinterpret_cast<float*>(take(4));
     const int tiles_m = (T + BM - 1) / BM;
-    w.sync_words = (rp.g1 || rp.g2) ? 2 * T + 2 * tiles_m : 0;
+    w.sync_words = (pl.rq.g1 || pl.rq.g2) ? 2 * T + 2 * tiles_m : 0;
     w.sync = reinterpret_cast<uint32_t*>(take((size_t)w.sync_words * 4));
-    const size_t part1 = use_skinny(T, dff, dm) ? 0 : splitk_partial_bytes(T, dff, dm);
-    const size_t part2 = use_skinny(T, dm, dff) ? 0 : splitk_partial_bytes(T, dm, dff);
-    w.part = reinterpret_cast<int32_t*>(take(std::max(part1, part2)));
+    w.part = reinterpret_cast<int32_t*>(take(std::max(pl.g1.part_bytes(T, dff), pl.g2.part_bytes(T, dm))));
     w.bytes = off;
     return w;
+}
+
+// One GEMM of the MLP with its epilogue: codes q and row scales qs (direct), or
+// fp16 rows p.c16 and absmax partials p.pmax.  kn: B is [K][N].
+template <int EPI>
+int run_gemm(const GemmPlan& g, bool rq, bool direct, bool kn, const int8_t* A, const int8_t* B,
+             int M, int N, int K, const EpiParams& p, int8_t* q, float* qs, uint32_t* amax,
+             uint32_t* arrived, int32_t* part, hipStream_t s) {
+    if (rq)
+        return kn ? launch_gemm_rq<EPI, true>(A, B, M, N, K, p, q, qs, amax, arrived, s)
+                  : launch_gemm_rq<EPI>(A, B, M, N, K, p, q, qs, amax, arrived, s);
+    int st = INT8K_OK;
+    if (g.route == Route::kTiled)
+        return kn ? launch_gemm<EPI, true>(A, B, M, N, K, p, s) : launch_gemm<EPI>(A, B, M, N, K, p, s);
+    if (g.route == Route::kSkinny) return launch_gemm_skinny<EPI>(A, B, M, N, K, p, s);
+    if (g.route == Route::kMid && g.splits == 0)
+        return kn ? launch_gemm_mid<EPI, true>(A, B, M, N, K, g.mid, p, s)
+                  : launch_gemm_mid<EPI, false>(A, B, M, N, K, g.mid, p, s);
+    EpiParams pi{};
+    pi.c32 = part;
+    pi.ldc = N;
+    if (g.route == Route::kStream)
+        st = kn ? launch_gemm_stream<true>(A, B, M, N, K, g.st, part, s)
+                : launch_gemm_stream<false>(A, B, M, N, K, g.st, part, s);
+    else
+        st = kn ? launch_gemm_mid<EPI_I32, true>(A, B, M, N, K, g.mid, pi, s)
+                : launch_gemm_mid<EPI_I32, false>(A, B, M, N, K, g.mid, pi, s);
+    if (st != INT8K_OK) return st;
+    if (direct) return launch_rows_epilogue<EPI>(part, g.splits, M, N, p, q, qs, s);
+    partial_epilogue_kernel<EPI><<<dim3((N + 255) / 256, M), 256, 0, s>>>(part, g.splits, M, N, p);
+    return check_launch("partial_epilogue_kernel");
 }
 
 PerDeviceOnce lds_once;
@@ -1495,15 +1804,24 @@ int configure_lds() {
         for (const void* k : epi_kernels)
             if (e == hipSuccess)
                 e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kEpiLdsBytes);
+        const void* stream_kernels[] = {
+            (const void*)gemm_i8_stream_kernel<1, false>, (const void*)gemm_i8_stream_kernel<2, false>,
+            (const void*)gemm_i8_stream_kernel<1, true>, (const void*)gemm_i8_stream_kernel<2, true>};
+        for (const void* k : stream_kernels)
+            if (e == hipSuccess)
+                e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        kStMaxWaves * StreamTile<true>::kBytes);
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void*)gemm_i8_a16_kernel,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kA16LdsBytes);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)gemm_i8_mid_kernel<EPI_GELU_F16>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMidEpiLds);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)gemm_i8_mid_kernel<EPI_F16>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMidEpiLds);
+        const void* mid_kernels[] = {
+            (const void*)gemm_i8_mid_kernel<EPI_GELU_F16, false>, (const void*)gemm_i8_mid_kernel<EPI_F16, false>,
+            (const void*)gemm_i8_mid_kernel<EPI_I32, false>, (const void*)gemm_i8_mid_kernel<EPI_GELU_F16, true>,
+            (const void*)gemm_i8_mid_kernel<EPI_F16, true>, (const void*)gemm_i8_mid_kernel<EPI_I32, true>};
+        for (const void* k : mid_kernels)
+            if (e == hipSuccess)
+                e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        MidLds<true>::kBytes);
         if (e != hipSuccess) {
             set_last_error("hipFuncSetAttribute", e);
             return (int)INT8K_ERR_HIP;
@@ -1584,11 +1902,10 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
     const bool prepacked = (flags & INT8K_MLP_WEIGHTS_PREPACKED) != 0;
     const bool per_tensor_out = (flags & INT8K_MLP_OUT_PER_TENSOR) != 0;
     const MlpPlan pl = mlp_plan(T, d_model, d_ff, flags);
-    const RqPlan& rp = pl.rq;
     // operands of 4 GiB or more on a 256 x 256 GEMM: refused before anything is launched
-    if (tiled_256(T, d_ff, d_model))
+    if (pl.g1.route == Route::kTiled)
         if (int st = check_tiled_operands(T, d_ff, d_model)) return st;
-    if (tiled_256(T, d_model, d_ff) && !pl.a16)
+    if (pl.g2.route == Route::kTiled && !pl.a16)
         if (int st = check_tiled_operands(T, d_model, d_ff)) return st;
     const MlpWorkspace w = carve_mlp(workspace, T, d_model, d_ff, prepacked, pl);
     if (!workspace || workspace_bytes < w.bytes) return INT8K_ERR_WORKSPACE;
@@ -1607,20 +1924,13 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
         if ((st = check_launch("rq_clear_kernel")) != INT8K_OK) return st;
     }
 
-    // W1t / W2t: [N][K] operands (prepacked, or transposed here), or the caller's
-    // [K][N] weights themselves where kn1 / kn2 read them as stored
-    const int8_t* W1t = W1;
     const int8_t* W2t = W2;
-    if (!prepacked && !pl.kn1) {
-        if ((st = launch_transpose(W1, w.w1t, d_model, d_ff, s)) != INT8K_OK) return st;
-        W1t = w.w1t;
-    }
     if (!prepacked && !pl.kn2) {
         if ((st = launch_transpose(W2, w.w2t, d_ff, d_model, s)) != INT8K_OK) return st;
         W2t = w.w2t;
     }
-    // GEMM1 + scale/bias/GELU epilogue -> int8 hidden + row scales (fused requant), or
-    // fp16 hidden + row absmax partials for the separate pass
+    // GEMM1 + scale/bias/GELU epilogue -> int8 hidden + row scales, or fp16 hidden + row
+    // absmax partials for the separate pass
     EpiParams p1{};
     p1.c16 = w.h16;
     p1.ldc = d_ff;
@@ -1630,27 +1940,16 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
     p1.sb_stride = n_scale_W1 == 1 ? 0 : 1;
     p1.bias = bias1;
     p1.pmax = w.p1;
-    const SplitKPlan sk1 = splitk_plan(T, d_ff, d_model);
-    if (rp.g1 && pl.kn1)
-        st = launch_gemm_rq<EPI_GELU_F16, true>(x, W1t, T, d_ff, d_model, p1, w.hq, w.sh, amax1,
-                                                arrived1, s);
-    else if (rp.g1)
-        st = launch_gemm_rq<EPI_GELU_F16>(x, W1t, T, d_ff, d_model, p1, w.hq, w.sh, amax1,
-                                          arrived1, s);
-    else if (pl.kn1)
-        st = launch_gemm<EPI_GELU_F16, true>(x, W1t, T, d_ff, d_model, p1, s);
-    else if (use_skinny(T, d_ff, d_model))
-        st = launch_gemm_skinny<EPI_GELU_F16>(x, W1t, T, d_ff, d_model, p1, s);
-    else if (sk1.use)
-        st = launch_gemm_splitk<EPI_GELU_F16>(x, W1t, T, d_ff, d_model, sk1, w.part, p1, s);
-    else if (use_mid(T, d_ff, d_model))
-        st = launch_gemm_mid<EPI_GELU_F16>(x, W1t, T, d_ff, d_model, p1, s);
-    else
-        st = launch_gemm<EPI_GELU_F16>(x, W1t, T, d_ff, d_model, p1, s);
+    st = run_gemm<EPI_GELU_F16>(pl.g1, pl.rq.g1, pl.direct1, pl.kn1, x, W1, T, d_ff, d_model, p1,
+                                w.hq, w.sh, amax1, arrived1, w.part, s);
     if (st != INT8K_OK) return st;
-    // GEMM2 + dequant epilogue -> int8 output + scales (fused requant), or fp16 output +
-    // absmax partials for the separate pass
-    const int tn1 = epi_tiles(T, d_ff, d_model);
+    // per-token requant of the fp16 hidden
+    if (!pl.direct1 && !pl.a16 &&
+        (st = launch_requant(w.h16, d_ff, w.p1, pl.g1.epi_tiles, nullptr, w.hq, d_ff, w.sh, T, d_ff,
+                             s)) != INT8K_OK)
+        return st;
+    // GEMM2 + dequant epilogue -> int8 output + scales, or fp16 output + absmax partials for
+    // the separate pass
     EpiParams p2{};
     p2.c16 = w.o16;
     p2.ldc = d_model;
@@ -1659,49 +1958,23 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
     p2.sb = scale_W2;
     p2.sb_stride = n_scale_W2 == 1 ? 0 : 1;
     p2.pmax = w.p2;
-    const SplitKPlan sk2 = splitk_plan(T, d_model, d_ff);
-    const bool skinny2 = use_skinny(T, d_model, d_ff);
-    // the on-load path has 256 x 256 tiles on every grid it runs
-    const bool a16 = pl.a16;
-    if (!rp.g1 && !a16) {
-        // per-token requant of the hidden (one absmax partial per row and 256-column
-        // tile, or per 32-column block of the skinny path)
-        if ((st = launch_requant(w.h16, d_ff, w.p1, tn1, nullptr, w.hq, d_ff, w.sh, T, d_ff,
-                                 s)) != INT8K_OK)
-            return st;
-    }
-    if (rp.g2 && pl.kn2)
-        return launch_gemm_rq<EPI_F16, true>(w.hq, W2t, T, d_model, d_ff, p2, out, out_scale,
-                                             amax2, arrived2, s);
-    if (rp.g2)
-        return launch_gemm_rq<EPI_F16>(w.hq, W2t, T, d_model, d_ff, p2, out, out_scale, amax2,
-                                       arrived2, s);
-    if (a16) {
-        // the tiled GEMM2 reads the fp16 hidden and quantizes it per row on load
-        const int tiles_m = (T + BM - 1) / BM, tiles_n = (d_model + BN - 1) / BN;
+    if (pl.a16) {
+        // GEMM2 on 256 x 256 tiles, reading the fp16 hidden and quantizing it per row on load
+        const int tiles_n = (d_model + BN - 1) / BN;
         gemm_i8_a16_kernel<<<tiles_m * tiles_n, kThreads, kA16LdsBytes, s>>>(
-            w.h16, W2t, T, d_model, d_ff, tiles_m, tiles_n, w.p1, tn1, p2);
-        if ((st = check_launch("gemm_i8_a16_kernel")) != INT8K_OK) return st;
+            w.h16, W2t, T, d_model, d_ff, tiles_m, tiles_n, w.p1, pl.g1.epi_tiles, p2);
+        st = check_launch("gemm_i8_a16_kernel");
     } else {
-        if (pl.kn2)
-            st = launch_gemm<EPI_F16, true>(w.hq, W2t, T, d_model, d_ff, p2, s);
-        else if (skinny2)
-            st = launch_gemm_skinny<EPI_F16>(w.hq, W2t, T, d_model, d_ff, p2, s);
-        else if (sk2.use)
-            st = launch_gemm_splitk<EPI_F16>(w.hq, W2t, T, d_model, d_ff, sk2, w.part, p2, s);
-        else if (use_mid(T, d_model, d_ff))
-            st = launch_gemm_mid<EPI_F16>(w.hq, W2t, T, d_model, d_ff, p2, s);
-        else
-            st = launch_gemm<EPI_F16>(w.hq, W2t, T, d_model, d_ff, p2, s);
-        if (st != INT8K_OK) return st;
+        st = run_gemm<EPI_F16>(pl.g2, pl.rq.g2, pl.direct2, pl.kn2, w.hq, W2t, T, d_model, d_ff, p2,
+                               out, out_scale, amax2, arrived2, w.part, s);
     }
-    const int tn2 = a16 ? (d_model + BN - 1) / BN : epi_tiles(T, d_model, d_ff);
+    if (st != INT8K_OK || pl.direct2) return st;
     const float* tmax = nullptr;
     if (per_tensor_out) {
-        tensor_absmax_kernel<<<1, 256, 0, s>>>(w.p2, (size_t)tn2 * T, w.tmax);
+        tensor_absmax_kernel<<<1, 256, 0, s>>>(w.p2, (size_t)pl.g2.epi_tiles * T, w.tmax);
         if ((st = check_launch("tensor_absmax_kernel")) != INT8K_OK) return st;
         tmax = w.tmax;
     }
-    return launch_requant(w.o16, d_model, w.p2, tn2, tmax, out, d_model, out_scale, T, d_model,
-                          s);
+    return launch_requant(w.o16, d_model, w.p2, pl.g2.epi_tiles, tmax, out, d_model, out_scale, T,
+                          d_model, s);
 }
