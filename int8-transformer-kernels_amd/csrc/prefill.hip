@@ -9,8 +9,9 @@
 // standard lower-triangular mask (key j visible to query i iff j <= i).
 //
 // Design (CDNA4): a block owns the queries of one (b,h), 32 per wave (256
-// queries on 8 waves at head_dim 128, 128 queries on 4 waves at 64 and 256),
-// and walks the KV sequence in tiles of 64 keys.  K (int8 rows), V (fp16,
+// queries on 8 waves at head_dim 128, 128 queries on 4 waves at 64 and 256; fewer
+// queries with the keys split over groups of waves where that grid would leave
+// CUs idle), and walks the KV sequence in tiles of 64 keys.  K (int8 rows), V (fp16,
 // row-major) and both key-scale vectors of a tile are staged in double-buffered LDS
 // by buffer loads: the next tile's loads are in flight in registers while the
 // current tile is computed, and there is one barrier per tile.  The LDS reads
@@ -40,6 +41,7 @@
 // input): the fp16 values the fp16 path would store, their row absmax, and
 // the per-token quantizer's codes and scale — the same bytes as
 // int8k_quantize_per_token over the fp16 output, without its round trip.
+#include <algorithm>
 #include <cmath>
 
 #include "int8k_common.h"
@@ -54,16 +56,19 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kKV = 64;  // keys per tile
-// Block shape per head_dim: one wave per 32 queries.  D = 128 runs 8 waves
-// (256 queries) at 2 waves per SIMD, so each staged K/V tile serves 256
-// queries; D = 64 keeps 4 waves (a 64-key tile has only 256 K chunks of 16 B)
-// and D = 256 keeps 4 waves at one wave per SIMD for its register budget.
-template <int D>
+// Block shapes: QW waves of 32 queries each, times KG groups of waves that share
+// the queries and walk every KG-th tile, each group with its own stages; the
+// groups' (m, l, O) merge in LDS at the end.  Large grids run KG = 1: D = 128 with
+// 8 waves (256 queries) at 2 waves per SIMD, so each staged K/V tile serves 256
+// queries; D = 64 with 4 waves (a 64-key tile has only 256 K chunks of 16 B); D = 256
+// with 4 waves at one wave per SIMD for its register budget.  Grids that leave CUs
+// idle split the keys of fewer queries over the groups (prefill_shape).
+template <int D, int QW, int KG = 1>
 struct Shape {
-    static constexpr int kWaves = D == 128 ? 8 : 4;
-    static constexpr int kThreads = 64 * kWaves;
-    static constexpr int kQ = 32 * kWaves;  // queries per block
-    static constexpr int kMinBlocks = D == 64 ? 2 : 1;  // 2 waves per SIMD at D <= 128
+    static constexpr int kGroupThreads = 64 * QW;
+    static constexpr int kThreads = 64 * QW * KG;
+    static constexpr int kQ = 32 * QW;  // queries per block
+    static constexpr int kMinBlocks = D == 64 && QW * KG == 4 ? 2 : 1;  // 2 waves per SIMD at D <= 128
 };
 // The V scales are applied once per staged tile, V' = fp16(v * sV * 2^-E), and
 // the probabilities enter the PV MFMA as P = fp16(p * 2^E), so
@@ -92,25 +97,25 @@ constexpr int kMaxVExp = 11;
 // a wave's loads of one key cover whole 64- or 128-byte runs of rows in memory
 // and its LDS writes whole runs of staged rows, and a thread's items share
 // their keys (one sV vector).
-template <int D>
+template <int D, int QW>
 struct VLayout {
     static constexpr int kRow = D + 32;  // halfs per staged row
-    static constexpr int kItems = 64 * D / 16 / Shape<D>::kThreads;
+    static constexpr int kItems = 64 * D / 16 / Shape<D, QW>::kGroupThreads;
     static constexpr int kW = D / 4 / kItems;  // dim groups per item row
 };
 
 // One LDS stage: K tile (int8 rows, 16-byte padded), V' tile (fp16 [key][dim],
 // the V scales applied), the key scales sK.
-template <int D>
+template <int D, int QW>
 struct Stage {
     static constexpr int kKStride = D + 16;  // bytes per K row
     static constexpr int kKBytes = kKV * kKStride;
-    static constexpr int kVtBytes = kKV * VLayout<D>::kRow * 2;
+    static constexpr int kVtBytes = kKV * VLayout<D, QW>::kRow * 2;
     static constexpr int kBytes = kKBytes + kVtBytes + kKV * 4;
-    static constexpr int kKChunks = kKV * D / 16 / Shape<D>::kThreads;  // 16-B K chunks per thread
-    static constexpr int kVItems = kKV * D / 16 / Shape<D>::kThreads;   // 4x4 V blocks per thread
-    static_assert(kKChunks >= 1 && kKChunks * 16 * Shape<D>::kThreads == kKV * D, "K tile split");
-    static_assert(kVItems >= 1 && kVItems * 16 * Shape<D>::kThreads == kKV * D, "V tile split");
+    static constexpr int kKChunks = kKV * D / 16 / Shape<D, QW>::kGroupThreads;  // 16-B K chunks per thread
+    static constexpr int kVItems = kKV * D / 16 / Shape<D, QW>::kGroupThreads;   // 4x4 V blocks per thread
+    static_assert(kKChunks >= 1 && kKChunks * 16 * Shape<D, QW>::kGroupThreads == kKV * D, "K tile split");
+    static_assert(kVItems >= 1 && kVItems * 16 * Shape<D, QW>::kGroupThreads == kKV * D, "V tile split");
 };
 
 // Buffer resources over one (b,h)'s K, V and scales.  Rows at or past S read
@@ -159,25 +164,23 @@ __device__ __forceinline__ uint2 load_v_f16x4(const v4i& desc, uint32_t voff, ui
     return make_uint2(r.x, r.y);
 }
 
-template <int D>
+// t: thread within its group.
+template <int D, int QW>
 __device__ __forceinline__ TileSrc make_tile_src(const int8_t* Kbh, const int8_t* Vbh,
                                                  const float* sKbh, const float* sVbh, int S,
-                                                 int dm) {
-    const int t = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    constexpr int kT = Shape<D>::kThreads;
+                                                 int dm, int t) {
+    constexpr int kT = Shape<D, QW>::kGroupThreads;
     TileSrc src;
     src.dm = (uint32_t)dm;
     src.k = make_buffer(Kbh, (uint32_t)S * dm);
     src.v = make_v_descriptor(Vbh, (uint32_t)S * dm);
-    (void)wave;
-    src.s = make_buffer(sKbh, (uint32_t)S * 4);    // wave 0 loads the tile's sK
+    src.s = make_buffer(sKbh, (uint32_t)S * 4);    // the group's first wave loads the tile's sK
     src.sv = make_buffer(sVbh, (uint32_t)S * 4);   // every thread: sV of its 4 V keys
     const int kcol = (t % (D / 16)) * 16;
     src.voff_k = (t / (D / 16)) * dm + kcol;
     src.kstep = (uint32_t)(kT * 16 / D) * dm;  // chunk t + n kT is kT*16/D rows further
     src.kvalid = kcol < dm;
-    using VL = VLayout<D>;
+    using VL = VLayout<D, QW>;
     const int dg = t % VL::kW, kg = t / VL::kW;
     src.voff_v = 4 * kg * dm + 4 * dg;
     src.vvalid = 0;
@@ -190,12 +193,12 @@ __device__ __forceinline__ TileSrc make_tile_src(const int8_t* Kbh, const int8_t
 }
 
 // Registers holding the next tile while the current one is computed.
-template <int D>
+template <int D, int QW>
 struct Prefetch {
-    int4 k[Stage<D>::kKChunks];
-    uint2 v[Stage<D>::kVItems][4];  // key 4 kg + i, dims 4 dg .. 4 dg + 3 as fp16 pairs
+    int4 k[Stage<D, QW>::kKChunks];
+    uint2 v[Stage<D, QW>::kVItems][4];  // key 4 kg + i, dims 4 dg .. 4 dg + 3 as fp16 pairs
     float4 sv;  // sV of keys 4 kg .. 4 kg + 3 (the keys of every item of the thread)
-    float sc;   // threads 0..63: sK of key tid
+    float sc;   // threads 0..63 of the group: sK of key t
 };
 
 // Thread t (of kT) loads 16-byte K chunk t + kT n (row (t + kT n) / (D/16);
@@ -203,14 +206,15 @@ struct Prefetch {
 // items (rows 4 kg .. 4 kg + 3, dims 4 dg .. 4 dg + 3; items n and n+1 are
 // 4 VLayout::kW bytes apart) and their 4 sV.  PAD: chunks and blocks past the
 // memory head_dim are zero.
-template <int D, bool PAD>
-__device__ __forceinline__ void prefetch_tile(Prefetch<D>& pf, const TileSrc& src, int k0) {
+template <int D, int QW, bool PAD>
+__device__ __forceinline__ void prefetch_tile(Prefetch<D, QW>& pf, const TileSrc& src, int k0,
+                                              int t) {
     typedef uint32_t v4u __attribute__((ext_vector_type(4)));
     typedef float v4f __attribute__((ext_vector_type(4)));
-    constexpr int kT = Shape<D>::kThreads;
+    constexpr int kT = Shape<D, QW>::kGroupThreads;
     const uint32_t dm = PAD ? src.dm : (uint32_t)D;
 #pragma unroll
-    for (int n = 0; n < Stage<D>::kKChunks; ++n) {
+    for (int n = 0; n < Stage<D, QW>::kKChunks; ++n) {
         if (!PAD || src.kvalid) {
             const v4u w = __builtin_amdgcn_raw_buffer_load_b128(
                 src.k, src.voff_k, k0 * dm + n * (PAD ? src.kstep : (uint32_t)(kT * 16)), 0);
@@ -220,12 +224,12 @@ __device__ __forceinline__ void prefetch_tile(Prefetch<D>& pf, const TileSrc& sr
         }
     }
 #pragma unroll
-    for (int n = 0; n < Stage<D>::kVItems; ++n) {
+    for (int n = 0; n < Stage<D, QW>::kVItems; ++n) {
         if (!PAD || (src.vvalid >> n) & 1u) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 pf.v[n][i] = load_v_f16x4(src.v, src.voff_v,
-                                          (k0 + i) * dm + n * 4 * VLayout<D>::kW);
+                                          (k0 + i) * dm + n * 4 * VLayout<D, QW>::kW);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i) pf.v[n][i] = make_uint2(0, 0);
@@ -234,25 +238,25 @@ __device__ __forceinline__ void prefetch_tile(Prefetch<D>& pf, const TileSrc& sr
     const v4f sv = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(src.sv, src.voff_sv,
                                                                                 k0 * 4, 0));
     pf.sv = make_float4(sv.x, sv.y, sv.z, sv.w);
-    if (threadIdx.x < kKV)
+    if (t < kKV)
         pf.sc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src.s, src.voff_s,
                                                                                k0 * 4, 0));
 }
 
 // vscale = 2^-E: V' = fp16(v * fp16(sV * 2^-E)) on v_pk_mul_f16, written as it
 // arrived: each key's 4 dims of an item as one 8-byte row piece.
-template <int D>
-__device__ __forceinline__ void commit_tile(const Prefetch<D>& pf, char* st, float vscale) {
+template <int D, int QW>
+__device__ __forceinline__ void commit_tile(const Prefetch<D, QW>& pf, char* st, float vscale,
+                                            int t) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    using VL = VLayout<D>;
-    const int t = threadIdx.x;
+    using VL = VLayout<D, QW>;
 #pragma unroll
-    for (int n = 0; n < Stage<D>::kKChunks; ++n) {
-        const int c = t + n * Shape<D>::kThreads;
+    for (int n = 0; n < Stage<D, QW>::kKChunks; ++n) {
+        const int c = t + n * Shape<D, QW>::kGroupThreads;
         const int row = c / (D / 16), col = (c % (D / 16)) * 16;
-        *reinterpret_cast<int4*>(st + row * Stage<D>::kKStride + col) = pf.k[n];
+        *reinterpret_cast<int4*>(st + row * Stage<D, QW>::kKStride + col) = pf.k[n];
     }
-    _Float16* vs = reinterpret_cast<_Float16*>(st + Stage<D>::kKBytes) +
+    _Float16* vs = reinterpret_cast<_Float16*>(st + Stage<D, QW>::kKBytes) +
                    (t / VL::kW) * 4 * VL::kRow + (t % VL::kW) * 4;
     // key 4 kg + i scaled by its sV * 2^-E (both dims of a word share the key)
     const float svk[4] = {pf.sv.x * vscale, pf.sv.y * vscale, pf.sv.z * vscale,
@@ -261,14 +265,14 @@ __device__ __forceinline__ void commit_tile(const Prefetch<D>& pf, char* st, flo
     for (int i = 0; i < 4; ++i) {
         const h2 sp = __builtin_convertvector((float __attribute__((ext_vector_type(2)))){svk[i], svk[i]}, h2);
 #pragma unroll
-        for (int n = 0; n < Stage<D>::kVItems; ++n) {
+        for (int n = 0; n < Stage<D, QW>::kVItems; ++n) {
             uint2 w;
             w.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, pf.v[n][i].x) * sp);
             w.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, pf.v[n][i].y) * sp);
             *reinterpret_cast<uint2*>(vs + i * VL::kRow + n * 4 * VL::kW) = w;
         }
     }
-    if (t < kKV) reinterpret_cast<float*>(st + Stage<D>::kKBytes + Stage<D>::kVtBytes)[t] = pf.sc;
+    if (t < kKV) reinterpret_cast<float*>(st + Stage<D, QW>::kKBytes + Stage<D, QW>::kVtBytes)[t] = pf.sc;
 }
 
 // Sum of the 32 fp16 P of a lane in fp32 (v_dot2_f32_f16 against {1, 1}).
@@ -288,20 +292,24 @@ __device__ __forceinline__ float psum(const v8h (&pfr)[4]) {
 
 // D: the kernel's head_dim.  PAD: the rows in memory have head_dim d_mem < D
 // (a multiple of 16); the dims past it read as zero and are not stored.
-template <int D, bool CAUSAL, bool PAD>
-__global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void prefill_kernel(
+template <int D, int QW, int KG, bool CAUSAL, bool PAD>
+__global__ __launch_bounds__((Shape<D, QW, KG>::kThreads), (Shape<D, QW, KG>::kMinBlocks)) void prefill_kernel(
     const int8_t* __restrict__ Q, const int8_t* __restrict__ K, const int8_t* __restrict__ V,
     const float* __restrict__ sQ, const float* __restrict__ sK, const float* __restrict__ sV,
     uint16_t* __restrict__ out, int8_t* __restrict__ qout, float* __restrict__ qout_scale, int S,
     int n_qtiles, float qk_scale_log2, int heads, int bshd, int d_mem) {
     constexpr int NS = D / 32;  // 32-wide d slices (QK k-steps) and O^T row tiles
     const int dm = PAD ? d_mem : D;  // head_dim of the rows in memory
-    using St = Stage<D>;
-    extern __shared__ __align__(16) char smem[];
+    using St = Stage<D, QW>;
+    using Sh = Shape<D, QW, KG>;
+    extern __shared__ __align__(16) char smem_all[];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5;
+    const int grp = KG > 1 ? wave / QW : 0;             // group of this wave
+    const int tg = threadIdx.x - grp * Sh::kGroupThreads;  // thread within the group
+    char* smem = smem_all + grp * 2 * St::kBytes;
     // Under the causal mask a query tile's work grows with its index, so the
     // grid is query-tile-major, heaviest tiles of every (b,h) first.  Without
     // it, the query tiles of one (b,h) share its K/V, so they run on one XCD
@@ -320,8 +328,8 @@ __global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void pref
         bh = tile / n_qtiles;
         qt = tile - bh * n_qtiles;
     }
-    constexpr int kQ = Shape<D>::kQ;
-    const int qw0 = qt * kQ + wave * 32;  // first query of this wave
+    constexpr int kQ = Sh::kQ;
+    const int qw0 = qt * kQ + (wave - grp * QW) * 32;  // first query of this wave
     const int q = qw0 + (lane & 31);      // this lane's query
     const bool qok = q < S;
 
@@ -362,21 +370,25 @@ __global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void pref
     const int kd = CAUSAL ? (qt * kQ) / kKV : 0;
     const int nd = n_kv - kd;
     auto tile_of = [&](int i) { return CAUSAL ? (i < nd ? kd + i : i - nd) : i; };
+    // This group's steps are walk positions grp, grp + KG, ...; every group runs the
+    // same number of steps (barriers), the last of them possibly past the end.
+    const int n_steps = (n_kv + KG - 1) / KG;
+    auto pos_of = [&](int step) { return step * KG + grp; };
 
     // The first tile's loads go out before the exponent's reduction, so their
     // latency overlaps it.
-    const TileSrc src = make_tile_src<D>(Kbh, Vbh, sKbh, sVbh, S, dm);
-    Prefetch<D> pa;
-    prefetch_tile<D, PAD>(pa, src, tile_of(0) * kKV);
+    const TileSrc src = make_tile_src<D, QW>(Kbh, Vbh, sKbh, sVbh, S, dm, tg);
+    Prefetch<D, QW> pa;
+    prefetch_tile<D, QW, PAD>(pa, src, tile_of(min(pos_of(0), n_kv - 1)) * kKV, tg);
 
     // E: the exponent that keeps the scaled V^T in fp16 range, from max |sV| over
     // the keys this block reads (a block-wide reduction through LDS).  Each thread
     // reads 16-byte vectors, kSvU of them in flight per round; dwords past kv_end
     // read as zero (the buffer range is checked per dword).
-    __shared__ float s_svmax[Shape<D>::kWaves];
+    __shared__ float s_svmax[QW * KG];
     {
         typedef float v4f __attribute__((ext_vector_type(4)));
-        constexpr int kT = Shape<D>::kThreads, kSvU = 4;
+        constexpr int kT = Sh::kThreads, kSvU = 4;
         const __amdgpu_buffer_rsrc_t svr = make_buffer(sVbh, (uint32_t)kv_end * 4);
         float a = 0.f;
         for (int j0 = 0; j0 < kv_end; j0 += 4 * kT * kSvU) {
@@ -408,7 +420,7 @@ __global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void pref
     __syncthreads();
     float svmax = s_svmax[0];
 #pragma unroll
-    for (int w = 1; w < Shape<D>::kWaves; ++w) svmax = fmaxf(svmax, s_svmax[w]);
+    for (int w = 1; w < QW * KG; ++w) svmax = fmaxf(svmax, s_svmax[w]);
     int vexp = 0;  // smallest E (up to kMaxVExp) with 127 max|sV| 2^-E <= 32768
     {
         const float need = svmax * (127.f / 32768.f);
@@ -446,7 +458,7 @@ __global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void pref
     typedef _Float16 v4h __attribute__((ext_vector_type(4)));
     typedef short v4s __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) v4s lds_v4s;
-    constexpr int kVRowB = 2 * VLayout<D>::kRow;  // bytes per staged V' row
+    constexpr int kVRowB = 2 * VLayout<D, QW>::kRow;  // bytes per staged V' row
     const int v_lane = (4 * (lane >> 5) + ((lane & 15) >> 2)) * kVRowB +
                        2 * (16 * ((lane >> 4) & 1) + 4 * (lane & 3));
     auto pv = [&](int kt, const v8h (&pfr)[4]) {
@@ -516,25 +528,26 @@ __global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void pref
     // to the other stage, refilled with step kt+2's tile, and the step's one
     // barrier follows.  The fast path runs as an inner loop that the slow path
     // leaves and re-enters, so O has no conditional update inside it.
-    commit_tile<D>(pa, smem, vscale);
-    if (n_kv > 1) prefetch_tile<D, PAD>(pa, src, tile_of(1) * kKV);
+    commit_tile<D, QW>(pa, smem, vscale, tg);
+    if (pos_of(1) < n_kv) prefetch_tile<D, QW, PAD>(pa, src, tile_of(pos_of(1)) * kKV, tg);
     __syncthreads();
     auto advance = [&](int kt) {
-        if (kt + 1 < n_kv) {
-            commit_tile<D>(pa, smem + ((kt + 1) & 1) * St::kBytes, vscale);
-            if (kt + 2 < n_kv) prefetch_tile<D, PAD>(pa, src, tile_of(kt + 2) * kKV);
+        if (pos_of(kt + 1) < n_kv) {
+            commit_tile<D, QW>(pa, smem + ((kt + 1) & 1) * St::kBytes, vscale, tg);
+            if (pos_of(kt + 2) < n_kv)
+                prefetch_tile<D, QW, PAD>(pa, src, tile_of(pos_of(kt + 2)) * kKV, tg);
         }
         // step kt+1's tile is in LDS and every wave is done reading stage kt&1
         __syncthreads();
     };
     bool have_m = false;  // wave-uniform: a slow step has set the running max
     int kt = 0;
-    while (kt < n_kv) {
+    while (kt < n_steps) {
         v16i sacc[2];
         bool slow = false;
-        for (; kt < n_kv; ++kt) {
-            const int tk = tile_of(kt);
-            if (computes(tk)) {
+        for (; kt < n_steps; ++kt) {
+            const int tk = tile_of(pos_of(kt));
+            if ((KG == 1 || pos_of(kt) < n_kv) && computes(tk)) {
                 const int k0 = tk * kKV;
                 const bool full = k0 + kKV <= S && !(CAUSAL && k0 + kKV - 1 > qw0);
                 if (!(full && qpos && have_m)) {
@@ -572,7 +585,7 @@ __global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void pref
         // Slow path for step kt (its S^T is in sacc): s = acc * qscale * sK with masked
         // keys at -inf, exact running max, rescale of O and l.
         {
-            const int k0 = tile_of(kt) * kKV;
+            const int k0 = tile_of(pos_of(kt)) * kKV;
             const float* sk_l = sk_of(kt);
             float sc[2][16];
             float mx = -INFINITY;
@@ -619,6 +632,39 @@ __global__ __launch_bounds__(Shape<D>::kThreads, Shape<D>::kMinBlocks) void pref
         ++kt;
     }
 
+    if constexpr (KG > 1) {
+        // Every group but the first leaves its waves' (m, l, O) in LDS (the stages are free
+        // after the last step's barrier), lane by lane; the first group's waves merge them.
+        constexpr int kWords = NS * 16 + 2;  // per lane, [word][lane]
+        static_assert((KG - 1) * QW * kWords * 64 * 4 <= KG * 2 * St::kBytes, "fits the stages");
+        float* ex = reinterpret_cast<float*>(smem_all) + lane;
+        if (grp > 0) {
+            float* e = ex + (wave - QW) * kWords * 64;
+            e[0] = m;
+            e[64] = lsum;
+#pragma unroll
+            for (int t = 0; t < NS; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) e[(2 + t * 16 + r) * 64] = o[t][r];
+        }
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; ++g) {
+            const float* e = ex + (g * QW + wave) * kWords * 64;
+            const float mg = e[0];
+            const float m_new = fmaxf(m, mg);
+            const float m_use = m_new == -INFINITY ? 0.f : m_new;
+            const float fa = fast_exp2(m - m_use), fb = fast_exp2(mg - m_use);
+            lsum = lsum * fa + e[64] * fb;
+#pragma unroll
+            for (int t = 0; t < NS; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    o[t][r] = o[t][r] * fa + e[(2 + t * 16 + r) * 64] * fb;
+            m = m_new;
+        }
+    }
     const float L = sum_xor32(lsum);
     if (!qok) return;  // lanes l and l^32 share q, so both leave or both stay
     // l carries the 2^E of P; O = sum p v sV does not
@@ -860,23 +906,24 @@ int set_lds_limit(PerDeviceOnce& once, int bytes, Kernels... kernels) {
 
 // D: the kernel's head_dim; dm: the head_dim of the rows in memory (dm <= D,
 // a multiple of 16; dm < D runs the padded instance).
-template <int D>
-int launch_prefill(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* out,
-                   int8_t* qout, float* qscale, const float* sQ, const float* sK, const float* sV,
-                   int BH, int heads, int S, int dm, bool causal, bool bshd, hipStream_t stream) {
-    constexpr int kQ = Shape<D>::kQ, kThreads = Shape<D>::kThreads;
+template <int D, int QW, int KG>
+int launch_prefill_shape(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* out,
+                         int8_t* qout, float* qscale, const float* sQ, const float* sK,
+                         const float* sV, int BH, int heads, int S, int dm, bool causal, bool bshd,
+                         hipStream_t stream) {
+    constexpr int kQ = Shape<D, QW, KG>::kQ, kThreads = Shape<D, QW, KG>::kThreads;
     const int n_qtiles = (S + kQ - 1) / kQ;
     const long long blocks = (long long)BH * n_qtiles;
     const float qk = (1.0f / std::sqrt((float)dm)) * kLog2e;
-    const int lds = 2 * Stage<D>::kBytes;
+    const int lds = KG * 2 * Stage<D, QW>::kBytes;
     static PerDeviceOnce lds_once;
-    const int st = set_lds_limit(lds_once, lds, prefill_kernel<D, true, false>,
-                                 prefill_kernel<D, false, false>, prefill_kernel<D, true, true>,
-                                 prefill_kernel<D, false, true>);
+    const int st = set_lds_limit(
+        lds_once, lds, prefill_kernel<D, QW, KG, true, false>, prefill_kernel<D, QW, KG, false, false>,
+        prefill_kernel<D, QW, KG, true, true>, prefill_kernel<D, QW, KG, false, true>);
     if (st != INT8K_OK) return st;
     const int b = bshd ? 1 : 0;
 #define INT8K_PREFILL_LAUNCH(C, P)                                                         \
-    prefill_kernel<D, C, P><<<(unsigned)blocks, kThreads, lds, stream>>>(                  \
+    prefill_kernel<D, QW, KG, C, P><<<(unsigned)blocks, kThreads, lds, stream>>>(          \
         Q, K, V, sQ, sK, sV, out, qout, qscale, S, n_qtiles, qk, heads, b, dm)
     if (dm == D) {
         if (causal) INT8K_PREFILL_LAUNCH(true, false);
@@ -887,6 +934,63 @@ int launch_prefill(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* 
     }
 #undef INT8K_PREFILL_LAUNCH
     return check_launch("prefill_kernel");
+}
+
+// The estimated time (0.01 us) of a block shape: a step (KG tiles) takes `step`, a
+// block's prologue, first tiles and epilogue `fixed` steps; `slots` blocks make
+// progress at once.  The grid is bound by its longest block or by its sum.
+struct ShapeCost {
+    int qw, kg, step, fixed_full, fixed_causal, slots;
+};
+inline long long shape_time(const ShapeCost& c, int BH, int S, bool causal) {
+    const long long kq = 32LL * c.qw, qt = ceil_div(S, kq);
+    auto steps = [&](long long keys) { return ceil_div(ceil_div(keys, kKV), c.kg); };
+    const long long longest = steps(S), shortest = causal ? steps(std::min<long long>(S, kq)) : longest;
+    const long long fixed = causal ? c.fixed_causal : c.fixed_full;
+    const long long blocks = (long long)BH * qt;
+    // equal blocks run in whole rounds; causal ones (heaviest first) fill the slots evenly
+    const long long sum =
+        causal ? (blocks * (longest + shortest + 2 * fixed) / 2 + c.slots - 1) / c.slots
+               : ceil_div(blocks, c.slots) * (longest + fixed);
+    return c.step * std::max(longest + fixed, sum);
+}
+
+// The costs fit runs of every shape at BH 8..128, S 100..8192.  us at the shape with the
+// most queries per block -> chosen: D = 64: BH 12 S 384 causal 13.8 -> 10.8, BH 12 S 1024
+// causal 24.6 -> 15.2, BH 32 S 1023 21.6 -> 17.4; D = 128: BH 32 S 256 causal 19.9 -> 11.7,
+// BH 32 S 1024 causal 38.7 -> 26.8, BH 8 S 8192 causal 208 -> 152, BH 32 S 1023 D = 80
+// 33.6 -> 24.5.  Another shape has to promise 5% over the first.
+template <int D>
+int launch_prefill(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* out,
+                   int8_t* qout, float* qscale, const float* sQ, const float* sK, const float* sV,
+                   int BH, int heads, int S, int dm, bool causal, bool bshd, hipStream_t stream) {
+    constexpr ShapeCost kCosts[3] = {
+        D == 64 ? ShapeCost{4, 1, 123, 4, 4, 512} : ShapeCost{8, 1, 200, 4, 4, 256},
+        D == 64 ? ShapeCost{4, 2, 144, 4, 6, 256} : ShapeCost{4, 2, 234, 4, 4, 256},
+        D == 64 ? ShapeCost{2, 4, 150, 5, 5, 256} : ShapeCost{2, 2, 195, 4, 4, 256}};
+    int pick = 0;
+    if constexpr (D <= 128) {
+        long long best = shape_time(kCosts[0], BH, S, causal) * 95 / 100;
+        for (int i = 1; i < 3; ++i) {
+            const long long t = shape_time(kCosts[i], BH, S, causal);
+            if (t < best) best = t, pick = i;
+        }
+    }
+#define INT8K_PREFILL_SHAPE(QW, KG)                                                           \
+    return launch_prefill_shape<D, QW, KG>(Q, K, V, out, qout, qscale, sQ, sK, sV, BH, heads, S, \
+                                           dm, causal, bshd, stream)
+    if constexpr (D == 64) {
+        if (pick == 1) INT8K_PREFILL_SHAPE(4, 2);
+        if (pick == 2) INT8K_PREFILL_SHAPE(2, 4);
+        INT8K_PREFILL_SHAPE(4, 1);
+    } else if constexpr (D == 128) {
+        if (pick == 1) INT8K_PREFILL_SHAPE(4, 2);
+        if (pick == 2) INT8K_PREFILL_SHAPE(2, 2);
+        INT8K_PREFILL_SHAPE(8, 1);
+    } else {
+        INT8K_PREFILL_SHAPE(4, 1);
+    }
+#undef INT8K_PREFILL_SHAPE
 }
 
 int launch_prefill_generic(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* out,
