@@ -1007,6 +1007,9 @@ int launch_decode_paged(const int8_t* Q, const int8_t* Kp, const int8_t* Vp, con
         g = one_launch ? GroupPlan{1, plan.nsplit, plan.chunk} : forced_groups(plan);
     else
         g = plan_groups(BH, max_context, D, NS, plan.nsplit);
+    // short chunks keep the plan's waves: more of them only add merges
+    if (g.blocks == 1 && one_launch && plan.chunk <= 4 * rows_per_iter(D, NS))
+        g = GroupPlan{1, plan.nsplit, plan.chunk};
     // page ids the rows of a block can span, staged in LDS
     const long long rows = (long long)g.waves * g.chunk;
     const long long n_tab = std::min<long long>(
