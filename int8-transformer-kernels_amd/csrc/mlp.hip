@@ -1188,12 +1188,15 @@ constexpr int kMidMaxBigTiles = 128;
 //    49; 2048 -> 8192, T = 64: 33 -> 28.5; with weights of at most 1 MiB up to 512
 //    rows (512 -> 2048, as stored);
 //  - packed weights of up to 4 MiB keep the skinny kernel to 2^30 multiply-adds, where
-//    a column tile of 128 leaves most CUs idle (1024 -> 4096, T = 64: 21 against 25);
+//    a column tile of 128 leaves most CUs idle (1024 -> 4096, T = 64: 21 against 25), if
+//    its own grid has at least 128 blocks (4096 -> 1024, T = 16: 32 blocks, GEMM and
+//    requantization 12.7 us, here 9.0);
 //  - then 128 x 128 tiles (split over K) to kMidMaxBigTiles: T = 333, 2048 -> 8192
 //    69 (split-K with a pass of its own for the epilogue and the requantization) ->
 //    45.6; T = 512, 1024 -> 4096 43 (skinny) -> 30; T = 512, 4096 -> 16384 172 -> 107.
 constexpr int kStreamRows = 128, kStreamRowsSmall = 512;
 constexpr long long kStreamSmallWeights = 1LL << 20, kSkinnyWeights = 1LL << 22;
+constexpr long long kSkinnyBlocks = 128;
 
 enum class Route { kStream, kSkinny, kMid, kTiled };
 
@@ -1201,7 +1204,8 @@ Route gemm_route(int M, int N, int K, bool packed) {
     const long long nk = (long long)N * K;
     const long long big_tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     const bool skinny = packed && N % kSkinnyN == 0 && K % 512 == 0 && nk <= kSkinnyWeights &&
-                        M * nk <= (1LL << 30);
+                        M * nk <= (1LL << 30) &&
+                        (long long)(N / kSkinnyN) * ((M + 31) / 32) >= kSkinnyBlocks;
     const int stream_rows = nk <= kStreamSmallWeights ? kStreamRowsSmall : kStreamRows;
     if (M <= stream_rows && N <= kRowsEpiMaxN && K < (1 << 24) && !skinny) return Route::kStream;
     if (skinny) return Route::kSkinny;
