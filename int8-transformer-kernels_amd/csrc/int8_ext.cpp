@@ -35,9 +35,22 @@ void check_status(int st, const char* op) {
                 (detail && detail[0]) ? std::string(" — ") + detail : std::string());
 }
 
-torch::Tensor workspace(size_t bytes, const torch::Device& dev) {
-    return torch::empty({(int64_t)std::max<size_t>(bytes, 1)},
-                        torch::TensorOptions().dtype(torch::kUInt8).device(dev));
+// Scratch of a call; none where the call needs none.
+struct Workspace {
+    torch::Tensor t;
+    void* data() const { return t.defined() ? t.data_ptr() : nullptr; }
+};
+
+Workspace workspace(size_t bytes, const torch::Device& dev) {
+    if (bytes == 0) return {};
+    return {torch::empty({(int64_t)bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(dev))};
+}
+
+// A scale tensor of n elements in row-major order, whatever its shape.  (A flat view
+// of it, which checks the same, costs a tensor per scale: 0.3 us each on calls of 6.)
+torch::Tensor flat_scale(const torch::Tensor& s, int64_t n, const char* name) {
+    TORCH_CHECK(s.numel() == n, name, " must have ", n, " elements, has ", s.numel());
+    return s.contiguous();
 }
 
 bool aligned16(const torch::Tensor& t) {
@@ -88,9 +101,9 @@ static std::vector<torch::Tensor> attention_impl(torch::Tensor Q, torch::Tensor 
                 "prefill attention supports head_dim 1..512");
     TORCH_CHECK(seq_len >= 1 && batch * heads * seq_len <= INT32_MAX, "seq_len out of range");
     const int64_t n_tokens = batch * heads * seq_len;
-    auto sQ = scale_Q.contiguous().view({n_tokens});
-    auto sK = scale_K.contiguous().view({n_tokens});
-    auto sV = scale_V.contiguous().view({n_tokens});
+    auto sQ = flat_scale(scale_Q, n_tokens, "scale_Q");
+    auto sK = flat_scale(scale_K, n_tokens, "scale_K");
+    auto sV = flat_scale(scale_V, n_tokens, "scale_V");
     auto q = aligned_i8(Q), k = aligned_i8(K), v = aligned_i8(V);
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(Q.device());
     const int flags = (is_causal ? INT8K_ATTN_CAUSAL : 0) | (out_bshd ? INT8K_ATTN_OUT_BSHD : 0);
@@ -172,9 +185,9 @@ static std::vector<torch::Tensor> decode_impl(torch::Tensor Q, torch::Tensor K, 
 
     const int64_t BH = batch * heads;
     TORCH_CHECK(BH <= INT32_MAX && seq_kv <= INT32_MAX, "decode shape too large");
-    auto sQ = scale_Q.contiguous().view({BH});
-    auto sK = scale_K.contiguous().view({BH * seq_kv});
-    auto sV = scale_V.contiguous().view({BH * seq_kv});
+    auto sQ = flat_scale(scale_Q, BH, "scale_Q");
+    auto sK = flat_scale(scale_K, BH * seq_kv, "scale_K");
+    auto sV = flat_scale(scale_V, BH * seq_kv, "scale_V");
     auto q = aligned_i8(Q), k = aligned_i8(K), v = aligned_i8(V);
 
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(Q.device());
@@ -190,7 +203,7 @@ static std::vector<torch::Tensor> decode_impl(torch::Tensor Q, torch::Tensor K, 
                          q.data_ptr<int8_t>(), k.data_ptr<int8_t>(), v.data_ptr<int8_t>(),
                          oq.data_ptr<int8_t>(), os.data_ptr<float>(), sQ.data_ptr<float>(),
                          sK.data_ptr<float>(), sV.data_ptr<float>(), (int)BH, (int)seq_kv,
-                         (int)head_dim, 0, ws.data_ptr(), ws_bytes, current_stream(Q)),
+                         (int)head_dim, 0, ws.data(), ws_bytes, current_stream(Q)),
                      "int8_decode_attention_forward_quant");
         return {oq, os};
     }
@@ -200,7 +213,7 @@ static std::vector<torch::Tensor> decode_impl(torch::Tensor Q, torch::Tensor K, 
         q.data_ptr<int8_t>(), k.data_ptr<int8_t>(), v.data_ptr<int8_t>(),
         reinterpret_cast<uint16_t*>(out.data_ptr<at::Half>()), sQ.data_ptr<float>(),
         sK.data_ptr<float>(), sV.data_ptr<float>(), (int)BH, (int)seq_kv, (int)head_dim, 0,
-        ws.data_ptr(), ws_bytes, current_stream(Q));
+        ws.data(), ws_bytes, current_stream(Q));
     check_status(st, "int8_decode_attention_forward");
     return {out};
 }
@@ -300,7 +313,7 @@ std::tuple<torch::Tensor, torch::Tensor> run_mlp(const torch::Tensor& x, const t
         out.data_ptr<int8_t>(), sx.data_ptr<float>(), (int)sx.numel(), sw1.data_ptr<float>(),
         (int)sw1.numel(), sw2.data_ptr<float>(), (int)sw2.numel(),
         bias1 ? bias1->data_ptr<float>() : nullptr, out_scale.data_ptr<float>(), (int)d.T,
-        (int)d.d_model, (int)d.d_ff, flags, ws.data_ptr(), ws_bytes, current_stream(x));
+        (int)d.d_model, (int)d.d_ff, flags, ws.data(), ws_bytes, current_stream(x));
     check_status(st, "int8_mlp_forward");
     return {out, out_scale};
 }
@@ -645,7 +658,7 @@ static std::vector<torch::Tensor> decode_cache_impl(torch::Tensor Q, torch::Tens
                          Q.data_ptr<int8_t>(), K_cache.data_ptr<int8_t>(),
                          V_cache.data_ptr<int8_t>(), oq.data_ptr<int8_t>(), os.data_ptr<float>(),
                          sQ.data_ptr<float>(), sK.data_ptr<float>(), sV.data_ptr<float>(), BH,
-                         (int)seq_len, (int)cap, (int)D, 0, ws.data_ptr(), ws_bytes,
+                         (int)seq_len, (int)cap, (int)D, 0, ws.data(), ws_bytes,
                          current_stream(Q)),
                      "int8_decode_attention_forward_cache_quant");
         return {oq, os};
@@ -655,7 +668,7 @@ static std::vector<torch::Tensor> decode_cache_impl(torch::Tensor Q, torch::Tens
         Q.data_ptr<int8_t>(), K_cache.data_ptr<int8_t>(), V_cache.data_ptr<int8_t>(),
         reinterpret_cast<uint16_t*>(out.data_ptr<at::Half>()), sQ.data_ptr<float>(),
         sK.data_ptr<float>(), sV.data_ptr<float>(), BH, (int)seq_len, (int)cap, (int)D, 0,
-        ws.data_ptr(), ws_bytes, current_stream(Q));
+        ws.data(), ws_bytes, current_stream(Q));
     check_status(st, "int8_decode_attention_forward_cache");
     return {out};
 }
@@ -723,7 +736,7 @@ static std::vector<torch::Tensor> decode_paged_impl(
                          V_pages.data_ptr<int8_t>(), oq.data_ptr<int8_t>(), os.data_ptr<float>(),
                          sQ.data_ptr<float>(), sK.data_ptr<float>(), sV.data_ptr<float>(),
                          bt.data_ptr<int32_t>(), cl.data_ptr<int32_t>(), (int)B, (int)H, (int)D,
-                         (int)NP, (int)P, (int)max_pages, (int)max_context, 0, ws.data_ptr(),
+                         (int)NP, (int)P, (int)max_pages, (int)max_context, 0, ws.data(),
                          ws_bytes, current_stream(Q)),
                      "int8_decode_attention_forward_paged_quant");
         return {oq, os};
@@ -734,7 +747,7 @@ static std::vector<torch::Tensor> decode_paged_impl(
         reinterpret_cast<uint16_t*>(out.data_ptr<at::Half>()), sQ.data_ptr<float>(),
         sK.data_ptr<float>(), sV.data_ptr<float>(), bt.data_ptr<int32_t>(),
         cl.data_ptr<int32_t>(), (int)B, (int)H, (int)D, (int)NP, (int)P, (int)max_pages,
-        (int)max_context, 0, ws.data_ptr(), ws_bytes, current_stream(Q));
+        (int)max_context, 0, ws.data(), ws_bytes, current_stream(Q));
     check_status(st, "int8_decode_attention_forward_paged");
     return {out};
 }
