@@ -1380,10 +1380,11 @@ int launch_rows_epilogue(const int32_t* partial, int splits, int M, int N, const
 // One block per row: reduce the row's absmax partials, then requantize the
 // fp16 row to int8 with scale max(amax,1e-8)/127 (quantize_rows semantics).
 // With `tensor_amax` set, that single value is used for every row instead
-// and `scales` receives it once (per-tensor output quantization).
+// and `scales` receives it once (per-tensor output quantization); with tensor_n
+// set, it is the max of the first tensor_n partials (few: every block takes it).
 __global__ __launch_bounds__(256) void requant_rows_kernel(
     const uint16_t* __restrict__ h, int ldh, const float* __restrict__ pmax, int tiles_n,
-    const float* __restrict__ tensor_amax, int8_t* __restrict__ q, int ldq,
+    const float* __restrict__ tensor_amax, int tensor_n, int8_t* __restrict__ q, int ldq,
     float* __restrict__ scales, int M, int N) {
     __shared__ float red[4];
     const int row = blockIdx.x;
@@ -1392,7 +1393,12 @@ __global__ __launch_bounds__(256) void requant_rows_kernel(
         amax = *tensor_amax;
     } else {
         float m = 0.f;
-        for (int t = threadIdx.x; t < tiles_n; t += 256) m = fmaxf(m, pmax[(size_t)t * M + row]);
+        if (tensor_n > 0) {
+#pragma unroll 4
+            for (int t = threadIdx.x; t < tensor_n; t += 256) m = fmaxf(m, pmax[t]);
+        } else {
+            for (int t = threadIdx.x; t < tiles_n; t += 256) m = fmaxf(m, pmax[(size_t)t * M + row]);
+        }
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -1401,8 +1407,8 @@ __global__ __launch_bounds__(256) void requant_rows_kernel(
     }
     amax = fmaxf(amax, 1e-8f);
     const float inv = 127.f / amax;
-    if (threadIdx.x == 0 && (tensor_amax == nullptr || row == 0))
-        scales[tensor_amax == nullptr ? row : 0] = amax / 127.f;
+    const bool tensor = tensor_amax != nullptr || tensor_n > 0;
+    if (threadIdx.x == 0 && (!tensor || row == 0)) scales[tensor ? 0 : row] = amax / 127.f;
     const uint16_t* hr = h + (size_t)row * ldh;
     int8_t* qr = q + (size_t)row * ldq;
     auto quant = [inv](uint16_t bits) -> int {
@@ -1481,18 +1487,21 @@ __global__ __launch_bounds__(256) void requant_rows_wave_kernel(
 // of up to 2048 columns when there are enough rows to fill the chip (at
 // T = 16384, 1024 columns: 17.1 -> 12.3 us), else one block per row.
 int launch_requant(const uint16_t* h, int ldh, const float* pmax, int tiles_n,
-                   const float* tensor_amax, int8_t* q, int ldq, float* scales, int M, int N,
-                   hipStream_t s) {
-    if (M >= 512 && N <= 2048 && N % 8 == 0 && ldh % 8 == 0 && ldq % 8 == 0 &&
+                   const float* tensor_amax, int tensor_n, int8_t* q, int ldq, float* scales, int M,
+                   int N, hipStream_t s) {
+    if (tensor_n == 0 && M >= 512 && N <= 2048 && N % 8 == 0 && ldh % 8 == 0 && ldq % 8 == 0 &&
         aligned_to(h, 16) && aligned_to(q, 8)) {
         requant_rows_wave_kernel<<<(M + 3) / 4, 256, 0, s>>>(h, ldh, pmax, tiles_n, tensor_amax,
                                                              q, ldq, scales, M, N);
         return check_launch("requant_rows_wave_kernel");
     }
-    requant_rows_kernel<<<M, 256, 0, s>>>(h, ldh, pmax, tiles_n, tensor_amax, q, ldq, scales, M,
-                                          N);
+    requant_rows_kernel<<<M, 256, 0, s>>>(h, ldh, pmax, tiles_n, tensor_amax, tensor_n, q, ldq,
+                                          scales, M, N);
     return check_launch("requant_rows_kernel");
 }
+
+// Most absmax partials that every block of the per-tensor requantization reduces.
+constexpr size_t kTensorPartials = 8192;
 
 // Max over all partials (per-tensor output scale), one block.
 __global__ __launch_bounds__(256) void tensor_absmax_kernel(const float* __restrict__ pmax,
@@ -1949,8 +1958,8 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
     if (st != INT8K_OK) return st;
     // per-token requant of the fp16 hidden
     if (!pl.direct1 && !pl.a16 &&
-        (st = launch_requant(w.h16, d_ff, w.p1, pl.g1.epi_tiles, nullptr, w.hq, d_ff, w.sh, T, d_ff,
-                             s)) != INT8K_OK)
+        (st = launch_requant(w.h16, d_ff, w.p1, pl.g1.epi_tiles, nullptr, 0, w.hq, d_ff, w.sh, T,
+                             d_ff, s)) != INT8K_OK)
         return st;
     // GEMM2 + dequant epilogue -> int8 output + scales, or fp16 output + absmax partials for
     // the separate pass
@@ -1973,12 +1982,16 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
                                out, out_scale, amax2, arrived2, w.part, s);
     }
     if (st != INT8K_OK || pl.direct2) return st;
+    // per-tensor output: few partials are reduced by the requantization itself (a launch
+    // less: T = 100, 1024 -> 4096 27.1 -> 24.3 us), more of them by a kernel before it
     const float* tmax = nullptr;
-    if (per_tensor_out) {
-        tensor_absmax_kernel<<<1, 256, 0, s>>>(w.p2, (size_t)pl.g2.epi_tiles * T, w.tmax);
+    const size_t n_part = (size_t)pl.g2.epi_tiles * T;
+    const int tensor_n = per_tensor_out && n_part <= kTensorPartials && T < 512 ? (int)n_part : 0;
+    if (per_tensor_out && tensor_n == 0) {
+        tensor_absmax_kernel<<<1, 256, 0, s>>>(w.p2, n_part, w.tmax);
         if ((st = check_launch("tensor_absmax_kernel")) != INT8K_OK) return st;
         tmax = w.tmax;
     }
-    return launch_requant(w.o16, d_model, w.p2, pl.g2.epi_tiles, tmax, out, d_model, out_scale, T,
-                          d_model, s);
+    return launch_requant(w.o16, d_model, w.p2, pl.g2.epi_tiles, tmax, tensor_n, out, d_model,
+                          out_scale, T, d_model, s);
 }
