@@ -74,6 +74,10 @@ constexpr long long kVecBlocks = 8192;
 // LayerNorm keeps gamma and beta in registers over a wave's rows: a grid of 4
 // blocks per CU, so that many rows share one read of them.
 constexpr long long kLnBlocks = 1024;
+// Elements per lane of the longest row of layernorm_quant_row_kernel (768 columns).
+// One wave per row loses from 1280 columns on, where a block per row loads more in
+// parallel: 4000 rows fp16, block -> wave: 24.2 -> 26.1 us at 1280, 31.0 -> 42.1 at 1600.
+constexpr int kRowElems = 12;
 
 template <typename Op>
 __device__ __forceinline__ float wave_reduce(float v, Op op) {
@@ -200,66 +204,46 @@ __device__ __forceinline__ void load_affine(const float* p, int col0, bool vec, 
 // LayerNorm + per-token quantizer with the row in registers: 1 << lg lanes per
 // row, NC 16-byte chunks per lane.  One read of x; the passes of the
 // one-element-per-lane kernel above become register passes.  PAD: slots past the
-// row repeat its last chunk and count for nothing in the sums.  ROWBLOCK: the 256
-// threads of a block hold one row (rows of more than kWaveRowChunks chunks, where one
-// wave would need 8 or more chunks per lane: 150-280 registers, 1-3 waves per
-// SIMD), reduced across the four waves through LDS.
-// HBM-bound, and latency-bound for few rows.  us with gamma and beta, before (one
-// element per lane, or gamma and beta element by element) -> here: 4000 x 768 bf16
-// 18.2 -> 7.1 (kernel time), 16384 x 1024 fp16 66 -> 16.7, 4096 x 8192 bf16 155 -> 30,
-// 100000 x 80 fp16 155 -> 16.7.
-constexpr int kWaveRowChunks = 256;
-
-template <int DT, int NC, bool PAD, bool ROWBLOCK>
+// row repeat its last chunk and count for nothing in the sums.  gamma and beta stay in
+// registers over a wave's rows where they fit (up to 4 chunks per lane): re-read per
+// row they are up to 4x the bytes of x through L2.
+// HBM-bound, and latency-bound for few rows.  us with gamma and beta, element by
+// element -> as vectors: 16384 x 1024 fp16 66 -> 16.7, 8192 x 5120 fp16 180 -> 63, 4096
+// x 8192 bf16 155 -> 66.
+template <int DT, int NC, bool PAD>
 __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
     const void* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
     float eps, int8_t* __restrict__ q, float* __restrict__ scales, void* __restrict__ y_out,
     uint32_t rows, int lg, uint32_t cpr, int affine_vec) {
     constexpr int W = Vec<DT>::W;
-    __shared__ float red[3][kWaves];
+    constexpr bool kHold = NC <= 4;  // gamma and beta in registers
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    if (ROWBLOCK) lg = 6;
     const uint32_t rpw = 64u >> lg;
-    const uint32_t c0 = ROWBLOCK ? threadIdx.x : lane & ((1u << lg) - 1);
-    const int slg = ROWBLOCK ? 8 : lg;  // chunks between a lane's slots, as a power of two
-    if (!PAD) cpr = (uint32_t)NC << slg;
-    auto real = [&](int i) { return !PAD || ((uint32_t)i << slg) + c0 < cpr; };
+    const uint32_t c0 = lane & ((1u << lg) - 1);
+    if (!PAD) cpr = (uint32_t)NC << lg;
+    auto real = [&](int i) { return !PAD || ((uint32_t)i << lg) + c0 < cpr; };
+    auto col_of = [&](int i) { return (int)(slot_chunk<PAD>(i, lg, c0, cpr) * W); };
     const int cols = (int)cpr * W;
-    // 1 / cols is exact where the row fills every slot (a power of two)
     const float inv_cols = 1.f / (float)cols;
-    auto over_cols = [&](float v) { return PAD ? v / (float)cols : v * inv_cols; };
     const uint4* src = reinterpret_cast<const uint4*>(x);
     auto add = [](float a, float b) { return a + b; };
-    auto mx = [](float a, float b) { return fmaxf(a, b); };
-    auto reduce = [&](float v, int k, auto op) {
-        v = row_reduce(v, lg, op);
-        if constexpr (ROWBLOCK) {
-            if (lane == 0) red[k][wave] = v;
-            __syncthreads();
-            v = op(op(red[k][0], red[k][1]), op(red[k][2], red[k][3]));
-        }
-        return v;
-    };
-    // gamma and beta stay in registers over the rows of a wave: re-read per row they
-    // are up to 4x the bytes of x through L2
-    float eg[NC][W], eb[NC][W];
+    float eg[kHold ? NC : 1][W], eb[kHold ? NC : 1][W];
+    if constexpr (kHold) {
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        const int col0 = (int)(slot_chunk<PAD>(i, slg, c0, cpr) * W);
-        if (gamma) load_affine<W>(gamma, col0, affine_vec, eg[i]);
-        if (beta) load_affine<W>(beta, col0, affine_vec, eb[i]);
+        for (int i = 0; i < NC; ++i) {
+            if (gamma) load_affine<W>(gamma, col_of(i), affine_vec, eg[i]);
+            if (beta) load_affine<W>(beta, col_of(i), affine_vec, eb[i]);
+        }
     }
-    const uint32_t step = gridDim.x * (ROWBLOCK ? 1u : 4u * rpw);
-    for (uint32_t rb = ROWBLOCK ? blockIdx.x : (blockIdx.x * 4 + wave) * rpw; rb < rows;
-         rb += step) {
+    const uint32_t nw = gridDim.x * 4;
+    for (uint32_t rb = (blockIdx.x * 4 + (threadIdx.x >> 6)) * rpw; rb < rows; rb += nw * rpw) {
         // rows past the end take the last row and store it again (the same bytes
         // its own lane stores): no divergent branch around loads or stores
-        const uint32_t r = ROWBLOCK ? rb : min(rb + (lane >> lg), rows - 1);
+        const uint32_t r = min(rb + (lane >> lg), rows - 1);
         uint4 w[NC];
 #pragma unroll
         for (int i = 0; i < NC; ++i)
-            w[i] = src[(size_t)r * cpr + slot_chunk<PAD>(i, slg, c0, cpr)];
+            w[i] = src[(size_t)r * cpr + slot_chunk<PAD>(i, lg, c0, cpr)];
         float sum = 0.f;
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
@@ -268,7 +252,7 @@ __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
 #pragma unroll
             for (int e = 0; e < W; ++e) sum += real(i) ? v[e] : 0.f;
         }
-        const float mean = over_cols(reduce(sum, 0, add));
+        const float mean = row_reduce(sum, lg, add) * inv_cols;
 #pragma unroll
         for (int i = 0; i < NC; ++i) reload_barrier(w[i]);
         float var = 0.f;
@@ -282,11 +266,14 @@ __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
                 var = fmaf(d, d, var);
             }
         }
-        const float rstd = 1.f / sqrtf(over_cols(reduce(var, 1, add)) + eps);
+        const float rstd = 1.f / sqrtf(row_reduce(var, lg, add) * inv_cols + eps);
 #pragma unroll
         for (int i = 0; i < NC; ++i) reload_barrier(w[i]);
         // y, rounded to the dtype, replaces x in the chunk registers (its storage
         // bits: unpacking them gives the rounded values back exactly)
+        const float* g = gamma;
+        const float* bt = beta;
+        asm volatile("" : "+s"(g), "+s"(bt));  // re-read here, not hoisted (!kHold)
         float m = 0.f;
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
@@ -295,12 +282,16 @@ __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
 #pragma unroll
             for (int e = 0; e < W; ++e) y[e] = (y[e] - mean) * rstd;
             if (gamma) {
+                float p[W];
+                if constexpr (!kHold) load_affine<W>(g, col_of(i), affine_vec, p);
 #pragma unroll
-                for (int e = 0; e < W; ++e) y[e] *= eg[i][e];
+                for (int e = 0; e < W; ++e) y[e] *= kHold ? eg[kHold ? i : 0][e] : p[e];
             }
             if (beta) {
+                float p[W];
+                if constexpr (!kHold) load_affine<W>(bt, col_of(i), affine_vec, p);
 #pragma unroll
-                for (int e = 0; e < W; ++e) y[e] += eb[i][e];
+                for (int e = 0; e < W; ++e) y[e] += kHold ? eb[kHold ? i : 0][e] : p[e];
             }
 #pragma unroll
             for (int e = 0; e < W; ++e) {
@@ -309,17 +300,81 @@ __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
             }
             w[i] = pack_chunk<DT>(y);
         }
-        const float sc = fmaxf(reduce(m, 2, mx), 1e-8f) / 127.f;
+        const float sc = fmaxf(row_reduce(m, lg, [](float a, float b) { return fmaxf(a, b); }),
+                               1e-8f) / 127.f;
         const float inv = 1.f / sc;
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
             float y[W];
             unpack_chunk<DT>(w[i], y);
-            const size_t chunk = (size_t)r * cpr + slot_chunk<PAD>(i, slg, c0, cpr);
+            const size_t chunk = (size_t)r * cpr + slot_chunk<PAD>(i, lg, c0, cpr);
             store_codes<W>(y, sc, inv, q + chunk * W);
             if (y_out) reinterpret_cast<uint4*>(y_out)[chunk] = w[i];
         }
         if (c0 == 0) scales[r] = sc;
+    }
+}
+
+// Short rows whose chunks fill neither a power of two of lanes nor whole waves (80, 768
+// columns): one wave per row, the row in registers, one element per lane and
+// 64 columns (NE of them).  The sums keep the order of layernorm_quant_kernel, whose
+// thread t + 64 w is this lane's column group w modulo 4, so both give the same
+// bytes: a code on a rounding tie follows the last bit of mean and rstd.  One read of
+// x instead of five.  Against a block per row, launches included: 100000 x 80 fp16
+// 155 -> 46 us, 4000 x 768 bf16 15.3 -> 13.5 us.
+template <int DT, int NE>
+__global__ __launch_bounds__(256) void layernorm_quant_row_kernel(
+    const void* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
+    float eps, int8_t* __restrict__ q, float* __restrict__ scales, void* __restrict__ y_out,
+    long long rows, int cols) {
+    const int lane = threadIdx.x & 63;
+    auto add = [](float a, float b) { return a + b; };
+    // the four waves' sums of a block, each over its 64 lanes, then in wave order
+    auto block_sum = [&](const float (&s)[4]) {
+        float r = row_reduce(s[0], 6, add);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) r = r + row_reduce(s[w], 6, add);
+        return r;
+    };
+    for (long long row = (long long)blockIdx.x * kWaves + (threadIdx.x >> 6); row < rows;
+         row += (long long)gridDim.x * kWaves) {
+        const size_t base = (size_t)row * (size_t)cols;
+        float v[NE];
+#pragma unroll
+        for (int k = 0; k < NE; ++k) v[k] = load_any(x, base + min(lane + 64 * k, cols - 1), DT);
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < NE; ++k) s[k & 3] += lane + 64 * k < cols ? v[k] : 0.f;
+        const float mean = block_sum(s) / (float)cols;
+        float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < NE; ++k) {
+            const float d = lane + 64 * k < cols ? v[k] - mean : 0.f;
+            t[k & 3] = fmaf(d, d, t[k & 3]);
+        }
+        const float rstd = 1.f / sqrtf(block_sum(t) / (float)cols + eps);
+        float m = 0.f;
+#pragma unroll
+        for (int k = 0; k < NE; ++k) {
+            const int c = min(lane + 64 * k, cols - 1);
+            float y = (v[k] - mean) * rstd;
+            if (gamma) y *= gamma[c];
+            if (beta) y += beta[c];
+            // past the row: the last column's x with the last column's parameters
+            v[k] = round_to(y, DT);
+            m = fmaxf(m, fabsf(v[k]));
+        }
+        const float sc =
+            fmaxf(row_reduce(m, 6, [](float a, float b) { return fmaxf(a, b); }), 1e-8f) / 127.f;
+#pragma unroll
+        for (int k = 0; k < NE; ++k) {
+            const int c = lane + 64 * k;
+            if (c < cols) {
+                q[base + c] = quantize(v[k], sc);
+                if (y_out) store_any(y_out, base + c, v[k], DT);
+            }
+        }
+        if (lane == 0) scales[row] = sc;
     }
 }
 
@@ -398,36 +453,35 @@ extern "C" int int8k_layernorm_quantize_per_token(const void* x, int dtype, cons
     hipStream_t st = as_stream(stream);
     const RowShape sh = row_shape(cols, dtype);
     const int w = dtype == INT8K_DTYPE_F32 ? 4 : 8;
-    if (sh.ok && rows < (1LL << 31) && aligned_to(x, 16) && aligned_to(q, w) &&
+    // rows that fill a power of two of lanes, or whole waves
+    const bool fills = sh.ok && (sh.nc == 1 ? sh.cpr == 1 << sh.lg : sh.cpr % 64 == 0);
+    if (fills && rows < (1LL << 31) && aligned_to(x, 16) && aligned_to(q, w) &&
         (!y_out || aligned_to(y_out, 16))) {
         const long long waves = ceil_div(rows, 64 >> sh.lg);
-        const bool row_block = sh.cpr > kWaveRowChunks;
-        const unsigned blocks =
-            (unsigned)std::min(row_block ? rows : ceil_div(waves, 4), kLnBlocks);
+        const unsigned blocks = (unsigned)std::min(ceil_div(waves, 4), kLnBlocks);
         const int affine_vec =
             (!gamma || aligned_to(gamma, 16)) && (!beta || aligned_to(beta, 16));
-        auto launch = [&](auto dt, auto nc, auto pad, auto rbk) {
-            layernorm_quant_vec_kernel<decltype(dt)::value, decltype(nc)::value,
-                                       decltype(pad)::value, decltype(rbk)::value>
-                <<<blocks, 256, 0, st>>>(x, gamma, beta, eps, q, scales, y_out, (uint32_t)rows,
-                                         sh.lg, (uint32_t)sh.cpr, affine_vec);
-        };
         with_dtype(dtype, [&](auto dt) {
-            if (row_block) {
-                if (sh.cpr <= 512)
-                    launch(dt, std::integral_constant<int, 2>{}, std::true_type{}, std::true_type{});
-                else if (sh.cpr <= 768)
-                    launch(dt, std::integral_constant<int, 3>{}, std::true_type{}, std::true_type{});
-                else
-                    launch(dt, std::integral_constant<int, 4>{}, std::true_type{}, std::true_type{});
-                return;
-            }
             with_chunks(sh, [&](auto ncc, auto pad) {
-                if constexpr (decltype(ncc)::value <= kWaveRowChunks / 64)
-                    launch(dt, ncc, pad, std::false_type{});
+                layernorm_quant_vec_kernel<decltype(dt)::value, decltype(ncc)::value,
+                                           decltype(pad)::value>
+                    <<<blocks, 256, 0, st>>>(x, gamma, beta, eps, q, scales, y_out,
+                                             (uint32_t)rows, sh.lg, (uint32_t)sh.cpr, affine_vec);
             });
         });
         return check_launch("layernorm_quant_vec_kernel");
+    }
+    if (cols <= 64 * kRowElems) {
+        const unsigned blocks = (unsigned)std::min(ceil_div(rows, kWaves), kMaxBlocks);
+        with_dtype(dtype, [&](auto dt) {
+            auto launch = [&](auto ne) {
+                layernorm_quant_row_kernel<decltype(dt)::value, decltype(ne)::value>
+                    <<<blocks, 256, 0, st>>>(x, gamma, beta, eps, q, scales, y_out, rows, cols);
+            };
+            if (cols <= 256) launch(std::integral_constant<int, 4>{});
+            else launch(std::integral_constant<int, kRowElems>{});
+        });
+        return check_launch("layernorm_quant_row_kernel");
     }
     layernorm_quant_kernel<<<(unsigned)std::min(rows, kMaxBlocks), 256, 0, st>>>(
         x, dtype, gamma, beta, eps, q, scales, y_out, rows, cols);

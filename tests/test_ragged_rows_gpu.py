@@ -1,8 +1,9 @@
 """Row kernels at row lengths that do not fill their lanes: 16-byte chunk counts around the
-powers of two, the per-lane instances (1, 2, 3, 4, 6, 8, 12, 16) and the switch to one block
-per row, where the last chunk is repeated in the spare slots.  The quantizers are exact
-against the oracle; LayerNorm as in test_producer_gpu.py: one storage ulp of y (its fp32 row
-sums differ from float64 by ~sqrt(cols) roundings, covered by 2^-17 relative for fp32)."""
+powers of two, the per-lane instances (1, 2, 3, 4, 6, 8, 12, 16), where the last chunk is
+repeated in the spare slots, and LayerNorm's switch to a block per row above 768 columns.
+The quantizers are exact against the oracle; LayerNorm as in test_producer_gpu.py: one
+storage ulp of y (its fp32 row sums differ from float64 by ~sqrt(cols) roundings, covered by
+2^-17 relative for fp32)."""
 import numpy as np
 import pytest
 import torch
@@ -13,7 +14,7 @@ from oracle import int8_oracle as O
 pytestmark = pytest.mark.gpu
 
 _DT = {torch.float16: "f16", torch.bfloat16: "bf16", torch.float32: "f32"}
-COLS = [8, 24, 80, 520, 776, 1600, 2040, 2056, 2568, 4096, 5128, 6152, 8184, 8200]
+COLS = [8, 24, 80, 520, 768, 776, 1600, 2040, 2056, 2568, 4096, 5128, 6152, 8184, 8200]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
