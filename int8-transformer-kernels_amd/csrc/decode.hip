@@ -170,10 +170,10 @@ constexpr int kNumCus = 256;
 // Automatic plans of the 8-wave kernels take the blocks per (b,h) (at most `most`)
 // with the smallest cost in wave iterations: a round is one block on each CU,
 // a block costs its waves' iterations plus about 2 for its first loads and its
-// merge, and the second launch about 6 at D = 64 and 2.5 at D = 128 (a CU streams
+// merge, and the second launch about 4 at D = 64 and 2 at D = 128 (a CU streams
 // one block at ~55 GB/s: 1.27 and 2.5 us per iteration).  So short sequences stay
-// on one block (paged B4 H16 D64 4000 rows: 15.7 us, 16.4 on four and a combine)
-// and longer ones spread (B1 H12 D64 4096 rows: 13.2 -> 12.3 us on 8 blocks,
+// on one block (B1 H16 D128 1500 rows, B1 H12 D64 2500 rows) and longer ones spread
+// (paged B4 H16 D64 4000 rows: 15.7 us on one block, 10.4 on four and a combine; B1 H12 D64 4096 rows: 13.2 -> 12.3 us on 8 blocks,
 // B1 H8 D128 3000 rows 19.6 -> 12.2, B4 H12 D128 2500 rows 18.4 -> 12.3).
 // Sweeps of 1..32 blocks at 8 to 64 (b,h) put the best time at one full round or
 // within 3% of it (B2 H8 D128 60013 rows: 53.2 / 44.1 / 46.0 us at 8 / 16 / 32
@@ -189,7 +189,7 @@ GroupPlan plan_groups(int BH, int S, int D, int slots, long long most) {
         const long long pw = ceil_div(iters, nb * kGroupWaves);
         const long long bl = ceil_div(iters, pw * kGroupWaves);
         const long long rounds = ceil_div(BH * bl, kNumCus);
-        const long long cost = 2 * rounds * (pw + 2) + (bl > 1 ? (D == 128 ? 5 : 12) : 0);
+        const long long cost = 2 * rounds * (pw + 2) + (bl > 1 ? (D == 128 ? 4 : 8) : 0);
         if (best < 0 || cost < best) best = cost, per_wave = pw, blocks = bl;
     }
     const int waves = (int)std::min<long long>(kGroupWaves, ceil_div(iters, per_wave));
