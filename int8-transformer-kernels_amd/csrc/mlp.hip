@@ -1176,9 +1176,10 @@ inline MidPlan mid_plan(int M, int N, int K) {
 
 // The 128 x 128 kernel takes the GEMMs that the few-token paths leave and whose
 // 256 x 256 grid has at most 128 tiles: then its 4x as many tiles fit one round
-// of two blocks on each of the 256 CUs (before the split over K was added:).  Measured per MLP (d_model 1024, d_ff
-// 4096, prepacked): T = 2048 86 -> 57 us, T = 4096 99 -> 82 us, T = 8192 (128
-// big tiles in GEMM2) 145 -> 140 us; at 192 big tiles (T = 12288) it lost 11%.
+// of two blocks on each of the 256 CUs.  Measured per MLP without a split over K
+// (d_model 1024, d_ff 4096, prepacked): T = 2048 86 -> 57 us, T = 4096 99 -> 82 us,
+// T = 8192 (128 big tiles in GEMM2) 145 -> 140 us; at 192 big tiles (T = 12288) it
+// lost 11%.
 constexpr int kMidMaxBigTiles = 128;
 
 // The kernel of an M x N x K GEMM (packed: B is [N][K]).  Measured, us per MLP,
@@ -1727,7 +1728,7 @@ MlpPlan mlp_plan(int T, int dm, int dff, int flags) {
 
 // Workspace layout of one MLP call (all offsets 256-byte aligned).
 struct MlpWorkspace {
-    int8_t* w2t;      // [d_model][d_ff]   (unpacked weights and the fp16-hidden GEMM2 only)
+    int8_t* w2t;      // [d_model][d_ff]   (unpacked weights, see w2_room)
     uint16_t* h16;    // [T][d_ff]          (absent with direct1)
     int8_t* hq;       // [T][d_ff]
     float* sh;        // [T]
@@ -1750,7 +1751,10 @@ MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const
         return r;
     };
     MlpWorkspace w{};
-    w.w2t = reinterpret_cast<int8_t*>(take(!prepacked && !pl.kn2 ? (size_t)dm * dff : 0));
+    // the room of W2's copy is asked for wherever GEMM2 may leave the 256 x 256 kernels,
+    // transposed or not: callers size their workspace once, and the switch is read per call
+    const bool w2_room = !prepacked && (!pl.kn2 || pl.g2.route != Route::kTiled);
+    w.w2t = reinterpret_cast<int8_t*>(take(w2_room ? (size_t)dm * dff : 0));
     w.h16 = reinterpret_cast<uint16_t*>(take(pl.direct1 ? 0 : (size_t)T * dff * 2));
     w.hq = reinterpret_cast<int8_t*>(take((size_t)T * dff));
     w.sh = reinterpret_cast<float*>(take((size_t)T * 4));
