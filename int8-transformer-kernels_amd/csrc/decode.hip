@@ -1095,7 +1095,7 @@ extern "C" int int8k_decode_attention_num_splits(int BH, int S, int head_dim, in
 
 // Workspace a contiguous-cache decode with this plan needs: none when the chunks
 // of each (b,h) merge on chip (decode_block_kernel writes no partials), else
-// the split kernel's m, l and acc[D] per unit.
+// room for m, l and acc[D] per chunk (its blocks leave one partial for up to 8).
 static size_t decode_partial_bytes(const SplitPlan& plan, long long BH, int D) {
     if (plan.nsplit <= kMaxBlockSplits && use_block_kernel()) return 0;
     return carve(nullptr, BH * plan.nsplit, D).bytes;
@@ -1104,6 +1104,20 @@ static size_t decode_partial_bytes(const SplitPlan& plan, long long BH, int D) {
 extern "C" size_t int8k_decode_attention_workspace_bytes(int BH, int S, int head_dim, int nsplit) {
     if (BH <= 0 || S <= 0 || (head_dim != 64 && head_dim != 128)) return 0;
     return decode_partial_bytes(plan_splits(BH, S, head_dim, nsplit), BH, head_dim);
+}
+
+// The call's plan with `have` bytes of workspace: an automatic plan whose partials do
+// not fit falls back to one block per (b,h) where its chunks merge on chip.
+static SplitPlan plan_within(int BH, int S, int D, int nsplit, size_t have) {
+    const SplitPlan plan = plan_splits(BH, S, D, nsplit);
+    if (plan.forced || plan.nsplit <= kMaxBlockSplits || have >= decode_partial_bytes(plan, BH, D))
+        return plan;
+    const SplitPlan small = plan_splits(BH, S, D, 0, true);
+    return small.nsplit <= kMaxBlockSplits ? small : plan;
+}
+
+size_t int8k::decode_partials_within(int BH, int S, int head_dim, int nsplit, size_t have) {
+    return decode_partial_bytes(plan_within(BH, S, head_dim, nsplit, have), BH, head_dim);
 }
 
 static bool out_ok(const DecodeOut& o) {
@@ -1124,14 +1138,7 @@ static int decode_impl(const int8_t* Q, const int8_t* K, const int8_t* V, const 
         !aligned_to(scale_Q, 4) || !aligned_to(scale_K, 4) || !aligned_to(scale_V, 4) ||
         !out_ok(out))
         return INT8K_ERR_MISALIGNED;
-    SplitPlan plan = plan_splits(BH, S, head_dim, nsplit);
-    // a short sequence spread over several blocks falls back to one block per (b,h) when
-    // the caller brings no workspace
-    if (!plan.forced && plan.nsplit > kMaxBlockSplits &&
-        (!workspace || workspace_bytes < decode_partial_bytes(plan, BH, head_dim))) {
-        const SplitPlan small = plan_splits(BH, S, head_dim, 0, true);
-        if (small.nsplit <= kMaxBlockSplits) plan = small;
-    }
+    const SplitPlan plan = plan_within(BH, S, head_dim, nsplit, workspace ? workspace_bytes : 0);
     const long long units = (long long)BH * plan.nsplit;
     if (units >= (1LL << 26)) return INT8K_ERR_UNSUPPORTED;  // 64 work-items per unit, < 2^32
     // the one-launch path reads no workspace: a null or short one is accepted there

@@ -46,6 +46,10 @@ constexpr size_t kWorkspaceAlign = 256;
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// Bytes of partials a contiguous decode leaves when it is handed `have` bytes of
+// workspace; more than `have` where no plan of the call fits (decode.hip).
+size_t decode_partials_within(int BH, int S, int head_dim, int nsplit, size_t have);
+
 // Set-up done once per device: hipFuncSetAttribute (the > 64 KiB dynamic LDS
 // limit) applies to the current device, so a process driving several GPUs
 // configures each.  Devices 0..63 are tracked (others run the set-up on every

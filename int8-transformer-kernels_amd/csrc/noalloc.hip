@@ -12,12 +12,14 @@
 // address of each GPU's copy comes from hipGetSymbolAddress, taken once per
 // device with that device current, and only that address is passed on.
 //
-// Only plans of more than 16 chunks per (b,h) run the split kernel and write
+// Only plans of more than 16 chunks per (b,h) run as several blocks each and write
 // partials; the one-launch plans merge their chunks on chip, need no scratch
-// and are never refused for size (the workspace query returns 0 for them).
+// and are never refused for size (the workspace query returns 0 for them).  An
+// automatic plan of several blocks whose partials exceed the scratch runs as one
+// launch instead where its (b,h) fill the GPU (B33 H16 D128 32768 rows).
 // Every call on a GPU shares that GPU's array and leaves its partials there.
-// Nothing in it has to start at zero: each unit of the split kernel writes its
-// partial before the combine kernel reads it.  Two calls that overlap on one
+// Nothing in it has to start at zero: each block writes its partial before the
+// combine kernel reads it.  Two calls that overlap on one
 // GPU (different streams, or different host threads) race on the array.
 #include <atomic>
 
@@ -77,8 +79,7 @@ extern "C" int int8k_decode_attention_forward_noalloc(
     if (BH <= 0 || S <= 0 || nsplit < 0) return INT8K_ERR_INVALID_ARGUMENT;
     if (head_dim != 64 && head_dim != 128) return INT8K_ERR_UNSUPPORTED;
     // the size check comes before any HIP call
-    const size_t need = int8k_decode_attention_workspace_bytes(BH, S, head_dim, nsplit);
-    if (need > kScratchBytes) {
+    if (decode_partials_within(BH, S, head_dim, nsplit, kScratchBytes) > kScratchBytes) {
         set_last_error_text(
             "int8k_decode_attention_forward_noalloc: the split partials of this call need more "
             "than the INT8K_DECODE_NOALLOC_SCRATCH_BYTES (8 MiB) of library scratch; use "

@@ -52,6 +52,17 @@ def test_noalloc_on_chip_plans_need_no_scratch(capi):
     assert capi.decode_workspace_bytes(65536, 64, 64) == 0
 
 
+@pytest.mark.parametrize("BH,S,D", [(519, 32768, 128), (1163, 131072, 128), (528, 65536, 128)])
+def test_noalloc_large_automatic_plans_fall_back_to_one_block(capi, BH, S, D):
+    # several blocks per (b,h) would leave more partials than the scratch holds: the call runs
+    # on one block per (b,h) instead.  (The odd K address is refused after the size check, so
+    # nothing is launched; without a GPU the scratch lookup before it fails.)
+    assert capi.decode_workspace_bytes(BH, S, D) > 8 << 20
+    args = [ctypes.c_void_p(0x10000 * (i + 1) + (i == 1)) for i in range(7)]
+    st = capi.load().int8k_decode_attention_forward_noalloc(*args, BH, S, D, 0, None)
+    assert st in (capi.INT8K_ERR_MISALIGNED, capi.INT8K_ERR_HIP), st
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("first,second", [
     ((2, 4, 128, 8192, 32), (1, 3, 128, 3000, 24)),   # D=128 through the scratch, twice
