@@ -148,7 +148,9 @@ __device__ __forceinline__ __half f16_of_f32(float x) {
 }
 
 // Raw buffer resource over [base, base + bytes): loads at offsets past the end
-// return zero, so tiles that overhang a matrix need no clamped addresses.  The
+// return zero, so tiles that overhang a matrix need no clamped addresses.  The scalar
+// offset of a load counts too, also where it alone is past the end (measured on
+// MI355X: 1024 bytes, scalar offsets 0 to 524288).  The
 // arguments must be the same for the whole wave (they go to scalar registers).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_buffer(const void* base, uint32_t bytes) {
     const uint64_t b = reinterpret_cast<uint64_t>(base);
