@@ -374,11 +374,13 @@ __global__ __launch_bounds__(256) void layernorm_quant_row_kernel(
         }
         const float sc =
             fmaxf(row_reduce(m, 6, [](float a, float b) { return fmaxf(a, b); }), 1e-8f) / 127.f;
+        const float inv = 1.f / sc;  // one division per row, not per element: 28.8 -> 28.1 us there
 #pragma unroll
         for (int k = 0; k < NE; ++k) {
             const int c = lane + 64 * k;
             if (c < cols) {
-                q[base + c] = quantize(v[k], sc);
+                q[base + c] = (int8_t)(int)__builtin_rintf(
+                    fminf(fmaxf(quotient(v[k], sc, inv), -128.f), 127.f));
                 if (y_out) store_any(y_out, base + c, v[k], DT);
             }
         }

@@ -143,6 +143,14 @@ __device__ __forceinline__ int quant_code(float y, float s) {
     return (int)__builtin_rintf(fminf(fmaxf(y / s, -128.f), 127.f));
 }
 
+// v / s, correctly rounded, from inv = 1 / s (see store_codes).
+__device__ __forceinline__ float quotient(float v, float s, float inv) {
+#pragma clang fp contract(off)
+    const float s_step = inv != 0.f ? s : 0.f;
+    const float t = v * inv;
+    return __builtin_fmaf(__builtin_fmaf(-t, s_step, v), inv, t);
+}
+
 // W codes of one chunk, stored as W consecutive bytes (W = 4 or 8): the same
 // codes as quant_code(v, s) for every input, without a division.  With
 // inv = 1/s correctly rounded, t = v * inv, r = v - t s (exact, one FMA) and
@@ -156,14 +164,9 @@ __device__ __forceinline__ int quant_code(float y, float s) {
 // store scheduling and cost them about 30%.
 template <int W>
 __device__ __forceinline__ void store_codes(const float (&v)[W], float s, float inv, int8_t* dst) {
-#pragma clang fp contract(off)
-    const float s_step = inv != 0.f ? s : 0.f;
     float q[W];
 #pragma unroll
-    for (int i = 0; i < W; ++i) {
-        const float t = v[i] * inv;
-        q[i] = __builtin_fmaf(__builtin_fmaf(-t, s_step, v[i]), inv, t);
-    }
+    for (int i = 0; i < W; ++i) q[i] = quotient(v[i], s, inv);
     uint32_t b[W / 4];
 #pragma unroll
     for (int j = 0; j < W / 4; ++j) {
