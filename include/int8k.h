@@ -219,6 +219,14 @@ int int8k_attention_forward(
     const float* scale_Q, const float* scale_K, const float* scale_V,
     int batch, int heads, int seq_len, int head_dim, int flags, void* stream);
 
+/* The block shape the forward calls run for BH = batch * heads, as
+ * int8k_decode_attention_num_splits tells a decode's: *query_waves waves of 32
+ * queries each, times *key_groups groups of waves that share a block's keys
+ * where the grid would leave CUs idle.  The result is independent of it up to
+ * fp32 rounding.  INT8K_ERR_UNSUPPORTED for the generic kernel's head dims. */
+int int8k_attention_block_shape(int BH, int seq_len, int head_dim, int flags, int* query_waves,
+                                int* key_groups);
+
 /* Attention output emitted as the next INT8 stage's input: out_q int8
  * [batch, heads, seq_len, head_dim] and out_scale fp32 [batch*heads*seq_len],
  * the per-token quantization (int8k_quantize_per_token) of the fp16 rows

@@ -43,6 +43,7 @@
 // int8k_quantize_per_token over the fp16 output, without its round trip.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "int8k_common.h"
 #include "rows.h"
@@ -58,11 +59,13 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int kKV = 64;  // keys per tile
 // Block shapes: QW waves of 32 queries each, times KG groups of waves that share
 // the queries and walk every KG-th tile, each group with its own stages; the
-// groups' (m, l, O) merge in LDS at the end.  Large grids run KG = 1: D = 128 with
+// groups' (l, O) are added in LDS at the end.  Large grids run KG = 1: D = 128 with
 // 8 waves (256 queries) at 2 waves per SIMD, so each staged K/V tile serves 256
 // queries; D = 64 with 4 waves (a 64-key tile has only 256 K chunks of 16 B); D = 256
 // with 4 waves at one wave per SIMD for its register budget.  Grids that leave CUs
-// idle split the keys of fewer queries over the groups (prefill_shape).
+// idle split the keys of fewer queries over the groups (pick_shape).
+template <int D>
+constexpr int kOneGroupWaves = D == 128 ? 8 : 4;
 template <int D, int QW, int KG = 1>
 struct Shape {
     static constexpr int kGroupThreads = 64 * QW;
@@ -74,7 +77,7 @@ struct Shape {
 // the probabilities enter the PV MFMA as P = fp16(p * 2^E), so
 // P . V' = sum_j p_j v_j sV_j as the reference's fp16(p * sV) . fp16(v)
 // (kernels/int8_attention.cu:530-572).  E >= 0 is chosen per block, from
-// max|sV| over the keys that block reads ([0, kv_end)), so that
+// max|sV| over the keys that a one-group block reads, so that
 // 127 * max|sV| * 2^-E <= 32768 (0 for V from fp16 data) and V' is finite
 // wherever the reference's P' is; E <= kMaxVExp.  Causal query tiles of one
 // (b,h) may use different E: each normalises with its own 2^E.
@@ -243,19 +246,27 @@ __device__ __forceinline__ void prefetch_tile(Prefetch<D, QW>& pf, const TileSrc
                                                                                k0 * 4, 0));
 }
 
-// vscale = 2^-E: V' = fp16(v * fp16(sV * 2^-E)) on v_pk_mul_f16, written as it
-// arrived: each key's 4 dims of an item as one 8-byte row piece.
+// A prefetched tile goes to its stage in three parts: K rows, key scales sK, and V.
 template <int D, int QW>
-__device__ __forceinline__ void commit_tile(const Prefetch<D, QW>& pf, char* st, float vscale,
-                                            int t) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    using VL = VLayout<D, QW>;
+__device__ __forceinline__ void commit_k(const Prefetch<D, QW>& pf, char* st, int t) {
 #pragma unroll
     for (int n = 0; n < Stage<D, QW>::kKChunks; ++n) {
         const int c = t + n * Shape<D, QW>::kGroupThreads;
         const int row = c / (D / 16), col = (c % (D / 16)) * 16;
         *reinterpret_cast<int4*>(st + row * Stage<D, QW>::kKStride + col) = pf.k[n];
     }
+}
+template <int D, int QW>
+__device__ __forceinline__ void commit_sk(const Prefetch<D, QW>& pf, char* st, int t) {
+    if (t < kKV) reinterpret_cast<float*>(st + Stage<D, QW>::kKBytes + Stage<D, QW>::kVtBytes)[t] = pf.sc;
+}
+
+// vscale = 2^-E: V' = fp16(v * fp16(sV * 2^-E)) on v_pk_mul_f16, written as it
+// arrived: each key's 4 dims of an item as one 8-byte row piece.
+template <int D, int QW>
+__device__ __forceinline__ void commit_v(const Prefetch<D, QW>& pf, char* st, float vscale, int t) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    using VL = VLayout<D, QW>;
     _Float16* vs = reinterpret_cast<_Float16*>(st + Stage<D, QW>::kKBytes) +
                    (t / VL::kW) * 4 * VL::kRow + (t % VL::kW) * 4;
     // key 4 kg + i scaled by its sV * 2^-E (both dims of a word share the key)
@@ -272,7 +283,13 @@ __device__ __forceinline__ void commit_tile(const Prefetch<D, QW>& pf, char* st,
             *reinterpret_cast<uint2*>(vs + i * VL::kRow + n * 4 * VL::kW) = w;
         }
     }
-    if (t < kKV) reinterpret_cast<float*>(st + Stage<D, QW>::kKBytes + Stage<D, QW>::kVtBytes)[t] = pf.sc;
+}
+
+template <int D, int QW>
+__device__ __forceinline__ void commit_tile(const Prefetch<D, QW>& pf, char* st, float vscale, int t) {
+    commit_k<D, QW>(pf, st, t);
+    commit_v<D, QW>(pf, st, vscale, t);
+    commit_sk<D, QW>(pf, st, t);
 }
 
 // Sum of the 32 fp16 P of a lane in fp32 (v_dot2_f32_f16 against {1, 1}).
@@ -367,31 +384,36 @@ __global__ __launch_bounds__((Shape<D, QW, KG>::kThreads), (Shape<D, QW, KG>::kM
     // does not see whole, which take the slow path anyway), so the running max is
     // set when the unmasked tiles 0 .. kd-1 follow on the fast path; otherwise the
     // first of those would take the slow path only to set it.
-    const int kd = CAUSAL ? (qt * kQ) / kKV : 0;
+    // (kQ1 queries: the one-group block that holds this block's queries, whose order
+    // and exponent below every shape keeps.)
+    constexpr int kQ1 = Shape<D, kOneGroupWaves<D>>::kQ;
+    const int q_block1 = kQ == kQ1 ? qt * kQ : qt * kQ / kQ1 * kQ1;
+    const int kd = CAUSAL ? q_block1 / kKV : 0;
     const int nd = n_kv - kd;
     auto tile_of = [&](int i) { return CAUSAL ? (i < nd ? kd + i : i - nd) : i; };
-    // This group's steps are walk positions grp, grp + KG, ...; every group runs the
-    // same number of steps (barriers), the last of them possibly past the end.
-    const int n_steps = (n_kv + KG - 1) / KG;
-    auto pos_of = [&](int step) { return step * KG + grp; };
+    // Step i of a group is position pos_of(i) of the walk; every group runs n_steps
+    // steps (barriers), the last of them possibly past the end.
+    const int n_steps = KG == 1 ? n_kv : (n_kv + KG - 1) / KG;
+    auto pos_of = [&](int step) { return KG == 1 ? step : step * KG + grp; };
 
     // The first tile's loads go out before the exponent's reduction, so their
     // latency overlaps it.
     const TileSrc src = make_tile_src<D, QW>(Kbh, Vbh, sKbh, sVbh, S, dm, tg);
     Prefetch<D, QW> pa;
-    prefetch_tile<D, QW, PAD>(pa, src, tile_of(min(pos_of(0), n_kv - 1)) * kKV, tg);
+    prefetch_tile<D, QW, PAD>(pa, src, tile_of(KG == 1 ? 0 : min(grp, n_kv - 1)) * kKV, tg);
 
     // E: the exponent that keeps the scaled V^T in fp16 range, from max |sV| over
-    // the keys this block reads (a block-wide reduction through LDS).  Each thread
-    // reads 16-byte vectors, kSvU of them in flight per round; dwords past kv_end
+    // the keys the one-group block reads (a block-wide reduction through LDS).  Each thread
+    // reads 16-byte vectors, kSvU of them in flight per round; dwords past e_end
     // read as zero (the buffer range is checked per dword).
     __shared__ float s_svmax[QW * KG];
+    const int e_end = kQ == kQ1 || !CAUSAL ? kv_end : min(S, q_block1 + kQ1);
     {
         typedef float v4f __attribute__((ext_vector_type(4)));
         constexpr int kT = Sh::kThreads, kSvU = 4;
-        const __amdgpu_buffer_rsrc_t svr = make_buffer(sVbh, (uint32_t)kv_end * 4);
+        const __amdgpu_buffer_rsrc_t svr = make_buffer(sVbh, (uint32_t)e_end * 4);
         float a = 0.f;
-        for (int j0 = 0; j0 < kv_end; j0 += 4 * kT * kSvU) {
+        for (int j0 = 0; j0 < e_end; j0 += 4 * kT * kSvU) {
             v4f v[kSvU];
 #pragma unroll
             for (int u = 0; u < kSvU; ++u)
@@ -523,42 +545,75 @@ __global__ __launch_bounds__((Shape<D, QW, KG>::kThreads), (Shape<D, QW, KG>::kM
     // the slow path, which sets m to the exact running max and rescales O and l.  l
     // sums the fp16 P that enter the PV product.
     //
-    // Step kt is computed from LDS stage kt&1.  The register set holds step
-    // kt+1's tile while step kt is computed; at the end of the step it is written
-    // to the other stage, refilled with step kt+2's tile, and the step's one
-    // barrier follows.  The fast path runs as an inner loop that the slow path
-    // leaves and re-enters, so O has no conditional update inside it.
     commit_tile<D, QW>(pa, smem, vscale, tg);
     if (pos_of(1) < n_kv) prefetch_tile<D, QW, PAD>(pa, src, tile_of(pos_of(1)) * kKV, tg);
     __syncthreads();
-    auto advance = [&](int kt) {
-        if (pos_of(kt + 1) < n_kv) {
-            commit_tile<D, QW>(pa, smem + ((kt + 1) & 1) * St::kBytes, vscale, tg);
-            if (pos_of(kt + 2) < n_kv)
-                prefetch_tile<D, QW, PAD>(pa, src, tile_of(pos_of(kt + 2)) * kKV, tg);
-        }
-        // step kt+1's tile is in LDS and every wave is done reading stage kt&1
-        __syncthreads();
-    };
-    bool have_m = false;  // wave-uniform: a slow step has set the running max
-    int kt = 0;
-    while (kt < n_steps) {
-        v16i sacc[2];
-        bool slow = false;
-        for (; kt < n_steps; ++kt) {
-            const int tk = tile_of(pos_of(kt));
-            if ((KG == 1 || pos_of(kt) < n_kv) && computes(tk)) {
-                const int k0 = tk * kKV;
-                const bool full = k0 + kKV <= S && !(CAUSAL && k0 + kKV - 1 > qw0);
-                if (!(full && qpos && have_m)) {
+
+    if constexpr (KG == 1) {
+        // Step kt is computed from LDS stage kt&1.  The register set holds step
+        // kt+1's tile while step kt is computed; at the end of the step it is written
+        // to the other stage, refilled with step kt+2's tile, and the step's one
+        // barrier follows.  The fast path runs as an inner loop that the slow path
+        // leaves and re-enters, so O has no conditional update inside it.  (Its parts are
+        // written out: called as the lambdas below, the compiler orders the fast step
+        // otherwise, 1-1.5% slower at BH 24 S 3000 causal.)
+        auto advance = [&](int kt) {
+            if (kt + 1 < n_kv) {
+                commit_tile<D, QW>(pa, smem + ((kt + 1) & 1) * St::kBytes, vscale, tg);
+                if (kt + 2 < n_kv) prefetch_tile<D, QW, PAD>(pa, src, tile_of(kt + 2) * kKV, tg);
+            }
+            // step kt+1's tile is in LDS and every wave is done reading stage kt&1
+            __syncthreads();
+        };
+        bool have_m = false;  // wave-uniform: a slow step has set the running max
+        int kt = 0;
+        while (kt < n_kv) {
+            v16i sacc[2];
+            bool slow = false;
+            for (; kt < n_kv; ++kt) {
+                const int tk = tile_of(kt);
+                if (computes(tk)) {
+                    const int k0 = tk * kKV;
+                    const bool full = k0 + kKV <= S && !(CAUSAL && k0 + kKV - 1 > qw0);
+                    if (!(full && qpos && have_m)) {
+                        qk(kt, sacc);
+                        slow = true;
+                        break;
+                    }
                     qk(kt, sacc);
-                    slow = true;
-                    break;
+                    const float* sk_l = sk_of(kt);
+                    const float shift = pexp - m;
+                    v8h pfr[4];
+#pragma unroll
+                    for (int T = 0; T < 2; ++T)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const float4 skv = *reinterpret_cast<const float4*>(sk_l + 32 * T + 8 * g + 4 * h);
+                            const float skk[4] = {skv.x, skv.y, skv.z, skv.w};
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) {
+                                const float u = static_cast<float>(sacc[T][4 * g + c]) * skk[c];
+                                pfr[2 * T + (g >> 1)][4 * (g & 1) + c] =
+                                    (_Float16)fast_exp2(fmaf(u, qscale, shift));
+                            }
+                        }
+                    schedule_qk();
+                    const float tsum = psum(pfr);
+                    if (__ballot(!(tsum <= 65504.f))) { slow = true; break; }
+                    lsum += tsum;
+                    pv(kt, pfr);
+                    schedule_pv();
                 }
-                qk(kt, sacc);
+                advance(kt);
+            }
+            if (!slow) break;
+            // Slow path for step kt (its S^T is in sacc): s = acc * qscale * sK with masked
+            // keys at -inf, exact running max, rescale of O and l.
+            {
+                const int k0 = tile_of(kt) * kKV;
                 const float* sk_l = sk_of(kt);
-                const float shift = pexp - m;
-                v8h pfr[4];
+                float sc[2][16];
+                float mx = -INFINITY;
 #pragma unroll
                 for (int T = 0; T < 2; ++T)
 #pragma unroll
@@ -567,27 +622,87 @@ __global__ __launch_bounds__((Shape<D, QW, KG>::kThreads), (Shape<D, QW, KG>::kM
                         const float skk[4] = {skv.x, skv.y, skv.z, skv.w};
 #pragma unroll
                         for (int c = 0; c < 4; ++c) {
-                            const float u = static_cast<float>(sacc[T][4 * g + c]) * skk[c];
-                            pfr[2 * T + (g >> 1)][4 * (g & 1) + c] =
-                                (_Float16)fast_exp2(fmaf(u, qscale, shift));
+                            float v = static_cast<float>(sacc[T][4 * g + c]) * qscale * skk[c];
+                            const int key = k0 + 32 * T + 8 * g + 4 * h + c;
+                            if (key >= S || (CAUSAL && key > q)) v = -INFINITY;
+                            sc[T][4 * g + c] = v;
+                            mx = fmaxf(mx, v);
                         }
                     }
-                schedule_qk();
-                const float tsum = psum(pfr);
-                if (__ballot(!(tsum <= 65504.f))) { slow = true; break; }
-                lsum += tsum;
+                mx = max_xor32(mx);
+                const float m_new = fmaxf(m, mx);
+                const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+                const float corr = fast_exp2(m - m_use);
+                lsum *= corr;
+#pragma unroll
+                for (int t = 0; t < NS; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[t][r] *= corr;
+                m = m_new;
+                const float shift = pexp - m_use;
+                v8h pfr[4];
+#pragma unroll
+                for (int T = 0; T < 2; ++T)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+                            pfr[2 * T + (g >> 1)][4 * (g & 1) + c] =
+                                (_Float16)fast_exp2(sc[T][4 * g + c] + shift);
+                lsum += psum(pfr);
                 pv(kt, pfr);
-                schedule_pv();
             }
+            have_m = true;
             advance(kt);
+            ++kt;
         }
-        if (!slow) break;
-        // Slow path for step kt (its S^T is in sacc): s = acc * qscale * sK with masked
-        // keys at -inf, exact running max, rescale of O and l.
-        {
-            const int k0 = tile_of(pos_of(kt)) * kKV;
+    } else {
+        // The groups keep one m per query, that of the one-group walk at every position: each
+        // P is rounded to fp16 against m, so only with the same m is it the same P, and O and
+        // l differ from that walk's by the order of their fp32 sums alone: no output by more
+        // than one step of fp16.  (A maximum of its own per group moved single outputs by up
+        // to 1.5e-2 of themselves or the rms.)
+        //
+        // In a round every wave whose tile is not in O yet computes S^T and, on the fast path,
+        // P with the m all groups share; it publishes whether its tile is slow (kDynamic: a
+        // sum past the fp16 range; kStatic: masked, negative scales or the walk's first) and a
+        // slow tile's maximum.  No slow tile in the block (the usual round): all go on to PV
+        // and the next step.  Otherwise the positions of a query wave are settled in walk
+        // order: those before its first slow tile keep their P, the slow tile (and static
+        // ones right behind it) raises m, and those behind it take another round with the
+        // new m.  One copy of each part: a short prompt's time is the first fetch of the
+        // code it runs.
+        //
+        // Step kt's tile is in LDS stage kt&1, step kt+1's in registers: its K goes to the
+        // other stage before the step's first barrier (step kt+1's S^T follows that) and its V
+        // after it (step kt-1's PV, the last reader there, is behind every wave by then).
+        // Nothing reads stage kt&1's K and sK behind a step's last barrier.
+
+        // P^T of a fast tile (its S^T in sacc) with the current m; returns the lane's sum of it.
+        auto fast_p = [&](int kt, const v16i (&sacc)[2], v8h (&pfr)[4]) -> float {
             const float* sk_l = sk_of(kt);
-            float sc[2][16];
+            const float shift = pexp - m;
+#pragma unroll
+            for (int T = 0; T < 2; ++T)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 skv = *reinterpret_cast<const float4*>(sk_l + 32 * T + 8 * g + 4 * h);
+                    const float skk[4] = {skv.x, skv.y, skv.z, skv.w};
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const float u = static_cast<float>(sacc[T][4 * g + c]) * skk[c];
+                        pfr[2 * T + (g >> 1)][4 * (g & 1) + c] =
+                            (_Float16)fast_exp2(fmaf(u, qscale, shift));
+                    }
+                }
+            schedule_qk();
+            return psum(pfr);
+        };
+        // Scores of a slow tile, s = acc * qscale * sK with masked keys at -inf; returns the
+        // maximum over the query's 64 keys.
+        auto slow_scores = [&](int kt, int tk, const v16i (&sacc)[2], float (&sc)[2][16]) -> float {
+            const int k0 = tk * kKV;
+            const float* sk_l = sk_of(kt);
             float mx = -INFINITY;
 #pragma unroll
             for (int T = 0; T < 2; ++T)
@@ -604,18 +719,9 @@ __global__ __launch_bounds__((Shape<D, QW, KG>::kThreads), (Shape<D, QW, KG>::kM
                         mx = fmaxf(mx, v);
                     }
                 }
-            mx = max_xor32(mx);
-            const float m_new = fmaxf(m, mx);
-            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-            const float corr = fast_exp2(m - m_use);
-            lsum *= corr;
-#pragma unroll
-            for (int t = 0; t < NS; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[t][r] *= corr;
-            m = m_new;
-            const float shift = pexp - m_use;
-            v8h pfr[4];
+            return max_xor32(mx);
+        };
+        auto slow_p = [&](const float (&sc)[2][16], float shift, v8h (&pfr)[4]) {
 #pragma unroll
             for (int T = 0; T < 2; ++T)
 #pragma unroll
@@ -624,45 +730,148 @@ __global__ __launch_bounds__((Shape<D, QW, KG>::kThreads), (Shape<D, QW, KG>::kM
                     for (int c = 0; c < 4; ++c)
                         pfr[2 * T + (g >> 1)][4 * (g & 1) + c] =
                             (_Float16)fast_exp2(sc[T][4 * g + c] + shift);
-            lsum += psum(pfr);
-            pv(kt, pfr);
-        }
-        have_m = true;
-        advance(kt);
-        ++kt;
-    }
-
-    if constexpr (KG > 1) {
-        // Every group but the first leaves its waves' (m, l, O) in LDS (the stages are free
-        // after the last step's barrier), lane by lane; the first group's waves merge them.
-        constexpr int kWords = NS * 16 + 2;  // per lane, [word][lane]
-        static_assert((KG - 1) * QW * kWords * 64 * 4 <= KG * 2 * St::kBytes, "fits the stages");
-        float* ex = reinterpret_cast<float*>(smem_all) + lane;
-        if (grp > 0) {
-            float* e = ex + (wave - QW) * kWords * 64;
-            e[0] = m;
-            e[64] = lsum;
+        };
+        auto rescale = [&](float corr) {
+            lsum *= corr;
 #pragma unroll
             for (int t = 0; t < NS; ++t)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) e[(2 + t * 16 + r) * 64] = o[t][r];
+                for (int r = 0; r < 16; ++r) o[t][r] *= corr;
+        };
+        auto is_full = [&](int tk) {
+            return tk * kKV + kKV <= S && !(CAUSAL && tk * kKV + kKV - 1 > qw0);
+        };
+        enum { kFast = 0, kDynamic = 1, kStatic = 2 };
+        using Kinds = std::conditional_t<QW * KG == 8, uint64_t, uint32_t>;
+        static_assert(QW * KG == 8 || QW * KG == 4, "one byte per wave");
+        // [round & 1]: a wave may publish its next round while another has yet to read this one
+        __shared__ __align__(8) uint8_t s_kind[2][QW * KG];  // [query wave][group]
+        __shared__ float s_mx[2][KG][32 * QW];
+        const int wq = wave - grp * QW;  // query wave
+        // the kinds of query wave i's positions, one byte each
+        auto kinds_of = [](Kinds f, int i) {
+            return (uint32_t)(f >> (8 * KG * i)) & (KG == 4 ? ~0u : 0xffffu);
+        };
+        // the last position that a round with slow tiles settles
+        auto last_settled = [](uint32_t kinds) {
+            int i = __builtin_ctz(kinds) >> 3;
+            while (i + 1 < KG && ((kinds >> (8 * (i + 1))) & 0xff) == kStatic) ++i;
+            return i;
+        };
+        int kt = 0, buf = 0;
+        bool first_round = true;  // of step kt; uniform over the block, as the rest but `pending`
+        int tk = tile_of(grp);
+        bool pending = grp < n_kv && computes(tk);  // wave-uniform
+        while (true) {
+            v16i sacc[2];
+            v8h pfr[4];
+            float sc[2][16];
+            float tsum = 0.f;
+            int kind = kFast;
+            if (pending) {
+                qk(kt, sacc);
+                if (!(is_full(tk) && qpos && pos_of(kt) > 0)) {
+                    kind = kStatic;
+                } else if (kt > 0 || !first_round) {  // before that there is no m
+                    tsum = fast_p(kt, sacc, pfr);
+                    if (__ballot(!(tsum <= 65504.f))) kind = kDynamic;
+                }
+                if (kind != kFast) {
+                    const float mx = slow_scores(kt, tk, sacc, sc);
+                    if (lane < 32) s_mx[buf][grp][32 * wq + lane] = mx;
+                }
+            }
+            if (first_round && pos_of(kt + 1) < n_kv) {
+                commit_k<D, QW>(pa, smem + ((kt + 1) & 1) * St::kBytes, tg);
+                commit_sk<D, QW>(pa, smem + ((kt + 1) & 1) * St::kBytes, tg);
+            }
+            if (lane == 0) s_kind[buf][wq * KG + grp] = (uint8_t)kind;
+            __syncthreads();
+            Kinds f = *reinterpret_cast<const Kinds*>(s_kind[buf]);
+            if constexpr (QW * KG == 8)
+                f = (Kinds)__builtin_amdgcn_readfirstlane((uint32_t)(f >> 32)) << 32 |
+                    (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)f);
+            else
+                f = __builtin_amdgcn_readfirstlane(f);
+            bool add = pending;
+            float after = 1.f;
+            if (f != 0) {
+                const uint32_t kinds = kinds_of(f, wq);
+                if (kinds != 0) {
+                    const int first = __builtin_ctz(kinds) >> 3, last = last_settled(kinds);
+                    float before = 1.f, shift = 0.f;
+                    for (int p = first; p <= last; ++p) {
+                        const float m_new = fmaxf(m, s_mx[buf][p][32 * wq + (lane & 31)]);
+                        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+                        const float corr = fast_exp2(m - m_use);
+                        if (p <= grp) before *= corr;
+                        else after *= corr;
+                        if (p == grp) shift = pexp - m_use;
+                        m = m_new;
+                    }
+                    add = pending && grp <= last;
+                    if (grp >= first) rescale(before);
+                    if (add && grp >= first) {
+                        slow_p(sc, shift, pfr);
+                        tsum = psum(pfr);
+                    }
+                }
+            }
+            if (add) {
+                lsum += tsum;
+                pv(kt, pfr);
+                schedule_pv();
+                pending = false;
+            }
+            if (f != 0) {
+                rescale(after);
+                // another round where a query wave has positions behind its last settled one
+                bool again = false;
+                for (int i = 0; i < QW; ++i) {
+                    const uint32_t k = kinds_of(f, i);
+                    again = again || (k != 0 && last_settled(k) < KG - 1);
+                }
+                if (again) {
+                    first_round = false;
+                    buf ^= 1;
+                    continue;
+                }
+            }
+            if (pos_of(kt + 1) < n_kv) {
+                commit_v<D, QW>(pa, smem + ((kt + 1) & 1) * St::kBytes, vscale, tg);
+                if (pos_of(kt + 2) < n_kv)
+                    prefetch_tile<D, QW, PAD>(pa, src, tile_of(pos_of(kt + 2)) * kKV, tg);
+            }
+            if (++kt == n_steps) break;
+            first_round = true;
+            buf ^= 1;
+            tk = tile_of(pos_of(kt));
+            pending = pos_of(kt) < n_kv && computes(tk);
+        }
+        // Every group but the first leaves its waves' (l, O) in LDS (the stages are free after
+        // the barrier), lane by lane; the first group's waves add them.
+        constexpr int kWords = NS * 16 + 1;  // per lane, [word][lane]
+        static_assert((KG - 1) * QW * kWords * 64 * 4 <= KG * 2 * St::kBytes, "fits the stages");
+        __syncthreads();
+        float* ex = reinterpret_cast<float*>(smem_all) + lane;
+        if (grp > 0) {
+            float* e = ex + (wave - QW) * kWords * 64;
+            e[0] = lsum;
+#pragma unroll
+            for (int t = 0; t < NS; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) e[(1 + t * 16 + r) * 64] = o[t][r];
         }
         __syncthreads();
         if (grp > 0) return;
 #pragma unroll
         for (int g = 0; g < KG - 1; ++g) {
             const float* e = ex + (g * QW + wave) * kWords * 64;
-            const float mg = e[0];
-            const float m_new = fmaxf(m, mg);
-            const float m_use = m_new == -INFINITY ? 0.f : m_new;
-            const float fa = fast_exp2(m - m_use), fb = fast_exp2(mg - m_use);
-            lsum = lsum * fa + e[64] * fb;
+            lsum += e[0];
 #pragma unroll
             for (int t = 0; t < NS; ++t)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    o[t][r] = o[t][r] * fa + e[(2 + t * 16 + r) * 64] * fb;
-            m = m_new;
+                for (int r = 0; r < 16; ++r) o[t][r] += e[(1 + t * 16 + r) * 64];
         }
     }
     const float L = sum_xor32(lsum);
@@ -940,58 +1149,67 @@ int launch_prefill_shape(const int8_t* Q, const int8_t* K, const int8_t* V, uint
 // block's prologue, first tiles and epilogue `fixed` steps; `slots` blocks make
 // progress at once.  The grid is bound by its longest block or by its sum.
 struct ShapeCost {
-    int qw, kg, step, fixed_full, fixed_causal, slots;
+    int qw, kg, step_full, fixed_full, step_causal, fixed_causal, slots;
 };
 inline long long shape_time(const ShapeCost& c, int BH, int S, bool causal) {
-    const long long kq = 32LL * c.qw, qt = ceil_div(S, kq);
+    const long long kq = 32LL * c.qw, blocks = BH * ceil_div(S, kq);
     auto steps = [&](long long keys) { return ceil_div(ceil_div(keys, kKV), c.kg); };
-    const long long longest = steps(S), shortest = causal ? steps(std::min<long long>(S, kq)) : longest;
-    const long long fixed = causal ? c.fixed_causal : c.fixed_full;
-    const long long blocks = (long long)BH * qt;
-    // equal blocks run in whole rounds; causal ones (heaviest first) fill the slots evenly
-    const long long sum =
-        causal ? (blocks * (longest + shortest + 2 * fixed) / 2 + c.slots - 1) / c.slots
-               : ceil_div(blocks, c.slots) * (longest + fixed);
-    return c.step * std::max(longest + fixed, sum);
+    // equal blocks run in whole rounds
+    if (!causal) return c.step_full * ceil_div(blocks, c.slots) * (steps(S) + c.fixed_full);
+    // causal ones go heaviest first: the shortest end the grid where they do not all fit at once
+    const long long longest = steps(S) + c.fixed_causal;
+    const long long shortest = steps(std::min<long long>(S, kq)) + c.fixed_causal;
+    if (blocks <= c.slots) return c.step_causal * longest;
+    const long long sum2 = blocks * (longest + shortest);  // twice the sum
+    return c.step_causal * std::max(2 * longest, (sum2 - 2 * shortest) / c.slots + 2 * shortest) / 2;
 }
 
-// The costs fit runs of every shape at BH 8..128, S 100..8192.  us at the shape with the
-// most queries per block -> chosen: D = 64: BH 12 S 384 causal 13.8 -> 10.8, BH 12 S 1024
-// causal 24.6 -> 15.2, BH 32 S 1023 21.6 -> 17.4; D = 128: BH 32 S 256 causal 19.9 -> 11.7,
-// BH 32 S 1024 causal 38.7 -> 26.8, BH 8 S 8192 causal 208 -> 152, BH 32 S 1023 D = 80
-// 33.6 -> 24.5.  Another shape has to promise 5% over the first.
+// The block shapes of a head_dim, the one with the most queries per block first, and their
+// costs.  They fit runs of every shape at BH 4..128, S 65..8192 (552 of them), where no pick
+// is more than 0.5% over the first shape; another shape has to promise 5% over it.  us of the
+// first shape -> of the pick (full / causal): D = 64: BH 12 S 384 10.6 -> 8.7 / 13.0 -> 9.9,
+// BH 12 S 1023 23.2 -> 14.0 / 22.9 -> 14.6, BH 32 S 1023 23.8 -> 19.6 / 23.4 -> 19.7; D = 128:
+// BH 32 S 256 14.2 -> 11.5 / 19.5 -> 15.7, BH 32 S 1023 33.7 -> 27.3 / 38.1 -> 28.4, BH 8 S
+// 8192 causal 217 -> 166; D = 80 (padded), BH 32 S 1023 32.1 -> 25.8.
+template <int D>
+constexpr ShapeCost kShapes[3] = {
+    D == 64 ? ShapeCost{4, 1, 123, 2, 123, 4, 512} : ShapeCost{8, 1, 200, 3, 200, 4, 256},
+    D == 64 ? ShapeCost{4, 2, 150, 3, 142, 4, 256} : ShapeCost{4, 2, 244, 3, 252, 3, 256},
+    D == 64 ? ShapeCost{2, 4, 168, 3, 140, 5, 256} : ShapeCost{2, 2, 238, 3, 323, 2, 256}};
+template <>
+constexpr ShapeCost kShapes<256>[1] = {ShapeCost{4, 1, 0, 0, 0, 0, 256}};
+
+template <int D>
+int pick_shape(int BH, int S, bool causal) {
+    int pick = 0;
+    if constexpr (D <= 128) {
+        long long best = shape_time(kShapes<D>[0], BH, S, causal) * 95 / 100;
+        for (int i = 1; i < 3; ++i) {
+            const long long t = shape_time(kShapes<D>[i], BH, S, causal);
+            if (t < best) best = t, pick = i;
+        }
+    }
+    return pick;
+}
+
 template <int D>
 int launch_prefill(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* out,
                    int8_t* qout, float* qscale, const float* sQ, const float* sK, const float* sV,
                    int BH, int heads, int S, int dm, bool causal, bool bshd, hipStream_t stream) {
-    constexpr ShapeCost kCosts[3] = {
-        D == 64 ? ShapeCost{4, 1, 123, 4, 4, 512} : ShapeCost{8, 1, 200, 4, 4, 256},
-        D == 64 ? ShapeCost{4, 2, 144, 4, 6, 256} : ShapeCost{4, 2, 234, 4, 4, 256},
-        D == 64 ? ShapeCost{2, 4, 150, 5, 5, 256} : ShapeCost{2, 2, 195, 4, 4, 256}};
-    int pick = 0;
+#define INT8K_PREFILL_SHAPE(I)                                                                   \
+    return launch_prefill_shape<D, kShapes<D>[I].qw, kShapes<D>[I].kg>(                          \
+        Q, K, V, out, qout, qscale, sQ, sK, sV, BH, heads, S, dm, causal, bshd, stream)
     if constexpr (D <= 128) {
-        long long best = shape_time(kCosts[0], BH, S, causal) * 95 / 100;
-        for (int i = 1; i < 3; ++i) {
-            const long long t = shape_time(kCosts[i], BH, S, causal);
-            if (t < best) best = t, pick = i;
-        }
+        const int pick = pick_shape<D>(BH, S, causal);
+        if (pick == 1) INT8K_PREFILL_SHAPE(1);
+        if (pick == 2) INT8K_PREFILL_SHAPE(2);
     }
-#define INT8K_PREFILL_SHAPE(QW, KG)                                                           \
-    return launch_prefill_shape<D, QW, KG>(Q, K, V, out, qout, qscale, sQ, sK, sV, BH, heads, S, \
-                                           dm, causal, bshd, stream)
-    if constexpr (D == 64) {
-        if (pick == 1) INT8K_PREFILL_SHAPE(4, 2);
-        if (pick == 2) INT8K_PREFILL_SHAPE(2, 4);
-        INT8K_PREFILL_SHAPE(4, 1);
-    } else if constexpr (D == 128) {
-        if (pick == 1) INT8K_PREFILL_SHAPE(4, 2);
-        if (pick == 2) INT8K_PREFILL_SHAPE(2, 2);
-        INT8K_PREFILL_SHAPE(8, 1);
-    } else {
-        INT8K_PREFILL_SHAPE(4, 1);
-    }
+    INT8K_PREFILL_SHAPE(0);
 #undef INT8K_PREFILL_SHAPE
 }
+
+// Head dims of the MFMA kernel; the generic one takes the others.
+inline bool on_mfma(int head_dim) { return head_dim % 16 == 0 && head_dim <= 256; }
 
 int launch_prefill_generic(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* out,
                            int8_t* qout, float* qscale, const float* sQ, const float* sK,
@@ -1025,7 +1243,7 @@ int prefill_entry(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* o
         return INT8K_ERR_INVALID_ARGUMENT;
     if (head_dim > kGenMaxD) return INT8K_ERR_UNSUPPORTED;
     const long long BH = (long long)batch * heads;
-    const bool mfma = head_dim % 16 == 0 && head_dim <= 256;
+    const bool mfma = on_mfma(head_dim);
     // work-items of the launch: 2 threads per query (MFMA kernel), 16 (generic)
     if (BH * (((long long)seq_len + 127) / 128) * 256 >= (1LL << 32)) return INT8K_ERR_UNSUPPORTED;
     if (!mfma && BH * (((long long)seq_len + kGenQ - 1) / kGenQ) * 256 >= (1LL << 32))
@@ -1060,6 +1278,22 @@ int prefill_entry(const int8_t* Q, const int8_t* K, const int8_t* V, uint16_t* o
 }  // namespace int8k
 
 using namespace int8k;
+
+extern "C" int int8k_attention_block_shape(int BH, int seq_len, int head_dim, int flags,
+                                           int* query_waves, int* key_groups) {
+    clear_last_error();
+    if (BH <= 0 || seq_len <= 0 || head_dim <= 0 || !query_waves || !key_groups ||
+        (flags & ~(INT8K_ATTN_CAUSAL | INT8K_ATTN_OUT_BSHD)) != 0)
+        return INT8K_ERR_INVALID_ARGUMENT;
+    if (!on_mfma(head_dim)) return INT8K_ERR_UNSUPPORTED;
+    const bool c = (flags & INT8K_ATTN_CAUSAL) != 0;
+    const ShapeCost& sh = head_dim <= 64    ? kShapes<64>[pick_shape<64>(BH, seq_len, c)]
+                          : head_dim <= 128 ? kShapes<128>[pick_shape<128>(BH, seq_len, c)]
+                                            : kShapes<256>[0];
+    *query_waves = sh.qw;
+    *key_groups = sh.kg;
+    return INT8K_OK;
+}
 
 extern "C" int int8k_attention_forward(const int8_t* Q, const int8_t* K, const int8_t* V,
                                        uint16_t* out, const float* scale_Q, const float* scale_K,

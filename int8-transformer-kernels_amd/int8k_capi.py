@@ -57,6 +57,7 @@ _SIGNATURES = {
     "int8k_quantize_heads": (_I, [_P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "int8k_decode_attention_forward_paged": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I,
                                                   _I, _I, _I, _I, _I, _P, _SZ, _P]),
+    "int8k_attention_block_shape": (_I, [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "int8k_attention_forward_quant": (_I, [_P] * 8 + [_I] * 5 + [_P]),
     "int8k_decode_attention_forward_quant": (_I, [_P] * 8 + [_I] * 4 + [_P, _SZ, _P]),
     "int8k_decode_attention_forward_cache_quant": (_I, [_P] * 8 + [_I] * 5 + [_P, _SZ, _P]),
@@ -260,6 +261,14 @@ ATTN_OUT_BSHD = 2  # INT8K_ATTN_OUT_BSHD
 
 def _attn_flags(causal, out_bshd):
     return (ATTN_CAUSAL if causal else 0) | (ATTN_OUT_BSHD if out_bshd else 0)
+
+
+def attention_block_shape(BH, S, D, causal=False):
+    """(query waves, key groups) of a prefill block for these arguments."""
+    qw, kg = _I(), _I()
+    check("int8k_attention_block_shape", load().int8k_attention_block_shape(
+        BH, S, D, _attn_flags(causal, False), ctypes.byref(qw), ctypes.byref(kg)))
+    return qw.value, kg.value
 
 
 def attention_forward(Qi, Ki, Vi, sQ, sK, sV, causal=False, out=None, out_bshd=False):
