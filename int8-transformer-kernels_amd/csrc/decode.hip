@@ -613,19 +613,27 @@ __device__ __forceinline__ void merge_block(float m, float l, float* acc, int la
             s_ml[w][1] = Lw;
         }
     }
+    constexpr int DPL = D / 64;
+    // chunks past nw are empty states (not another chunk's with weight 0: it may hold
+    // infinities)
+    for (int c = nw + w; c < MAXW; c += nw) {
+#pragma unroll
+        for (int i = 0; i < DPL; ++i) s_acc[c][lane * DPL + i] = 0.f;
+        if (lane == 0) {
+            s_ml[c][0] = -INFINITY;
+            s_ml[c][1] = 0.f;
+        }
+    }
     __syncthreads();
     if (w != 0) return;
-    constexpr int DPL = D / 64;
-    // unrolled, so that the LDS reads of all chunks go out together; chunks past nw
-    // count as empty
+    // unrolled, so that the LDS reads of all chunks go out together
     float mc[MAXW], lc[MAXW], oc[MAXW][DPL];
 #pragma unroll
     for (int c = 0; c < MAXW; ++c) {
-        const int k = min(c, nw - 1);
-        mc[c] = c < nw ? s_ml[k][0] : -INFINITY;
-        lc[c] = s_ml[k][1];
+        mc[c] = s_ml[c][0];
+        lc[c] = s_ml[c][1];
 #pragma unroll
-        for (int i = 0; i < DPL; ++i) oc[c][i] = s_acc[k][lane * DPL + i];
+        for (int i = 0; i < DPL; ++i) oc[c][i] = s_acc[c][lane * DPL + i];
     }
     float Mall = mc[0];
 #pragma unroll

@@ -78,6 +78,33 @@ def test_short_sequences_without_workspace_stay_on_one_block(gpu):
     assert outs[0][0] == capi.INT8K_OK
 
 
+def _decode(c, S, ws):
+    """Status and rows of the cache entry with the workspace tensor `ws` (None: a null one)."""
+    B, H, cap, D = c["Ki"].shape
+    out = torch.empty((B * H, D), dtype=torch.float16, device=c["Ki"].device)
+    st = capi.load().int8k_decode_attention_forward_cache(
+        *(ctypes.c_void_p(t.data_ptr()) for t in (c["Qi"], c["Ki"], c["Vi"], out, c["sQ"],
+                                                  c["sK"], c["sV"])),
+        B * H, S, cap, D, 0, ctypes.c_void_p(0 if ws is None else ws.data_ptr()),
+        0 if ws is None else ws.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return st, out.float().reshape(B, H, D).cpu().numpy()
+
+
+@pytest.mark.parametrize("D,S", [(64, 130), (128, 130), (64, 400), (128, 64), (64, 1)])
+def test_infinite_value_scale_stays_in_its_dims(gpu, D, S):
+    # fewer chunks than the block kernel's 8 waves: the absent ones add nothing, also where
+    # a present one holds infinities (inf, with the sign of v, and NaN only where v is 0)
+    c = workloads.decode_case(1, 3, D, S, seed=D + S, device=gpu, outlier_frac=0.0)
+    assert capi.decode_num_splits(3, S, D) < 8
+    c["sV"][..., S - 1] = float("inf")
+    st, out = _decode(c, S, None)
+    assert st == capi.INT8K_OK
+    v = c["Vi"][:, :, S - 1].cpu().numpy().astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_array_equal(out, v * np.inf)
+
+
 @pytest.mark.parametrize("D,page,lens", [(64, 16, [6000, 1, 17, 3000]), (128, 64, [9000, 65]),
                                          (64, 1024, [5001, 0]), (128, 16, [20000])])
 def test_grouped_paged_plans_match_float64(gpu, D, page, lens):
