@@ -68,8 +68,12 @@ const char* int8k_last_error(void);
 /*                                                                          */
 /* The workspace holds split partials.  Plans of at most 16 chunks per (b,h) */
 /* merge their chunks on chip and need none: the query returns 0 and the    */
-/* call accepts a null workspace for them.  Automatic plans above 16 chunks  */
-/* whose (b,h) would also fit that way fall back to it without a workspace.  */
+/* call accepts a null workspace for them.  Automatic plans above that run   */
+/* several blocks per (b,h) and need room for a partial of each, at most     */
+/* max(8, 256 / BH); where the chunks of a (b,h) also fit one block (a short */
+/* sequence), a call with no or a smaller workspace runs that way instead of */
+/* being refused.  Forced plans above 16 chunks need room for a partial per  */
+/* chunk.                                                                    */
 /* ------------------------------------------------------------------------ */
 size_t int8k_decode_attention_workspace_bytes(int BH, int S, int head_dim, int nsplit);
 
@@ -88,7 +92,9 @@ int int8k_decode_attention_forward_quant(
     int BH, int S, int head_dim, int nsplit,
     void* workspace, size_t workspace_bytes, void* stream);
 
-/* The split count the forward call uses for this shape (after clamping). */
+/* The split count the forward call uses for this shape (after clamping).  An
+ * automatic plan above 16 is run by as many blocks of up to 8 waves per (b,h)
+ * as fill the GPU, each wave on a chunk of its own. */
 int int8k_decode_attention_num_splits(int BH, int S, int head_dim, int nsplit);
 
 /* int8k_decode_attention_forward without a workspace argument, for callers

@@ -91,10 +91,25 @@ struct DecodeTuning {
     int pair_flags;    // load flags of the paired-row kernels (D=64, 4 slots, <= 8 chunks)
 };
 
+
+// How the chunks of a (b,h) are laid out on blocks: `blocks` blocks of `waves`
+// waves, each wave `chunk` rows.  The states of a block's waves merge on chip;
+// with more than one block per (b,h) each leaves a partial for
+// decode_combine_kernel.
+struct GroupPlan {
+    int blocks, waves, chunk;
+};
+
+// A decode's plan: chunks per (b,h) and their rows, the blocks that run them, and the
+// partials per (b,h) that the workspace has room for.  An automatic plan above
+// kMaxBlockSplits chunks has its own rows per wave in g; its nsplit is only what
+// num_splits reports.
 struct SplitPlan {
     int nsplit;
     int chunk;
     bool forced;  // the caller's split count
+    GroupPlan g;
+    int partials;
 };
 
 // Most waves (chunks) per block of the one-launch and grouped kernels' fast instance.
@@ -158,14 +173,12 @@ DecodeTuning tuning_for(int D) {
     return t;
 }
 
-// How the chunks of a (b,h) are laid out on blocks: `blocks` blocks of `waves`
-// waves, each wave `chunk` rows.  The states of a block's waves merge on chip;
-// with more than one block per (b,h) each leaves a partial for
-// decode_combine_kernel.
-struct GroupPlan {
-    int blocks, waves, chunk;
-};
 constexpr int kNumCus = 256;
+
+// Most blocks per (b,h) of an automatic plan: 8, or one for each CU.
+inline long long most_groups(int BH, long long iters) {
+    return std::min(ceil_div(iters, kGroupWaves), std::max(8LL, (long long)kNumCus / BH));
+}
 
 // Automatic plans of the 8-wave kernels take the blocks per (b,h) (at most `most`)
 // with the smallest cost in wave iterations: a round is one block on each CU,
@@ -173,8 +186,9 @@ constexpr int kNumCus = 256;
 // merge, and the second launch about 4 at D = 64 and 2 at D = 128 (a CU streams
 // one block at ~55 GB/s: 1.27 and 2.5 us per iteration).  So short sequences stay
 // on one block (B1 H16 D128 1500 rows, B1 H12 D64 2500 rows) and longer ones spread
-// (paged B4 H16 D64 4000 rows: 15.7 us on one block, 10.4 on four and a combine; B1 H12 D64 4096 rows: 13.2 -> 12.3 us on 8 blocks,
-// B1 H8 D128 3000 rows 19.6 -> 12.2, B4 H12 D128 2500 rows 18.4 -> 12.3).
+// (paged B4 H16 D64 4000 rows: 15.7 us on one block, 10.4 on four and a combine; B1 H12
+// D64 4096 rows: 13.2 -> 12.3 us on 8 blocks, B1 H8 D128 3000 rows 19.6 -> 12.2, B4 H12
+// D128 2500 rows 18.4 -> 12.3).
 // Sweeps of 1..32 blocks at 8 to 64 (b,h) put the best time at one full round or
 // within 3% of it (B2 H8 D128 60013 rows: 53.2 / 44.1 / 46.0 us at 8 / 16 / 32
 // blocks; B1 H32 D64 128K: 103 / 87 / 88 us at 4 / 8 / 16): a partial extra round
@@ -182,8 +196,7 @@ constexpr int kNumCus = 256;
 GroupPlan plan_groups(int BH, int S, int D, int slots, long long most) {
     const int R = rows_per_iter(D, slots);
     const long long iters = ceil_div(S, R);
-    most = std::max(1LL, std::min({most, ceil_div(iters, kGroupWaves),
-                                   std::max(8LL, (long long)kNumCus / BH)}));
+    most = std::max(1LL, std::min(most, most_groups(BH, iters)));
     long long best = -1, per_wave = 0, blocks = 1;
     for (long long nb = 1; nb <= most; ++nb) {
         const long long pw = ceil_div(iters, nb * kGroupWaves);
@@ -196,14 +209,23 @@ GroupPlan plan_groups(int BH, int S, int D, int slots, long long most) {
     return GroupPlan{(int)blocks, waves, (int)(per_wave * R)};
 }
 
+// A forced plan keeps its chunks, up to kGroupWaves to a block.
+inline GroupPlan forced_groups(int nsplit, int chunk) {
+    const int blocks = (int)ceil_div(nsplit, kGroupWaves);
+    return GroupPlan{blocks, (int)ceil_div(nsplit, blocks), chunk};
+}
+
 // Split-count choice: a unit is one wave over one KV chunk of one (b,h);
 // aim for tuning.target_units units in total, each chunk a multiple of the
-// rows one wave iteration covers.
+// rows one wave iteration covers.  on_chip: an automatic plan that merges on chip
+// wherever it did without the choice of several blocks.
 SplitPlan plan_splits(int BH, int S, int D, int nsplit_req, bool on_chip = false) {
     const DecodeTuning tn = tuning_for(D);
     const int R = rows_per_iter(D, tn.slots);
     const long long max_split = ceil_div(S, R);
     long long ns;
+    bool several = false;  // blocks per (b,h) from plan_groups
+    GroupPlan g{};
     if (nsplit_req > 0) {
         ns = nsplit_req;
     } else {
@@ -215,26 +237,26 @@ SplitPlan plan_splits(int BH, int S, int D, int nsplit_req, bool on_chip = false
             1, std::max(ceil_div(S, 4LL * R), std::min<long long>(kMaxAutoBlockSplits, ceil_div(S, R))));
         ns = std::min(ns, by_len);
         if (ns > kMaxAutoBlockSplits && ns <= kMaxBlockSplits) ns = kMaxAutoBlockSplits;
-        // Few (b,h): several blocks each, where that pays for the second launch.  nsplit
-        // then only sizes the workspace (above kMaxBlockSplits, so that it is one).
+        // Few (b,h): several blocks each, where that pays for the second launch; reported
+        // as 8 chunks per block, and more than kMaxBlockSplits also for two blocks
         if (ns == kMaxAutoBlockSplits && !on_chip && max_split > kMaxBlockSplits) {
-            const GroupPlan g = plan_groups(BH, S, D, tn.slots, max_split);
+            g = plan_groups(BH, S, D, tn.slots, max_split);
             if (g.blocks > 1)
                 ns = std::min(max_split, std::max(3LL, (long long)g.blocks) * kGroupWaves);
-            if (ns > kMaxBlockSplits)
-                return SplitPlan{(int)ns, (int)round_up((size_t)ceil_div(S, ns), (size_t)R), false};
+            several = ns > kMaxBlockSplits;
         }
     }
     ns = std::max<long long>(1, std::min(ns, max_split));
     long long chunk = round_up((size_t)ceil_div(S, ns), (size_t)R);
-    ns = ceil_div(S, chunk);
-    return SplitPlan{(int)ns, (int)chunk, nsplit_req > 0};
-}
-
-// A forced plan keeps its chunks, up to kGroupWaves to a block.
-inline GroupPlan forced_groups(const SplitPlan& plan) {
-    const int blocks = (int)ceil_div(plan.nsplit, kGroupWaves);
-    return GroupPlan{blocks, (int)ceil_div(plan.nsplit, blocks), plan.chunk};
+    if (!several) ns = ceil_div(S, chunk);
+    if (ns <= kMaxBlockSplits && use_block_kernel())
+        return SplitPlan{(int)ns, (int)chunk, nsplit_req > 0, GroupPlan{1, (int)ns, (int)chunk}, 0};
+    if (nsplit_req > 0 || !use_block_kernel())
+        return SplitPlan{(int)ns, (int)chunk, nsplit_req > 0, forced_groups((int)ns, (int)chunk), (int)ns};
+    if (!several) g = plan_groups(BH, S, D, tn.slots, ns);
+    // room for the most blocks, not those picked: it does not shrink with S, so that a
+    // workspace sized for the longest sequence serves the shorter ones
+    return SplitPlan{(int)ns, (int)chunk, false, g, (int)most_groups(BH, max_split)};
 }
 
 struct Int4 {
@@ -988,24 +1010,15 @@ int launch_decode(const DecodeArgs& a, const DecodeOut& o, const SplitPlan& plan
         if (tn.slots == 4) f(std::integral_constant<int, 4>{});
         else f(std::integral_constant<int, 8>{});
     };
-    if (plan.nsplit <= kMaxBlockSplits && use_block_kernel()) {
-        // one launch: the chunks of a (b,h) are the waves of one block
-        const GroupPlan g{1, plan.nsplit, plan.chunk};
-        with_ns([&](auto ns) {
-            if (plan.nsplit <= kGroupWaves)
-                launch_block<D, ns.value, kGroupWaves, false>(tn, a, o, g, w, stream);
-            else
-                launch_block<D, ns.value, kMaxBlockSplits, false>(tn, a, o, g, w, stream);
-        });
-        return check_launch("decode_block_kernel");
-    }
-    const GroupPlan g = plan.forced || !use_block_kernel()
-                            ? forced_groups(plan)
-                            : plan_groups(a.BH, a.S, D, tn.slots, plan.nsplit);
+    const GroupPlan& g = plan.g;
     const bool group = g.blocks > 1 || !use_block_kernel();
     with_ns([&](auto ns) {
-        if (group) launch_block<D, ns.value, kGroupWaves, true>(tn, a, o, g, w, stream);
-        else launch_block<D, ns.value, kGroupWaves, false>(tn, a, o, g, w, stream);
+        if (group)
+            launch_block<D, ns.value, kGroupWaves, true>(tn, a, o, g, w, stream);
+        else if (g.waves <= kGroupWaves)  // one launch: the waves of one block
+            launch_block<D, ns.value, kGroupWaves, false>(tn, a, o, g, w, stream);
+        else
+            launch_block<D, ns.value, kMaxBlockSplits, false>(tn, a, o, g, w, stream);
     });
     int st = check_launch("decode_block_kernel");
     if (st != INT8K_OK || !group) return st;
@@ -1030,7 +1043,7 @@ int launch_decode_paged(const int8_t* Q, const int8_t* Kp, const int8_t* Vp, con
     const bool one_launch = plan.nsplit <= kGroupWaves && use_block_kernel();
     GroupPlan g;
     if (plan.forced || !use_block_kernel())
-        g = one_launch ? GroupPlan{1, plan.nsplit, plan.chunk} : forced_groups(plan);
+        g = plan.g;
     else
         g = plan_groups(BH, max_context, D, NS, plan.nsplit);
     // short chunks keep the plan's waves: more of them only add merges
@@ -1101,12 +1114,9 @@ extern "C" int int8k_decode_attention_num_splits(int BH, int S, int head_dim, in
     return plan_splits(BH, S, head_dim, nsplit).nsplit;
 }
 
-// Workspace a contiguous-cache decode with this plan needs: none when the chunks
-// of each (b,h) merge on chip (decode_block_kernel writes no partials), else
-// room for m, l and acc[D] per chunk (its blocks leave one partial for up to 8).
+// Workspace a contiguous-cache decode with this plan needs: m, l and acc[D] per partial.
 static size_t decode_partial_bytes(const SplitPlan& plan, long long BH, int D) {
-    if (plan.nsplit <= kMaxBlockSplits && use_block_kernel()) return 0;
-    return carve(nullptr, BH * plan.nsplit, D).bytes;
+    return plan.partials > 0 ? carve(nullptr, BH * plan.partials, D).bytes : 0;
 }
 
 extern "C" size_t int8k_decode_attention_workspace_bytes(int BH, int S, int head_dim, int nsplit) {
@@ -1118,10 +1128,9 @@ extern "C" size_t int8k_decode_attention_workspace_bytes(int BH, int S, int head
 // not fit falls back to one block per (b,h) where its chunks merge on chip.
 static SplitPlan plan_within(int BH, int S, int D, int nsplit, size_t have) {
     const SplitPlan plan = plan_splits(BH, S, D, nsplit);
-    if (plan.forced || plan.nsplit <= kMaxBlockSplits || have >= decode_partial_bytes(plan, BH, D))
-        return plan;
+    if (plan.forced || have >= decode_partial_bytes(plan, BH, D)) return plan;
     const SplitPlan small = plan_splits(BH, S, D, 0, true);
-    return small.nsplit <= kMaxBlockSplits ? small : plan;
+    return small.partials == 0 ? small : plan;
 }
 
 size_t int8k::decode_partials_within(int BH, int S, int head_dim, int nsplit, size_t have) {
@@ -1147,15 +1156,16 @@ static int decode_impl(const int8_t* Q, const int8_t* K, const int8_t* V, const 
         !out_ok(out))
         return INT8K_ERR_MISALIGNED;
     const SplitPlan plan = plan_within(BH, S, head_dim, nsplit, workspace ? workspace_bytes : 0);
-    const long long units = (long long)BH * plan.nsplit;
-    if (units >= (1LL << 26)) return INT8K_ERR_UNSUPPORTED;  // 64 work-items per unit, < 2^32
+    // 64 work-items per unit, < 2^32
+    const long long waves = std::max<long long>(plan.forced ? plan.nsplit : 0,
+                                                (long long)plan.g.blocks * plan.g.waves);
+    if (BH * waves >= (1LL << 26)) return INT8K_ERR_UNSUPPORTED;
     // the one-launch path reads no workspace: a null or short one is accepted there
-    if (decode_partial_bytes(plan, BH, head_dim) > 0) {
-        if (!workspace || workspace_bytes < carve(nullptr, units, head_dim).bytes)
-            return INT8K_ERR_WORKSPACE;
+    if (const size_t need = decode_partial_bytes(plan, BH, head_dim)) {
+        if (!workspace || workspace_bytes < need) return INT8K_ERR_WORKSPACE;
         if (!aligned_to(workspace, 16)) return INT8K_ERR_MISALIGNED;
     }
-    const DecodeWorkspace w = carve(workspace, units, head_dim);
+    const DecodeWorkspace w = carve(workspace, (long long)BH * plan.partials, head_dim);
     const DecodeArgs a{Q,  K, V,     scale_Q, scale_K, scale_V,
                        BH, S, S_cap, (1.0f / std::sqrt((float)head_dim)) * kLog2e};
     return head_dim == 128 ? launch_decode<128>(a, out, plan, w, as_stream(stream))
@@ -1221,7 +1231,10 @@ static SplitPlan plan_paged(int BH, int max_context, int D, int nsplit_req) {
     ns = std::max<long long>(1, std::min(ns, max_split));
     const long long chunk = round_up((size_t)ceil_div(max_context, ns), (size_t)R);
     ns = ceil_div(max_context, chunk);
-    return SplitPlan{(int)ns, (int)chunk, nsplit_req > 0};
+    const GroupPlan g = ns <= kGroupWaves && use_block_kernel()
+                            ? GroupPlan{1, (int)ns, (int)chunk}
+                            : forced_groups((int)ns, (int)chunk);
+    return SplitPlan{(int)ns, (int)chunk, nsplit_req > 0, g, (int)ns};
 }
 
 extern "C" size_t int8k_decode_attention_paged_workspace_bytes(int B, int H, int max_context,

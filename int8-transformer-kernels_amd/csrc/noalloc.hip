@@ -14,9 +14,9 @@
 //
 // Only plans of more than 16 chunks per (b,h) run as several blocks each and write
 // partials; the one-launch plans merge their chunks on chip, need no scratch
-// and are never refused for size (the workspace query returns 0 for them).  An
-// automatic plan of several blocks whose partials exceed the scratch runs as one
-// launch instead where its (b,h) fill the GPU (B33 H16 D128 32768 rows).
+// and are never refused for size (the workspace query returns 0 for them).
+// Automatic plans of several blocks leave a partial per block, which the scratch
+// holds (B33 H16 D128 32768 rows: 1.1 MB); forced plans need one per chunk.
 // Every call on a GPU shares that GPU's array and leaves its partials there.
 // Nothing in it has to start at zero: each block writes its partial before the
 // combine kernel reads it.  Two calls that overlap on one

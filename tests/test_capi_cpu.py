@@ -46,7 +46,7 @@ def test_decode_argument_validation(capi):
     assert _decode_call(lib, D=256) == capi.INT8K_ERR_UNSUPPORTED
     assert _decode_call(lib, K=0x20001) == capi.INT8K_ERR_MISALIGNED
     assert _decode_call(lib, sK=0x60002) == capi.INT8K_ERR_MISALIGNED
-    # a forced 32-chunk plan runs the split kernel, whose partials need a workspace
+    # a forced 32-chunk plan runs several blocks per (b,h), whose partials need a workspace
     need = capi.decode_workspace_bytes(4, 8192, 128, 32)
     assert need > 0
     assert _decode_call(lib, S=8192, nsplit=32, ws_bytes=need - 1) == capi.INT8K_ERR_WORKSPACE
@@ -76,7 +76,7 @@ def test_decode_split_plan(capi, BH, S, D):
 
 def test_decode_auto_plans_skip_9_to_16_chunks(capi):
     # automatic plans take at most 8 chunks per (b,h) on the one-launch kernel (the 8-wave
-    # instance) or more than 16 on the split kernel; forced counts of 9..16 are honoured
+    # instance) or report more than 16 and run several blocks; forced counts of 9..16 are honoured
     for D in (64, 128):
         for BH in (1, 2, 12, 32, 64, 128, 256, 384, 512, 1024, 4096):
             for S in (1, 63, 64, 100, 1024, 2048, 3000, 4096, 8192, 16384, 40000, 131072):
@@ -84,6 +84,16 @@ def test_decode_auto_plans_skip_9_to_16_chunks(capi):
                 assert 1 <= ns <= 8 or ns > 16, (BH, S, D, ns)
         assert capi.decode_num_splits(12, 1024, D, 16) == 16
     assert capi.decode_num_splits(12, 1024, 64) == 8
+
+
+@pytest.mark.parametrize("BH,D", [(2, 64), (12, 64), (100, 64), (16, 128), (384, 128), (528, 128)])
+def test_decode_workspace_of_automatic_plans(capi, BH, D):
+    # one partial per block, at most 8 blocks or as many as fill 256 CUs, and no less for a
+    # longer sequence: a workspace sized for the longest serves the shorter ones
+    sizes = [capi.decode_workspace_bytes(BH, S, D) for S in range(64, 131072, 97)]
+    used = [n for n in sizes if n]
+    assert used and used == sorted(used)
+    assert used[-1] <= BH * max(8, 256 // BH) * (D + 2) * 4 + 512
 
 
 @pytest.mark.parametrize("B,H,S,D", [(1, 1, 1, 64), (8, 32, 32768, 64), (32, 32, 8192, 128),
@@ -204,7 +214,7 @@ def test_quantized_attention_output_validation(capi):
         assert fwd(flags) == capi.INT8K_ERR_UNSUPPORTED
     for flags in (4, 8, -1):
         assert fwd(flags) == capi.INT8K_ERR_INVALID_ARGUMENT
-    # a forced 32-chunk plan: the split kernel, whose partials need a workspace
+    # a forced 32-chunk plan: several blocks per (b,h), whose partials need a workspace
     dec = lambda q=0x40000, s=0x48000, ws_bytes=1 << 30: (  # noqa: E731
         lib.int8k_decode_attention_forward_quant(
             F(0x10000), F(0x20000), F(0x30000), F(q), F(s), F(0x50000), F(0x60000), F(0x70000),

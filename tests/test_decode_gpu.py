@@ -93,7 +93,7 @@ def test_decode_chunk_iteration_counts(capi, gpu, D):
 @pytest.mark.parametrize("D", [64, 128])
 def test_decode_few_heads_long_context(capi, gpu, D):
     # few (b,h) and a long context: the automatic plan has more than 16 chunks per
-    # (b,h), so it runs the split kernel and the combine kernel
+    # (b,h), so it runs several blocks per (b,h) and the combine kernel
     case = workloads.decode_case(1, 2, D, 40000, seed=17, outlier_frac=0.01, device=gpu)
     assert capi.decode_num_splits(2, 40000, D, 0) > 16
     out = _run_capi(capi, case)

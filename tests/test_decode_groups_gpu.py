@@ -3,8 +3,7 @@
 Shapes sit at the edges of the layout: one row past a whole wave iteration, odd row
 strides at D = 64 (the paired rows count from the row before a head that starts in the
 middle of a 128-byte line), a cache longer than the sequence, chunks that end inside an
-iteration, empty tail blocks, and the same calls without a workspace (one block per
-(b,h)).  Against float64 attention with fp32 sums' bound: the fp16 rounding of the
+iteration, empty tail blocks, and the same calls without a workspace.  Against float64 attention with fp32 sums' bound: the fp16 rounding of the
 output (2^-11 relative) plus the 2e-3 that the fp32 softmax over up to 2^15 rows moves.
 """
 import ctypes
@@ -28,56 +27,6 @@ def _ref(c, S):
     return (torch.softmax(s, -1).unsqueeze(-1) * v).sum(2).cpu().numpy()
 
 
-@pytest.mark.parametrize("B,H,D,S,cap", [
-    (1, 3, 64, 4097, 4097), (1, 5, 64, 8191, 8191), (2, 3, 64, 5000, 5001), (1, 2, 64, 33, 37),
-    (1, 3, 64, 2049, 2050), (3, 7, 64, 63, 63), (1, 3, 128, 2113, 2113), (2, 2, 128, 12001, 12288),
-    (1, 1, 128, 1600, 1601), (1, 300, 64, 515, 515), (5, 60, 128, 3001, 3001)])
-def test_grouped_plans_match_float64(gpu, B, H, D, S, cap):
-    c = workloads.decode_case(B, H, D, cap, seed=S, device=gpu, outlier_frac=0.01)
-    BH = B * H
-    out = torch.empty((BH, D), dtype=torch.float16, device=gpu)
-    n = capi.decode_workspace_bytes(BH, S, D)
-    ref = _ref(c, S)
-    for ws in ([torch.empty(max(n, 1), dtype=torch.uint8, device=gpu)] +
-               ([None] if capi.decode_num_splits(BH, S, D) * 64 <= 8 * 2048 else [])):
-        st = capi.load().int8k_decode_attention_forward_cache(
-            *(ctypes.c_void_p(t.data_ptr()) for t in (c["Qi"], c["Ki"], c["Vi"], out, c["sQ"],
-                                                      c["sK"], c["sV"])),
-            BH, S, cap, D, 0, ctypes.c_void_p(ws.data_ptr() if ws is not None else 0),
-            n if ws is not None else 0,
-            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-        torch.cuda.synchronize()
-        if ws is None and st == capi.INT8K_ERR_WORKSPACE:
-            assert n > 0  # a plan that always leaves partials
-            continue
-        assert st == capi.INT8K_OK
-        assert_attn_close(out.float().reshape(B, H, D).cpu().numpy(), ref, f"{B} {H} {D} {S} {cap}")
-
-
-def test_short_sequences_without_workspace_stay_on_one_block(gpu):
-    # spread over more blocks with a workspace, one block per (b,h) without: both accepted
-    B, H, D, S = 1, 12, 64, 6000
-    c = workloads.decode_case(B, H, D, S, seed=5, device=gpu)
-    outs = []
-    for ws_bytes in (capi.decode_workspace_bytes(12, S, D), 0):
-        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=gpu)
-        out = torch.empty((B * H, D), dtype=torch.float16, device=gpu)
-        st = capi.load().int8k_decode_attention_forward(
-            *(ctypes.c_void_p(t.data_ptr()) for t in (c["Qi"], c["Ki"], c["Vi"], out, c["sQ"],
-                                                      c["sK"], c["sV"])),
-            B * H, S, D, 0, ctypes.c_void_p(ws.data_ptr() if ws_bytes else 0), ws_bytes,
-            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-        torch.cuda.synchronize()
-        outs.append((st, out.float().cpu().numpy()))
-    ref = _ref(c, S).reshape(B * H, D)
-    for i, (st, o) in enumerate(outs):
-        if st != capi.INT8K_OK:
-            assert i == 1 and capi.decode_num_splits(12, S, D) > 16
-        else:
-            assert_attn_close(o, ref, f"workspace {i == 0}")
-    assert outs[0][0] == capi.INT8K_OK
-
-
 def _decode(c, S, ws):
     """Status and rows of the cache entry with the workspace tensor `ws` (None: a null one)."""
     B, H, cap, D = c["Ki"].shape
@@ -89,6 +38,34 @@ def _decode(c, S, ws):
         0 if ws is None else ws.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     torch.cuda.synchronize()
     return st, out.float().reshape(B, H, D).cpu().numpy()
+
+
+# null: what a call without a workspace does: "none" is needed, it falls back to "one" block per
+# (b,h), or it is refused (a plan of more than 16 chunks that never merged on chip)
+@pytest.mark.parametrize("B,H,D,S,cap,null", [
+    (1, 3, 64, 4097, 4097, "refused"), (1, 5, 64, 8191, 8191, "refused"),
+    (2, 3, 64, 5000, 5001, "refused"), (1, 12, 64, 6000, 6000, "refused"),
+    (2, 2, 128, 12001, 12288, "refused"), (1, 12, 64, 4096, 4096, "one"),
+    (1, 3, 128, 2113, 2113, "one"), (1, 1, 128, 1600, 1601, "one"), (4, 16, 128, 2000, 2001, "one"),
+    (1, 2, 64, 33, 37, "none"), (1, 3, 64, 2049, 2050, "none"), (3, 7, 64, 63, 63, "none"),
+    (1, 300, 64, 515, 515, "none"), (5, 60, 128, 3001, 3001, "none")])
+def test_grouped_plans_match_float64(gpu, B, H, D, S, cap, null):
+    c = workloads.decode_case(B, H, D, cap, seed=S, device=gpu, outlier_frac=0.01)
+    n = capi.decode_workspace_bytes(B * H, S, D)
+    assert (n == 0) == (null == "none")
+    ref = _ref(c, S)
+    label = f"{B} {H} {D} {S} {cap}"
+    st, out = _decode(c, S, torch.empty(max(n, 1), dtype=torch.uint8, device=gpu))
+    assert st == capi.INT8K_OK
+    assert_attn_close(out, ref, label)
+    # no workspace, and one byte less than the plan's partials
+    for ws in [None] + ([torch.empty(n - 1, dtype=torch.uint8, device=gpu)] if n else []):
+        st, out = _decode(c, S, ws)
+        if null == "refused":
+            assert st == capi.INT8K_ERR_WORKSPACE
+        else:
+            assert st == capi.INT8K_OK
+            assert_attn_close(out, ref, label)
 
 
 @pytest.mark.parametrize("D,S", [(64, 130), (128, 130), (64, 400), (128, 64), (64, 1)])

@@ -70,7 +70,7 @@ def test_paged_decode_via_torch_op(ext, gpu):
 @pytest.mark.parametrize("nsplit", [1, 2, 7, 64])
 def test_paged_decode_forced_splits(gpu, D, nsplit):
     # up to 8 chunks: the one-launch kernel (paired rows at D=64, whose 8-row pair
-    # blocks must stay inside one page); 64: the split kernel and the combine
+    # blocks must stay inside one page); 64: several blocks per (b,h) and the combine
     lens = [1000, 64, 513]
     c = workloads.paged_case(3, 2, D, 32, lens, seed=nsplit + D, device=gpu)
     out = capi.decode_attention_paged(c["Qi"], c["K_pages"], c["V_pages"], c["sQ"],
@@ -139,7 +139,7 @@ def test_paged_decode_zero_length_and_clamped_pages(gpu):
 @pytest.mark.parametrize("nsplit", [4, 64])
 def test_paged_bad_page_ids_are_counted(gpu, nsplit):
     # an out-of-range id among the entries a sequence uses is counted (the one-launch kernel
-    # at 4 chunks, the split kernel at 64); ids in entries past a sequence's length are never
+    # at 4 chunks, several blocks at 64); ids in entries past a sequence's length are never
     # read and never counted
     lens = [1000, 40]
     c = workloads.paged_case(2, 2, 64, 16, lens, seed=6, device=gpu)

@@ -3,7 +3,7 @@
 The no-alloc entry point runs the same kernels with the split partials in the
 library's device scratch instead of a caller workspace, so its output must
 equal the workspace entry point's byte for byte.  Only plans of more than 16
-chunks per (b,h) run the split kernel and touch the scratch, so every pair
+chunks per (b,h) run several blocks and touch the scratch, so every pair
 below forces such plans on both calls: the second call, smaller, must not see
 the first call's partials.  Plans that merge their chunks on chip need no
 scratch and are accepted at any size.  The size limit itself is checked on
@@ -52,12 +52,14 @@ def test_noalloc_on_chip_plans_need_no_scratch(capi):
     assert capi.decode_workspace_bytes(65536, 64, 64) == 0
 
 
-@pytest.mark.parametrize("BH,S,D", [(519, 32768, 128), (1163, 131072, 128), (528, 65536, 128)])
-def test_noalloc_large_automatic_plans_fall_back_to_one_block(capi, BH, S, D):
-    # several blocks per (b,h) would leave more partials than the scratch holds: the call runs
-    # on one block per (b,h) instead.  (The odd K address is refused after the size check, so
-    # nothing is launched; without a GPU the scratch lookup before it fails.)
-    assert capi.decode_workspace_bytes(BH, S, D) > 8 << 20
+@pytest.mark.parametrize("BH,S,D", [(519, 32768, 128), (1163, 131072, 128), (528, 65536, 128),
+                                    (64, 2000, 128), (12, 4096, 64), (12, 6000, 64)])
+def test_noalloc_takes_every_automatic_plan(capi, BH, S, D):
+    # several blocks per (b,h), at most 8 or as many as fill 256 CUs, leave one partial each,
+    # which fits the scratch.  (The odd K address is refused after the size check, so nothing is
+    # launched; without a GPU the scratch lookup before it fails.)
+    partials = BH * max(8, 256 // BH) * (D + 2) * 4
+    assert 0 < capi.decode_workspace_bytes(BH, S, D) <= min(partials + 512, 8 << 20)
     args = [ctypes.c_void_p(0x10000 * (i + 1) + (i == 1)) for i in range(7)]
     st = capi.load().int8k_decode_attention_forward_noalloc(*args, BH, S, D, 0, None)
     assert st in (capi.INT8K_ERR_MISALIGNED, capi.INT8K_ERR_HIP), st
