@@ -289,7 +289,15 @@ int int8k_attention_forward_quant(
  * counterpart in the reference; for comparison and measurement). */
 #define INT8K_MLP_SEPARATE_REQUANT 4
 
+/* int8k_mlp_workspace_bytes: a workspace of this size serves every call of up
+ * to T rows with the same d_model, d_ff and flags.  (Few rows are split over K
+ * into partials, so a shorter call may need more than a longer one.  Unpacked
+ * weights: GEMM2 off the 256 x 256 kernels also asks for the room of a
+ * transposed W2, which the size for a T on them does not hold.)
+ * int8k_mlp_call_workspace_bytes: what a call of exactly T rows needs, for
+ * callers that allocate per call. */
 size_t int8k_mlp_workspace_bytes(int T, int d_model, int d_ff, int flags);
+size_t int8k_mlp_call_workspace_bytes(int T, int d_model, int d_ff, int flags);
 
 /* Diagnostics of the fused requantization: *count receives how many tiles, on
  * the current device since the library was loaded, stopped waiting for their

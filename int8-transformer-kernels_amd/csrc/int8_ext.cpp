@@ -306,7 +306,7 @@ std::tuple<torch::Tensor, torch::Tensor> run_mlp(const torch::Tensor& x, const t
     auto out_scale = torch::empty({per_tensor ? 1 : d.T},
                                   torch::TensorOptions().dtype(torch::kFloat32).device(x.device()));
     const size_t ws_bytes =
-        int8k_mlp_workspace_bytes((int)d.T, (int)d.d_model, (int)d.d_ff, flags);
+        int8k_mlp_call_workspace_bytes((int)d.T, (int)d.d_model, (int)d.d_ff, flags);
     auto ws = workspace(ws_bytes, x.device());
     const int st = int8k_mlp_forward(
         xa.data_ptr<int8_t>(), w1.data_ptr<int8_t>(), w2.data_ptr<int8_t>(),

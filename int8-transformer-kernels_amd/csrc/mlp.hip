@@ -1728,7 +1728,6 @@ MlpPlan mlp_plan(int T, int dm, int dff, int flags) {
 
 // Workspace layout of one MLP call (all offsets 256-byte aligned).
 struct MlpWorkspace {
-    int8_t* w2t;      // [d_model][d_ff]   (unpacked weights, see w2_room)
     uint16_t* h16;    // [T][d_ff]          (absent with direct1)
     int8_t* hq;       // [T][d_ff]
     float* sh;        // [T]
@@ -1739,10 +1738,14 @@ struct MlpWorkspace {
     uint32_t* sync;   // fused requant: amax1 [T], amax2 [T], arrived1 [tiles_m], arrived2 [tiles_m]
     int sync_words;
     int32_t* part;    // int32 partials (the larger GEMM's)
+    int8_t* w2t;      // [d_model][d_ff]   (unpacked weights, see carve_mlp)
     size_t bytes;
 };
 
-MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const MlpPlan& pl) {
+// Unpacked calls ask for the room of W2's transposed copy wherever GEMM2 may leave the
+// 256 x 256 kernels; copy_room: whether to count it where the call does not transpose.
+MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const MlpPlan& pl,
+                       bool copy_room = true) {
     char* p = static_cast<char*>(base);
     size_t off = 0;
     auto take = [&](size_t n) {
@@ -1751,10 +1754,6 @@ MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const
         return r;
     };
     MlpWorkspace w{};
-    // the room of W2's copy is asked for wherever GEMM2 may leave the 256 x 256 kernels,
-    // transposed or not: callers size their workspace once, and the switch is read per call
-    const bool w2_room = !prepacked && (!pl.kn2 || pl.g2.route != Route::kTiled);
-    w.w2t = reinterpret_cast<int8_t*>(take(w2_room ? (size_t)dm * dff : 0));
     w.h16 = reinterpret_cast<uint16_t*>(take(pl.direct1 ? 0 : (size_t)T * dff * 2));
     w.hq = reinterpret_cast<int8_t*>(take((size_t)T * dff));
     w.sh = reinterpret_cast<float*>(take((size_t)T * 4));
@@ -1766,6 +1765,8 @@ MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const
     w.sync_words = (pl.rq.g1 || pl.rq.g2) ? 2 * T + 2 * tiles_m : 0;
     w.sync = reinterpret_cast<uint32_t*>(take((size_t)w.sync_words * 4));
     w.part = reinterpret_cast<int32_t*>(take(std::max(pl.g1.part_bytes(T, dff), pl.g2.part_bytes(T, dm))));
+    const bool copy = !prepacked && (!pl.kn2 || (copy_room && pl.g2.route != Route::kTiled));
+    w.w2t = reinterpret_cast<int8_t*>(take(copy ? (size_t)dm * dff : 0));
     w.bytes = off;
     return w;
 }
@@ -1876,10 +1877,57 @@ extern "C" int int8k_transpose_int8_weights(const int8_t* W1, const int8_t* W2, 
     return launch_transpose(W2, W2T, d_ff, d_model, as_stream(stream));
 }
 
+// The last T from `t` on with the routes and tile counts of t (`t` itself at least).
+static int plan_range_end(int t, int dm, int dff) {
+    const long long nk = (long long)dm * dff;
+    int end = t <= kStreamRows || (nk <= kStreamSmallWeights && t <= kStreamRowsSmall)
+                  ? (t + 31) / 32 * 32
+                  : (t + kMidB - 1) / kMidB * kMidB;
+    // where the skinny kernel starts to have the blocks it needs, and its last T
+    const long long edges[3] = {32 * (ceil_div(kSkinnyBlocks * kSkinnyN, dm) - 1),
+                                32 * (ceil_div(kSkinnyBlocks * kSkinnyN, dff) - 1),
+                                (1LL << 30) / nk};
+    for (const long long e : edges)
+        if (e >= t) end = (int)std::min<long long>(end, e);
+    return end;
+}
+
 extern "C" size_t int8k_mlp_workspace_bytes(int T, int d_model, int d_ff, int flags) {
     if (T <= 0 || d_model <= 0 || d_ff <= 0) return 0;
-    return carve_mlp(nullptr, T, d_model, d_ff, (flags & INT8K_MLP_WEIGHTS_PREPACKED) != 0,
-                     mlp_plan(T, d_model, d_ff, flags))
+    const bool prepacked = (flags & INT8K_MLP_WEIGHTS_PREPACKED) != 0;
+    const MlpPlan pl = mlp_plan(T, d_model, d_ff, flags);
+    size_t need = carve_mlp(nullptr, T, d_model, d_ff, prepacked, pl).bytes;
+    // Shorter calls may need more: their GEMMs split K into partials, more of them the fewer
+    // tiles there are.  (W2's copy aside, which T alone asks for or not.)  Within a range of
+    // one route and tile count a plan has fewer splits the longer the call: the range's first
+    // splits with its last rows bound it.  About 1 us a range: 128 -> 384 rows 4 ranges, 16384
+    // rows of 512 -> 2048 40.
+    const size_t copy = need - carve_mlp(nullptr, T, d_model, d_ff, true, pl).bytes;
+    for (int t = 1; t < T;) {
+        const MlpPlan first = mlp_plan(t, d_model, d_ff, flags);
+        if (first.g1.route == Route::kTiled && first.g2.route == Route::kTiled && t > kStreamRowsSmall)
+            break;  // and from here on: no partials, less than T needs
+        const int end = std::min(plan_range_end(t, d_model, d_ff), T);
+        MlpPlan last = mlp_plan(end, d_model, d_ff, flags);
+        last.g1.splits = std::max(last.g1.splits, first.g1.splits);
+        last.g2.splits = std::max(last.g2.splits, first.g2.splits);
+        need = std::max(need, carve_mlp(nullptr, end, d_model, d_ff, true, last).bytes + copy);
+        t = end + 1;
+    }
+    return need;
+}
+
+// The workspace of one call.  On 128 x 128 tiles the room of a copy that is not made is the
+// query's alone: a workspace sized for a longer call, on 256 x 256 tiles, has none.
+static MlpWorkspace call_workspace(void* base, int T, int dm, int dff, bool prepacked,
+                                   const MlpPlan& pl) {
+    return carve_mlp(base, T, dm, dff, prepacked, pl, pl.g2.route != Route::kMid);
+}
+
+extern "C" size_t int8k_mlp_call_workspace_bytes(int T, int d_model, int d_ff, int flags) {
+    if (T <= 0 || d_model <= 0 || d_ff <= 0) return 0;
+    return call_workspace(nullptr, T, d_model, d_ff, (flags & INT8K_MLP_WEIGHTS_PREPACKED) != 0,
+                          mlp_plan(T, d_model, d_ff, flags))
         .bytes;
 }
 
@@ -1924,7 +1972,7 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
         if (int st = check_tiled_operands(T, d_ff, d_model)) return st;
     if (pl.g2.route == Route::kTiled && !pl.a16)
         if (int st = check_tiled_operands(T, d_model, d_ff)) return st;
-    const MlpWorkspace w = carve_mlp(workspace, T, d_model, d_ff, prepacked, pl);
+    const MlpWorkspace w = call_workspace(workspace, T, d_model, d_ff, prepacked, pl);
     if (!workspace || workspace_bytes < w.bytes) return INT8K_ERR_WORKSPACE;
     if (!aligned_to(workspace, 256)) return INT8K_ERR_MISALIGNED;
     int st = configure_lds();

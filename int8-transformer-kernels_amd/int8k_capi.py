@@ -39,6 +39,7 @@ _SIGNATURES = {
     "int8k_decode_attention_num_splits": (_I, [_I, _I, _I, _I]),
     "int8k_decode_attention_forward": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _SZ, _P]),
     "int8k_mlp_workspace_bytes": (_SZ, [_I, _I, _I, _I]),
+    "int8k_mlp_call_workspace_bytes": (_SZ, [_I, _I, _I, _I]),
     "int8k_mlp_forward": (_I, [_P, _P, _P, _P, _P, _I, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I,
                                _P, _SZ, _P]),
     "int8k_transpose_int8_weights": (_I, [_P, _P, _P, _P, _I, _I, _P]),
@@ -216,6 +217,10 @@ def mlp_workspace_bytes(T, d_model, d_ff, flags=0):
     return load().int8k_mlp_workspace_bytes(T, d_model, d_ff, flags)
 
 
+def mlp_call_workspace_bytes(T, d_model, d_ff, flags=0):
+    return load().int8k_mlp_call_workspace_bytes(T, d_model, d_ff, flags)
+
+
 def mlp_sync_timeouts() -> int:
     """Tiles whose wait for their stripe's row maxima gave up (fused requantization), on the
     current device since the library was loaded; synchronises with the device."""
@@ -239,9 +244,9 @@ def mlp_forward(x, W1, W2, sx, sW1, sW2, bias1=None, flags=0, out=None, out_scal
     if out_scale is None:
         n = 1 if flags & MLP_OUT_PER_TENSOR else T
         out_scale = torch.empty(n, dtype=torch.float32, device=x.device)
-    ws_bytes = mlp_workspace_bytes(T, dm, dff, flags)
     if workspace is None:
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+        workspace = torch.empty(mlp_call_workspace_bytes(T, dm, dff, flags), dtype=torch.uint8,
+                                device=x.device)
     st = load().int8k_mlp_forward(
         _ptr(x), _ptr(W1), _ptr(W2), _ptr(out), _ptr(sx), sx.numel(), _ptr(sW1), sW1.numel(),
         _ptr(sW2), sW2.numel(), _ptr(bias1), _ptr(out_scale), T, dm, dff, flags,

@@ -286,10 +286,25 @@ def test_bench_refuses_more_than_one_gpu():
     assert "one GPU" in r.stderr
 
 
+@pytest.mark.parametrize("dm,dff", [(512, 2048), (1024, 4096), (4096, 16384), (768, 3072),
+                                    (4096, 1024), (528, 2192), (1024, 32)])
+def test_mlp_workspace_serves_shorter_calls(capi, dm, dff):
+    # a GEMM of few rows splits K into partials, more of them the fewer tiles it has: a call of
+    # fewer rows may need more than a longer one, and the query covers them all (unpacked: up
+    # to 512 rows, where every call asks for the room of W2's copy)
+    P, PT, SEP = (capi.MLP_WEIGHTS_PREPACKED, capi.MLP_OUT_PER_TENSOR, capi.MLP_SEPARATE_REQUANT)
+    for flags in (P, P | PT, P | SEP, 0):
+        rows = list(range(1, 515 if flags == 0 else 2300)) + ([5000, 9000] if flags else [])
+        sizes = [capi.mlp_workspace_bytes(T, dm, dff, flags) for T in rows]
+        assert sizes == sorted(sizes)
+        needs = [capi.mlp_call_workspace_bytes(T, dm, dff, flags) for T in rows]
+        assert all(n <= s for n, s in zip(needs, sizes))
+
+
 def test_mlp_unpacked_workspace_holds_no_weight_copies(capi):
     # where both GEMMs run the 256 x 256 kernels, the unpacked weights are read as stored:
-    # the workspace holds no transposed copies; the 128 x 128 GEMM2 of (2048, 2048, 8192)
-    # still reads a transposed W2
+    # the workspace holds no transposed copies; with the 128 x 128 GEMM2 of (2048, 2048, 8192)
+    # the query keeps room for a transposed W2 (the fp16-hidden switch reads one)
     P = capi.MLP_WEIGHTS_PREPACKED
     assert capi.mlp_workspace_bytes(4096, 4096, 16384, 0) == capi.mlp_workspace_bytes(
         4096, 4096, 16384, P)
