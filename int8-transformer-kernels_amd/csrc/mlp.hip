@@ -35,7 +35,8 @@
 // gemm_i8_mid_kernel<EPI> runs 128 x 128 tiles, two blocks per CU, with the fp16
 // epilogue or, where the grid leaves CUs idle, split over K into the same partials.
 // gemm_route and mid_plan choose.  The integer sums and the epilogue's expressions
-// are the same on every path.
+// are the same on every path: fp32 values, rounded to fp16 as such (f16_of_f32 where the
+// compiler would round the last product once, v_fma_mixlo_f16).
 #include <algorithm>
 #include <cstdlib>
 
@@ -227,7 +228,8 @@ __device__ __forceinline__ void epilogue_edge(const v16i (&acc)[TM_][TN_], const
                 const float v = epi_value<EPI>(acc[i][j][r], esa[rl], esb[cl], ebias[cl]);
                 if (cok) rmax[r] = fmaxf(rmax[r], fabsf(v));
                 const int row = rbase + i * 32 + acc_row(r, lane);
-                if (row < M && cok) p.c16[(size_t)row * p.ldc + cbase + j * 32] = f32_to_f16_bits(v);
+                if (row < M && cok)
+                    p.c16[(size_t)row * p.ldc + cbase + j * 32] = __half_as_ushort(f16_of_f32(v));
             }
         }
         tile_rowmax(rmax, rowmax + wn * BM_ + wm * WM_ + i * 32, lane);
@@ -1327,7 +1329,7 @@ __global__ __launch_bounds__(256) void gemm_i8_skinny_kernel(const int8_t* __res
     for (int j = 0; j < 4; ++j) {
         const int row = m0 + (threadIdx.x >> 5) + 8 * j;
         if (row < M) {
-            p.c16[(size_t)row * p.ldc + col] = f32_to_f16_bits(v[j]);
+            p.c16[(size_t)row * p.ldc + col] = __half_as_ushort(f16_of_f32(v[j]));
             if (c == 0) p.pmax[(size_t)blockIdx.x * M + row] = __int_as_float(mx[j]);
         }
     }
