@@ -30,8 +30,8 @@
 // Few tokens (decode-time MLPs, T = B): the time is the read of the weights, and
 // gemm_i8_stream_kernel streams them in either layout over all CUs, the K range
 // split over waves and blocks; rows_epilogue_kernel<EPI> then sums the exact int32
-// partials of a row, applies the epilogue and requantizes it.  Small packed GEMMs run
-// gemm_i8_skinny_kernel (32 x 32 tiles).  Between those and 128 big tiles,
+// partials of a row, applies the epilogue and requantizes it.  Small GEMMs run
+// gemm_i8_skinny_kernel (32 x 32 tiles, packed weights or transposed copies).  Between those and 128 big tiles,
 // gemm_i8_mid_kernel<EPI> runs 128 x 128 tiles, two blocks per CU, with the fp16
 // epilogue or, where the grid leaves CUs idle, split over K into the same partials.
 // gemm_route and mid_plan choose.  The integer sums and the epilogue's expressions
@@ -837,9 +837,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_i8_a16_kernel(
 // ---------------------------------------------------------------- few tokens
 // gemm_i8_stream_kernel<MT, BKN>: a GEMM of up to 32 MT rows per row block, whose time
 // is the read of the weights (4096 -> 16384 as stored, 32 rows: 17.5 us per GEMM of 64
-// MiB, 3.8 TB/s, of which ~5 us are the first loads, the merge and the stores).  A wave owns 128 columns over its own range of K and
-// streams 128 x 128-byte weight tiles through its own piece of LDS: 16 loads of
-// 16 bytes per lane in flight, each covering whole 128-byte runs (8 weight rows
+// MiB, 3.8 TB/s, of which ~5 us are the first loads, the merge and the stores).  A wave
+// owns 128 columns over its own range of K and streams 128 x 128-byte weight tiles
+// through its own piece of LDS: 16 loads of 16 bytes per lane in flight, each covering whole 128-byte runs (8 weight rows
 // per instruction) for both layouts, the next tile's loads issued before the
 // current one's MFMAs, no block barrier in the loop.  Fragments come from LDS as
 // in the tiled kernels: 16-byte reads of [N][K] rows, or transposing reads of
@@ -1116,7 +1116,7 @@ __global__ __launch_bounds__(256) void partial_epilogue_kernel(const int32_t* __
 // lane, two groups of four 32-deep k slices in flight.  The four int32
 // partial tiles meet in LDS and the block's 256 threads apply the epilogue,
 // writing one absmax partial per (32-column block, row).  No partial sums
-// leave the chip; split-K over blocks (above) would write them to memory.
+// leave the chip, as those of a K split over blocks do.
 // Rows past M read row M-1 and are not stored.
 // It runs at ~3 us + 7 us per 2^30 multiply-adds on MI355X (latency-bound
 // loads; the tiles re-read A and Bt through L2, ~MNK/16 bytes); see gemm_route for
@@ -1184,36 +1184,49 @@ inline MidPlan mid_plan(int M, int N, int K) {
 // lost 11%.
 constexpr int kMidMaxBigTiles = 128;
 
-// The kernel of an M x N x K GEMM (packed: B is [N][K]).  Measured, us per MLP,
-// packed unless said, in turn:
+// The kernel of an M x N x K GEMM (packed: B is [N][K]; per_token: its rows are requantized
+// one by one).  Measured, us per MLP (GPU time of captured calls), packed unless said:
+//  - packed weights of up to 4 MiB run the skinny kernel to 2^30 multiply-adds, where a
+//    column tile of 128 leaves most CUs idle (streaming -> skinny: 512 -> 512, T = 1 13.7 ->
+//    10.3, T = 64 20.5 -> 12.4; 1024 -> 2048, T = 64 22.7 -> 16.5).  A block reads 32
+//    columns over all of K, so long ones need more blocks (GEMM2 of K = 4096, N = 1024,
+//    skinny / streaming: T = 16 17.9 / 16.1, T = 64 20.8 / 19.8, T = 128 22.9 / 22.1; K =
+//    3072: T = 16 16.3 / 15.4, T = 64 18.2 / 19.1), but for a per-tensor output, which takes
+//    a pass more behind partials (K = 3072, T = 16 16.9 / 18.0; K = 4096 18.3 / 18.4);
+//  - weights as stored are transposed for it above 128 rows, to 5/4 2^28 multiply-adds
+//    (transposes + skinny / streaming / 128 x 128 tiles: 512 -> 512, T = 512 17.4 / 21.4 /
+//    19.0; 1024 -> 1024, T = 256 19.8 / 22.5 / 21.1, T = 384 23.8 / 23.5 / 23.5; 512 -> 2048,
+//    T = 320 23.3 / 25.7 on tiles), in whole transposing tiles (1024 -> 96, T = 320 32.9
+//    against 18.3 on 128 x 128 tiles);
 //  - up to 128 rows the weights' read is the time and the streaming kernel takes it:
 //    4096 -> 16384, T = 32: 62 (skinny) -> 48, as stored 109 (transposes + skinny) ->
-//    49; 2048 -> 8192, T = 64: 33 -> 28.5; with weights of at most 1 MiB up to 512
-//    rows (512 -> 2048, as stored);
-//  - packed weights of up to 4 MiB keep the skinny kernel to 2^30 multiply-adds, where
-//    a column tile of 128 leaves most CUs idle (1024 -> 4096, T = 64: 21 against 25), if
-//    its own grid has at least 128 blocks (4096 -> 1024, T = 16: 32 blocks, GEMM and
-//    requantization 12.7 us, here 9.0);
+//    49; 2048 -> 8192, T = 64: 33 -> 28.5; weights of up to 3 MiB up to 32 rows (as stored,
+//    T = 64, streaming / 128 x 128 tiles: 1024 -> 1024 22.1 / 18.1, 1024 -> 3072 23.0 / 21.9,
+//    1024 -> 4096 23.4 / 23.7);
 //  - then 128 x 128 tiles (split over K) to kMidMaxBigTiles: T = 333, 2048 -> 8192
 //    69 (split-K with a pass of its own for the epilogue and the requantization) ->
 //    45.6; T = 512, 1024 -> 4096 43 (skinny) -> 30; T = 512, 4096 -> 16384 172 -> 107.
-constexpr int kStreamRows = 128, kStreamRowsSmall = 512;
-constexpr long long kStreamSmallWeights = 1LL << 20, kSkinnyWeights = 1LL << 22;
-constexpr long long kSkinnyBlocks = 128;
+constexpr int kStreamRows = 128, kStreamRowsSmall = 32, kFewRows = 512;
+constexpr long long kStreamSmallWeights = 3LL << 20, kSkinnyWeights = 1LL << 22;
+constexpr long long kSkinnyMacs = 1LL << 30, kSkinnyCopyMacs = 5LL << 26;
 
 enum class Route { kStream, kSkinny, kMid, kTiled };
 
-Route gemm_route(int M, int N, int K, bool packed) {
+// Blocks that the skinny kernel needs for a GEMM of depth K.
+inline long long skinny_blocks(int K) { return (K - 2048) / 16; }
+
+Route gemm_route(int M, int N, int K, bool packed, bool per_token) {
     const long long nk = (long long)N * K;
     const long long big_tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const bool skinny = packed && N % kSkinnyN == 0 && K % 512 == 0 && nk <= kSkinnyWeights &&
-                        M * nk <= (1LL << 30) &&
-                        (long long)(N / kSkinnyN) * ((M + 31) / 32) >= kSkinnyBlocks;
+    const bool in_range = packed ? N % kSkinnyN == 0 && M * nk <= kSkinnyMacs
+                                 : N % 128 == 0 && M > kStreamRows && M * nk <= kSkinnyCopyMacs;
+    if (in_range && K % 512 == 0 && nk <= kSkinnyWeights &&
+        (!per_token || (long long)(N / kSkinnyN) * ((M + 31) / 32) >= skinny_blocks(K)))
+        return Route::kSkinny;
     const int stream_rows = nk <= kStreamSmallWeights ? kStreamRowsSmall : kStreamRows;
-    if (M <= stream_rows && N <= kRowsEpiMaxN && K < (1 << 24) && !skinny) return Route::kStream;
-    if (skinny) return Route::kSkinny;
+    if (M <= stream_rows && N <= kRowsEpiMaxN && K < (1 << 24)) return Route::kStream;
     // (few rows of very wide weights: also operands of 4 GiB and more, see check_tiled_operands)
-    const bool few = M <= kStreamRowsSmall && big_tiles < 256;
+    const bool few = M <= kFewRows && big_tiles < 256;
     return few || big_tiles <= kMidMaxBigTiles ? Route::kMid : Route::kTiled;
 }
 
@@ -1227,9 +1240,9 @@ struct GemmPlan {
     size_t part_bytes(int M, int N) const { return (size_t)splits * M * N * 4; }
 };
 
-GemmPlan gemm_plan(int M, int N, int K, bool packed) {
+GemmPlan gemm_plan(int M, int N, int K, bool packed, bool per_token) {
     GemmPlan g{};
-    g.route = gemm_route(M, N, K, packed);
+    g.route = gemm_route(M, N, K, packed, per_token);
     g.epi_tiles = (N + BN - 1) / BN;
     if (g.route == Route::kStream) {
         g.st = stream_plan(M, N, K);
@@ -1690,8 +1703,8 @@ struct RqPlan {
 };
 
 // The kernels of one MLP call.  Unpacked weights are read as the caller stores
-// them ([K][N]) by every GEMM but the fp16-hidden GEMM2, which reads a transposed
-// copy in the workspace.
+// them ([K][N]) by every GEMM but the skinny kernel's and the fp16-hidden GEMM2, which
+// read transposed copies in the workspace.
 struct MlpPlan {
     GemmPlan g1, g2;
     RqPlan rq;
@@ -1711,8 +1724,8 @@ MlpPlan mlp_plan(int T, int dm, int dff, int flags) {
     const bool per_token = (flags & INT8K_MLP_OUT_PER_TENSOR) == 0;
     const bool fused = env_on && (flags & INT8K_MLP_SEPARATE_REQUANT) == 0;
     MlpPlan pl;
-    pl.g1 = gemm_plan(T, dff, dm, packed);
-    pl.g2 = gemm_plan(T, dm, dff, packed);
+    pl.g1 = gemm_plan(T, dff, dm, packed, true);
+    pl.g2 = gemm_plan(T, dm, dff, packed, per_token);
     pl.a16 = gemm2_reads_fp16_hidden() &&
              (pl.g2.route == Route::kMid || pl.g2.route == Route::kTiled);
     auto fusable = [](const GemmPlan& g, int N) {
@@ -1720,8 +1733,8 @@ MlpPlan mlp_plan(int T, int dm, int dff, int flags) {
     };
     pl.rq.g1 = fused && !pl.a16 && fusable(pl.g1, dff);
     pl.rq.g2 = fused && per_token && !pl.a16 && fusable(pl.g2, dm);
-    pl.kn1 = !packed;
-    pl.kn2 = !packed && !pl.a16;
+    pl.kn1 = !packed && pl.g1.route != Route::kSkinny;
+    pl.kn2 = !packed && !pl.a16 && pl.g2.route != Route::kSkinny;
     pl.direct1 = pl.rq.g1 || (!pl.a16 && pl.g1.splits > 0 && dff <= kRowsEpiMaxN);
     pl.direct2 = pl.rq.g2 || (per_token && !pl.a16 && pl.g2.splits > 0 && dm <= kRowsEpiMaxN);
     if (pl.a16) pl.g2.splits = 0, pl.g2.epi_tiles = (dm + BN - 1) / BN;
@@ -1740,6 +1753,7 @@ struct MlpWorkspace {
     uint32_t* sync;   // fused requant: amax1 [T], amax2 [T], arrived1 [tiles_m], arrived2 [tiles_m]
     int sync_words;
     int32_t* part;    // int32 partials (the larger GEMM's)
+    int8_t* w1t;      // [d_ff][d_model]   (unpacked weights that GEMM1 reads transposed)
     int8_t* w2t;      // [d_model][d_ff]   (unpacked weights, see carve_mlp)
     size_t bytes;
 };
@@ -1767,6 +1781,7 @@ MlpWorkspace carve_mlp(void* base, int T, int dm, int dff, bool prepacked, const
     w.sync_words = (pl.rq.g1 || pl.rq.g2) ? 2 * T + 2 * tiles_m : 0;
     w.sync = reinterpret_cast<uint32_t*>(take((size_t)w.sync_words * 4));
     w.part = reinterpret_cast<int32_t*>(take(std::max(pl.g1.part_bytes(T, dff), pl.g2.part_bytes(T, dm))));
+    w.w1t = reinterpret_cast<int8_t*>(take(!prepacked && !pl.kn1 ? (size_t)dm * dff : 0));
     const bool copy = !prepacked && (!pl.kn2 || (copy_room && pl.g2.route != Route::kTiled));
     w.w2t = reinterpret_cast<int8_t*>(take(copy ? (size_t)dm * dff : 0));
     w.bytes = off;
@@ -1882,13 +1897,11 @@ extern "C" int int8k_transpose_int8_weights(const int8_t* W1, const int8_t* W2, 
 // The last T from `t` on with the routes and tile counts of t (`t` itself at least).
 static int plan_range_end(int t, int dm, int dff) {
     const long long nk = (long long)dm * dff;
-    int end = t <= kStreamRows || (nk <= kStreamSmallWeights && t <= kStreamRowsSmall)
-                  ? (t + 31) / 32 * 32
-                  : (t + kMidB - 1) / kMidB * kMidB;
-    // where the skinny kernel starts to have the blocks it needs, and its last T
-    const long long edges[3] = {32 * (ceil_div(kSkinnyBlocks * kSkinnyN, dm) - 1),
-                                32 * (ceil_div(kSkinnyBlocks * kSkinnyN, dff) - 1),
-                                (1LL << 30) / nk};
+    int end = t <= kStreamRows ? (t + 31) / 32 * 32 : (t + kMidB - 1) / kMidB * kMidB;
+    // the skinny kernel's last T, and the one before it has the blocks it needs
+    auto before = [](int N, int K) { return 32 * (ceil_div(skinny_blocks(K) * kSkinnyN, N) - 1); };
+    const long long edges[4] = {before(dff, dm), before(dm, dff), kSkinnyMacs / nk,
+                                kSkinnyCopyMacs / nk};
     for (const long long e : edges)
         if (e >= t) end = (int)std::min<long long>(end, e);
     return end;
@@ -1898,22 +1911,22 @@ extern "C" size_t int8k_mlp_workspace_bytes(int T, int d_model, int d_ff, int fl
     if (T <= 0 || d_model <= 0 || d_ff <= 0) return 0;
     const bool prepacked = (flags & INT8K_MLP_WEIGHTS_PREPACKED) != 0;
     const MlpPlan pl = mlp_plan(T, d_model, d_ff, flags);
-    size_t need = carve_mlp(nullptr, T, d_model, d_ff, prepacked, pl).bytes;
+    // (a T on 256 x 256 tiles does not ask for the room of W2's copy, nor for shorter calls)
+    const bool copy_room = pl.g2.route != Route::kTiled;
+    size_t need = carve_mlp(nullptr, T, d_model, d_ff, prepacked, pl, copy_room).bytes;
     // Shorter calls may need more: their GEMMs split K into partials, more of them the fewer
-    // tiles there are.  (W2's copy aside, which T alone asks for or not.)  Within a range of
-    // one route and tile count a plan has fewer splits the longer the call: the range's first
-    // splits with its last rows bound it.  About 1 us a range: 128 -> 384 rows 4 ranges, 16384
-    // rows of 512 -> 2048 40.
-    const size_t copy = need - carve_mlp(nullptr, T, d_model, d_ff, true, pl).bytes;
+    // tiles there are.  Within a range of one route and tile count a plan has fewer splits the
+    // longer the call: the range's first splits with its last rows bound it.  About 1 us a
+    // range: 384 rows 7 of them, 16384 rows of 512 -> 2048 40.
     for (int t = 1; t < T;) {
         const MlpPlan first = mlp_plan(t, d_model, d_ff, flags);
-        if (first.g1.route == Route::kTiled && first.g2.route == Route::kTiled && t > kStreamRowsSmall)
+        if (first.g1.route == Route::kTiled && first.g2.route == Route::kTiled && t > kFewRows)
             break;  // and from here on: no partials, less than T needs
         const int end = std::min(plan_range_end(t, d_model, d_ff), T);
         MlpPlan last = mlp_plan(end, d_model, d_ff, flags);
         last.g1.splits = std::max(last.g1.splits, first.g1.splits);
         last.g2.splits = std::max(last.g2.splits, first.g2.splits);
-        need = std::max(need, carve_mlp(nullptr, end, d_model, d_ff, true, last).bytes + copy);
+        need = std::max(need, carve_mlp(nullptr, end, d_model, d_ff, prepacked, last, copy_room).bytes);
         t = end + 1;
     }
     return need;
@@ -1991,7 +2004,11 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
         if ((st = check_launch("rq_clear_kernel")) != INT8K_OK) return st;
     }
 
-    const int8_t* W2t = W2;
+    const int8_t *W1t = W1, *W2t = W2;
+    if (!prepacked && !pl.kn1) {
+        if ((st = launch_transpose(W1, w.w1t, d_model, d_ff, s)) != INT8K_OK) return st;
+        W1t = w.w1t;
+    }
     if (!prepacked && !pl.kn2) {
         if ((st = launch_transpose(W2, w.w2t, d_ff, d_model, s)) != INT8K_OK) return st;
         W2t = w.w2t;
@@ -2007,7 +2024,7 @@ extern "C" int int8k_mlp_forward(const int8_t* x, const int8_t* W1, const int8_t
     p1.sb_stride = n_scale_W1 == 1 ? 0 : 1;
     p1.bias = bias1;
     p1.pmax = w.p1;
-    st = run_gemm<EPI_GELU_F16>(pl.g1, pl.rq.g1, pl.direct1, pl.kn1, x, W1, T, d_ff, d_model, p1,
+    st = run_gemm<EPI_GELU_F16>(pl.g1, pl.rq.g1, pl.direct1, pl.kn1, x, W1t, T, d_ff, d_model, p1,
                                 w.hq, w.sh, amax1, arrived1, w.part, s);
     if (st != INT8K_OK) return st;
     // per-token requant of the fp16 hidden

@@ -115,10 +115,10 @@ def test_mlp_mid_tiles_vs_oracle(ext, gpu, T, dm, dff):
                  f"mid per-tensor T{T}")
 
 
-# Small GEMMs (M N K <= 2^31, K % 512 == 0) take the skinny path (32 x 32 tiles, K split
-# over the waves of a block): 1, 33 (a partial row tile), 64, 128, 200, 256, 300 rows.
-# K not a multiple of 512 takes split-K (128 x 128 tiles, K split over blocks, int32
-# partials): GEMM2 of (96, 512, 1408), both GEMMs of (128, 640, 1408).
+# Small GEMMs (K % 512 == 0) take the skinny path (32 x 32 tiles, K split over the waves of
+# a block): 1, 33 (a partial row tile), 64, 128, 200, 256, 300 rows.  K not a multiple of
+# 512 takes 128 x 128 tiles with K split over blocks (int32 partials): GEMM2 of (96, 512,
+# 1408), both GEMMs of (128, 640, 1408).
 @pytest.mark.parametrize("T,dm,dff", [(128, 1024, 4096), (64, 512, 2048), (1, 512, 1024),
                                       (33, 512, 1024), (200, 1024, 4096), (256, 512, 2048),
                                       (300, 512, 1024), (96, 512, 1408), (128, 640, 1408)])

@@ -2,7 +2,7 @@
 
 Rows around the 32- and 64-row blocks of the streaming kernel and the 128-row tiles, K and N
 off the 128 grid (the API asks for multiples of 16), K ranges that leave the last wave or split
-short or empty, the widest row of the fused epilogue (32768 columns) and one past it, both
+short or empty, small weights on the skinny kernel (as stored: through transposed copies), the widest row of the fused epilogue (32768 columns) and one past it, both
 weight layouts, bias, scalar scales and the per-tensor output.  The integer sums are exact, so
 the codes are within one of the oracle's and at most 2% of them differ (an fp32 epilogue in
 another order moves a code only on a rounding tie), as in test_mlp_gpu.py.
@@ -46,7 +46,7 @@ def _check(T, dm, dff, gpu, bias=False, scalar=False):
 
 
 @pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 128])
-@pytest.mark.parametrize("dm,dff", [(400, 1040), (1296, 2064)])
+@pytest.mark.parametrize("dm,dff", [(400, 1040), (1296, 2064), (1552, 2064)])  # 3 MiB between
 def test_stream_row_blocks(gpu, T, dm, dff):
     _check(T, dm, dff, gpu, bias=T % 2 == 1, scalar=T == 32)
 
@@ -54,7 +54,7 @@ def test_stream_row_blocks(gpu, T, dm, dff):
 @pytest.mark.parametrize("T,dm,dff", [
     (3, 16, 16), (5, 16, 4112), (2, 4112, 16), (1, 144, 128), (40, 2192, 784),
     (2, 48, 32768), (2, 48, 32784), (3, 6160, 64),
-    (200, 512, 1024), (512, 256, 1040),      # weights of at most 1 MiB: up to 512 rows
+    (32, 528, 1024), (32, 256, 1040),        # weights of at most 3 MiB: up to 32 rows
 ])
 def test_stream_edges(gpu, T, dm, dff):
     _check(T, dm, dff, gpu, bias=True)
@@ -63,9 +63,22 @@ def test_stream_edges(gpu, T, dm, dff):
 @pytest.mark.parametrize("T,dm,dff", [
     (129, 1296, 2064), (256, 2064, 784), (257, 784, 4112), (333, 1040, 4112), (513, 528, 2192),
     (640, 2048, 1536), (130, 1040, 16400),
+    (33, 16, 16), (100, 16, 4112), (64, 512, 1024), (128, 256, 1040), (300, 512, 1040),
+    (33, 528, 1040), (128, 1040, 2064),  # weights of at most 3 MiB: from 33 rows
 ])
 def test_mid_tiles_and_splits(gpu, T, dm, dff):
     _check(T, dm, dff, gpu, bias=T % 2 == 0)
+
+
+@pytest.mark.parametrize("T,dm,dff", [
+    # both GEMMs, packed; as stored through transposed copies above 128 rows to 2^28
+    # multiply-adds: the range's ends, GEMM2 alone (K = 1040 is off the kernel's grid), row tails
+    (1, 512, 512), (33, 512, 1024), (128, 512, 512), (129, 512, 512), (257, 512, 1024),
+    (1280, 512, 512), (1281, 512, 512), (200, 1024, 1024), (640, 512, 1024), (140, 1024, 96),
+    (16, 1024, 3072), (64, 1024, 3072), (140, 640, 512),
+])
+def test_skinny_with_copies(gpu, T, dm, dff):
+    _check(T, dm, dff, gpu, bias=T % 2 == 1)
 
 
 def test_stream_unaligned_scales(gpu):
