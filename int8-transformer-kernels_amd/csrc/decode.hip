@@ -41,6 +41,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "int8k_common.h"
 #include "rows.h"
@@ -274,6 +275,17 @@ __device__ __forceinline__ float load_f32(const float* p) {
     else return *p;
 }
 
+// Four scales of consecutive rows as one 16-byte load, which needs only the
+// alignment of a float.
+template <bool NT>
+__device__ __forceinline__ void load_scales4(const float* p, float* s) {
+    typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));
+    v4f v;
+    if constexpr (NT) v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p));
+    else v = *reinterpret_cast<const v4f*>(p);
+    s[0] = v.x, s[1] = v.y, s[2] = v.z, s[3] = v.w;
+}
+
 template <bool NT>
 __device__ __forceinline__ Int4 load_kv16(const int8_t* p) {
     if constexpr (NT) {
@@ -313,14 +325,15 @@ __device__ __forceinline__ float quad_bcast(float x, int t) {
 // QK^T, online softmax and PV for one wave iteration whose NSLOT rows per
 // group are loaded (kv, vv, sk, sv).  MASKED: rows outside [jlo, j1) get score -inf
 // and weight 0 (their loads point at some valid row), and sk[t] / sv[t] are slot t's
-// scales.  Otherwise lane s of a quad holds those of slots s, s + 4 in sk[0],
-// sk[1] and the quad reads them with quad_bcast.  RS: rows between slots (2 for
-// paired rows).
-template <int D, int NS, bool MASKED, int RS = 1>
+// scales, as they are unmasked without QUAD.  QUAD: lane s of a quad holds those of
+// slots s, s + 4 in sk[0], sk[1] and the quad reads them with quad_bcast.  RS: rows
+// between slots (2 for paired rows, the only ones with a jlo).
+template <int D, int NS, bool MASKED, int RS = 1, bool QUAD = true>
 __device__ __forceinline__ void decode_math(const Int4 (&kv)[NS], const Int4 (&vv)[NS],
                                             const float (&sk)[NS], const float (&sv)[NS],
                                             int row0, int j1, const Int4& q, float qscale,
                                             float& m, float& l, float* acc, int jlo = 0) {
+    constexpr bool QB = !MASKED && QUAD;
     // QK^T: exact int32 dot per row, summed over the LPR lanes of the group.
     float sc[NS];
 #pragma unroll
@@ -330,10 +343,10 @@ __device__ __forceinline__ void decode_math(const Int4 (&kv)[NS], const Int4 (&v
         d = __builtin_amdgcn_sdot4(q.z, kv[t].z, d, false);
         d = __builtin_amdgcn_sdot4(q.w, kv[t].w, d, false);
         d = group_sum<D>(d);
-        const float skt = MASKED ? sk[t] : quad_bcast(sk[t >> 2], t & 3);
+        const float skt = QB ? quad_bcast(sk[t >> 2], t & 3) : sk[t];
         sc[t] = static_cast<float>(d) * qscale * skt;
         if constexpr (MASKED) {
-            if (row0 + t * RS >= j1 || row0 + t * RS < jlo) sc[t] = -INFINITY;
+            if (row0 + t * RS >= j1 || (RS == 2 && row0 + t * RS < jlo)) sc[t] = -INFINITY;
         }
     }
 
@@ -351,9 +364,9 @@ __device__ __forceinline__ void decode_math(const Int4 (&kv)[NS], const Int4 (&v
     for (int t = 0; t < NS; ++t) {
         const float p = fast_exp2(sc[t] - m_use);
         l += p;
-        float w = p * (MASKED ? sv[t] : quad_bcast(sv[t >> 2], t & 3));
+        float w = p * (QB ? quad_bcast(sv[t >> 2], t & 3) : sv[t]);
         if constexpr (MASKED) {
-            if (row0 + t * RS >= j1 || row0 + t * RS < jlo) w = 0.f;
+            if (row0 + t * RS >= j1 || (RS == 2 && row0 + t * RS < jlo)) w = 0.f;
         }
         fma_bytes(acc + 0, vv[t].x, w);
         fma_bytes(acc + 4, vv[t].y, w);
@@ -372,8 +385,12 @@ struct IterBuf {
 };
 
 // The loads of an unmasked wave iteration whose group rows start at row0 and
-// lie RS rows apart.
-template <int D, int NS, int FL, int RS = 1>
+// lie RS rows apart.  QUAD: one scale per lane and 4 slots (see decode_math).  The
+// contiguous kernels load consecutive rows' scales as vectors instead: the 16 quad
+// reads of an iteration at D = 128 show where a CU has few waves (one chunk of 5000
+// rows 69.3 -> 66.9 us, B6 H32 D128 2048 rows 17.2 -> 16.6; the paged D = 128 kernel,
+// whose scales are 8 rows of one page, is 1-2% faster with them).
+template <int D, int NS, int FL, int RS, bool QUAD>
 __device__ __forceinline__ void load_iter(IterBuf<NS>& b, const int8_t* __restrict__ Kbh,
                                           const int8_t* __restrict__ Vbh,
                                           const float* __restrict__ sKbh,
@@ -384,17 +401,26 @@ __device__ __forceinline__ void load_iter(IterBuf<NS>& b, const int8_t* __restri
     for (int t = 0; t < NS; ++t) b.kv[t] = load_kv16<(FL & kNtKV) != 0>(kp + t * RS * D);
 #pragma unroll
     for (int t = 0; t < NS; ++t) b.vv[t] = load_kv16<(FL & kNtKV) != 0>(vp + t * RS * D);
+    if constexpr (QUAD) {
 #pragma unroll
-    for (int i = 0; i < NS / 4; ++i) {
-        const size_t r = row0 + RS * ((sub & 3) + 4 * i);
-        b.sk[i] = load_f32<(FL & kNtScales) != 0>(sKbh + r);
-        b.sv[i] = load_f32<(FL & kNtScales) != 0>(sVbh + r);
+        for (int i = 0; i < NS / 4; ++i) {
+            const size_t r = row0 + RS * ((sub & 3) + 4 * i);
+            b.sk[i] = load_f32<(FL & kNtScales) != 0>(sKbh + r);
+            b.sv[i] = load_f32<(FL & kNtScales) != 0>(sVbh + r);
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < NS; t += 4) {
+            load_scales4<(FL & kNtScales) != 0>(sKbh + row0 + t, &b.sk[t]);
+            load_scales4<(FL & kNtScales) != 0>(sVbh + row0 + t, &b.sv[t]);
+        }
     }
 }
 
 // A partial wave iteration: rows outside [jlo, j1) get score -inf and weight 0
 // (their loads are redirected to a row inside).  RS: rows between slots (2 for
-// paired rows).
+// paired rows; jlo is 0 for the others).  What the scores need is loaded before V,
+// and all of it before the math (B519 D128 300 rows 17.9 -> 15.7 us).
 template <int D, int NS, int FL, int RS = 1>
 __device__ __forceinline__ void decode_tail(
     const int8_t* __restrict__ Kbh, const int8_t* __restrict__ Vbh,
@@ -404,12 +430,17 @@ __device__ __forceinline__ void decode_tail(
     IterBuf<NS> b;
 #pragma unroll
     for (int t = 0; t < NS; ++t) {
-        const int r = max(min(row0 + t * RS, j1 - 1), jlo);
+        const int r = RS == 2 ? max(min(row0 + t * RS, j1 - 1), jlo) : min(row0 + t * RS, j1 - 1);
         b.kv[t] = load_kv16<(FL & kNtKV) != 0>(Kbh + (size_t)r * D + sub * 16);
-        b.vv[t] = load_kv16<(FL & kNtKV) != 0>(Vbh + (size_t)r * D + sub * 16);
         b.sk[t] = load_f32<(FL & kNtScales) != 0>(sKbh + r);
+    }
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+        const int r = RS == 2 ? max(min(row0 + t * RS, j1 - 1), jlo) : min(row0 + t * RS, j1 - 1);
+        b.vv[t] = load_kv16<(FL & kNtKV) != 0>(Vbh + (size_t)r * D + sub * 16);
         b.sv[t] = load_f32<(FL & kNtScales) != 0>(sVbh + r);
     }
+    __builtin_amdgcn_sched_barrier(0);
     decode_math<D, NS, true, RS>(b.kv, b.vv, b.sk, b.sv, row0, j1, q, qscale, m, l, acc, jlo);
 }
 
@@ -557,7 +588,7 @@ __global__ __launch_bounds__(kBlockThreads) void decode_combine_kernel(
 // group's first row in iteration i; RS: rows between its slots.  PIPE: two
 // register sets, iteration k+1's loads issued before iteration k is computed
 // (the fences keep the compiler from sinking them).
-template <int D, int NS, int FL, bool PIPE, int RS, typename RowOff>
+template <int D, int NS, int FL, bool PIPE, int RS, bool QUAD, typename RowOff>
 __device__ __forceinline__ void walk_iters(const int8_t* __restrict__ K,
                                            const int8_t* __restrict__ V,
                                            const float* __restrict__ sK,
@@ -566,10 +597,10 @@ __device__ __forceinline__ void walk_iters(const int8_t* __restrict__ K,
                                            float& l, float* acc) {
     auto nxt = [&](int i) { return (i + 1 == n_full) ? 0 : i + 1; };
     auto load = [&](IterBuf<NS>& b, int i) {
-        load_iter<D, NS, FL, RS>(b, K, V, sK, sV, roff(i), sub);
+        load_iter<D, NS, FL, RS, QUAD>(b, K, V, sK, sV, roff(i), sub);
     };
     auto math = [&](const IterBuf<NS>& b) {
-        decode_math<D, NS, false, RS>(b.kv, b.vv, b.sk, b.sv, 0, 0, q, qscale, m, l, acc);
+        decode_math<D, NS, false, RS, QUAD>(b.kv, b.vv, b.sk, b.sv, 0, 0, q, qscale, m, l, acc);
     };
     if constexpr (PIPE) {
         IterBuf<NS> ba, bb;
@@ -635,43 +666,47 @@ __device__ __forceinline__ void merge_block(float m, float l, float* acc, int la
             s_ml[w][1] = Lw;
         }
     }
-    constexpr int DPL = D / 64;
-    // chunks past nw are empty states (not another chunk's with weight 0: it may hold
-    // infinities)
-    for (int c = nw + w; c < MAXW; c += nw) {
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) s_acc[c][lane * DPL + i] = 0.f;
-        if (lane == 0) {
-            s_ml[c][0] = -INFINITY;
-            s_ml[c][1] = 0.f;
-        }
-    }
     __syncthreads();
     if (w != 0) return;
-    // unrolled, so that the LDS reads of all chunks go out together
-    float mc[MAXW], lc[MAXW], oc[MAXW][DPL];
+    constexpr int DPL = D / 64;
+    // The reads are unrolled, so that those of all chunks go out together.  A shorter
+    // sequence has fewer chunks; the absent ones are empty states (another chunk's with
+    // weight 0 may hold infinities), set in registers: left in LDS by the waves they cost
+    // a one-chunk block 0.2 us, and a loop over the chunks 0.2 us at five (300 rows).
+    float Mall, L = 0.f, o[DPL];
+    auto merge = [&](auto full) {
+        constexpr int N = decltype(full)::value ? MAXW : MAXW - 1;
+        float mc[N], lc[N], oc[N][DPL];
 #pragma unroll
-    for (int c = 0; c < MAXW; ++c) {
-        mc[c] = s_ml[c][0];
-        lc[c] = s_ml[c][1];
+        for (int c = 0; c < N; ++c) {
+            mc[c] = -INFINITY, lc[c] = 0.f;
 #pragma unroll
-        for (int i = 0; i < DPL; ++i) oc[c][i] = s_acc[c][lane * DPL + i];
-    }
-    float Mall = mc[0];
+            for (int i = 0; i < DPL; ++i) oc[c][i] = 0.f;
+        }
 #pragma unroll
-    for (int c = 1; c < MAXW; ++c) Mall = fmaxf(Mall, mc[c]);
-    const float M_use = (Mall == -INFINITY) ? 0.f : Mall;
-    float L = 0.f;
-    float o[DPL];
+        for (int c = 0; c < N; ++c) {
+            if (!decltype(full)::value && c >= nw) break;
+            mc[c] = s_ml[c][0];
+            lc[c] = s_ml[c][1];
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) o[i] = 0.f;
+            for (int i = 0; i < DPL; ++i) oc[c][i] = s_acc[c][lane * DPL + i];
+        }
+        Mall = mc[0];
 #pragma unroll
-    for (int c = 0; c < MAXW; ++c) {
-        const float wt = fast_exp2(mc[c] - M_use);
-        L += lc[c] * wt;
+        for (int c = 1; c < N; ++c) Mall = fmaxf(Mall, mc[c]);
+        const float M_use = (Mall == -INFINITY) ? 0.f : Mall;
 #pragma unroll
-        for (int i = 0; i < DPL; ++i) o[i] = fmaf(oc[c][i], wt, o[i]);
-    }
+        for (int i = 0; i < DPL; ++i) o[i] = 0.f;
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            const float wt = fast_exp2(mc[c] - M_use);
+            L += lc[c] * wt;
+#pragma unroll
+            for (int i = 0; i < DPL; ++i) o[i] = fmaf(oc[c][i], wt, o[i]);
+        }
+    };
+    if (nw == MAXW) merge(std::true_type{});
+    else merge(std::false_type{});
     if (part_ml != nullptr) {
 #pragma unroll
         for (int i = 0; i < DPL; ++i) part_acc[(size_t)bh * D + lane * DPL + i] = o[i];
@@ -693,7 +728,7 @@ __device__ __forceinline__ void merge_block(float m, float l, float* acc, int la
 // The 8-wave instance has twice the registers per wave, which lets it keep the
 // next iteration's loads in flight (a second register set, two_sets) while the
 // current one computes: at 4 slots a short chunk is only a few dependent load
-// rounds, so their latency would show; at D = 128 with 8 slots (184 VGPRs, two
+// rounds, so their latency would show; at D = 128 with 8 slots (204 VGPRs, two
 // waves per SIMD) the stream then runs at fewer waves per CU with the same
 // bytes in flight, which the HBM read rate prefers.
 //
@@ -754,7 +789,7 @@ __global__ __launch_bounds__(64 * MAXW) void decode_block_kernel(
     const unsigned unit = blockIdx.x * (unsigned)nw + (unsigned)w;
     const int it = stagger ? (int)((unit * 2654435761u) >> 16) % max(n_full, 1) : 0;
     const int jf = j0 + head;
-    walk_iters<D, NS, FL, two_sets(D, NS, MAXW), RS>(
+    walk_iters<D, NS, FL, two_sets(D, NS, MAXW), RS, PAIRED>(
         Kbh, Vbh, sKbh, sVbh, [&](int i) { return (size_t)(jf + i * G::kRowsPerIter + g0); },
         n_full, it, sub, q, qscale_l, m, l, acc);
     // partial iterations: the end of the chunk, and the head
@@ -850,7 +885,7 @@ __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
     constexpr bool PAIRED = paired_rows(D, NS, MAXW);
     constexpr int RS = PAIRED ? 2 : 1;
     const int g0 = group_row0<PAIRED, NS>(grp);
-    walk_iters<D, NS, FL, two_sets(D, NS, MAXW), RS>(
+    walk_iters<D, NS, FL, two_sets(D, NS, MAXW), RS, true>(
         Kp, Vp, sKp, sVp, [&](int i) { return row_off(j0 + i * G::kRowsPerIter + g0); },
         n_full, it, sub, q, qscale_l, m, l, acc);
     const int base = j0 + n_full * G::kRowsPerIter;
@@ -861,10 +896,15 @@ __global__ __launch_bounds__(64 * MAXW) void decode_paged_block_kernel(
         for (int t = 0; t < NS; ++t) {
             const size_t r = row_off(min(row0 + t * RS, j1 - 1));
             bt.kv[t] = load_kv16<(FL & kNtKV) != 0>(Kp + r * D + sub * 16);
-            bt.vv[t] = load_kv16<(FL & kNtKV) != 0>(Vp + r * D + sub * 16);
             bt.sk[t] = load_f32<(FL & kNtScales) != 0>(sKp + r);
+        }
+#pragma unroll
+        for (int t = 0; t < NS; ++t) {
+            const size_t r = row_off(min(row0 + t * RS, j1 - 1));
+            bt.vv[t] = load_kv16<(FL & kNtKV) != 0>(Vp + r * D + sub * 16);
             bt.sv[t] = load_f32<(FL & kNtScales) != 0>(sVp + r);
         }
+        __builtin_amdgcn_sched_barrier(0);
         decode_math<D, NS, true, RS>(bt.kv, bt.vv, bt.sk, bt.sv, row0, j1, q, qscale_l, m, l,
                                      acc);
     }
@@ -930,7 +970,7 @@ __global__ __launch_bounds__(kBlockThreads) void decode_paged_kernel(
         it = (it + 1 == n_full) ? 0 : it + 1;
         if (k + 1 < n_full) r_next = row_off(j0 + it * G::kRowsPerIter + grp * NS);
         IterBuf<NS> b;
-        load_iter<D, NS, FL>(b, Kp, Vp, sKp, sVp, r0, sub);
+        load_iter<D, NS, FL, 1, true>(b, Kp, Vp, sKp, sVp, r0, sub);
         decode_math<D, NS, false>(b.kv, b.vv, b.sk, b.sv, 0, 0, q, qscale, m, l, acc);
     }
     const int base = j0 + n_full * G::kRowsPerIter;
