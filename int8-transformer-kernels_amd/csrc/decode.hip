@@ -1086,8 +1086,16 @@ int launch_decode_paged(const int8_t* Q, const int8_t* Kp, const int8_t* Vp, con
         g = plan.g;
     else
         g = plan_groups(BH, max_context, D, NS, plan.nsplit);
-    // short chunks keep the plan's waves: more of them only add merges
-    if (g.blocks == 1 && one_launch && plan.chunk <= 4 * rows_per_iter(D, NS))
+    // Short chunks keep the plan's waves: more of them only add merges, and blocks where
+    // the (b,h) fill the GPU (page 64, ragged: B32 H32 D64 1000 rows 15.9 us on the
+    // plan's 2 waves and 20.1 on 8, B20 H32 1500 rows 16.6 and 20.5 on 4 and 8, B64 H32
+    // D128 1500 rows 80 and 89 on 4 and 8).  Past about 32 iterations, or 128 / waves,
+    // 8 waves are the faster (B24 H16 D64 2048 rows 19.1 us on 6, 18.3 on 8; B20 H32 4000
+    // rows 40.5 on 4, 36.2 on 8).
+    const long long iters = ceil_div(max_context, rows_per_iter(D, NS));
+    if (g.blocks == 1 && one_launch &&
+        (plan.chunk <= 4 * rows_per_iter(D, NS) ||
+         (iters <= 4 * kGroupWaves && iters * plan.nsplit <= 16 * kGroupWaves)))
         g = GroupPlan{1, plan.nsplit, plan.chunk};
     // page ids the rows of a block can span, staged in LDS
     const long long rows = (long long)g.waves * g.chunk;

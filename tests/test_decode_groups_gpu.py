@@ -103,3 +103,29 @@ def test_grouped_paged_plans_match_float64(gpu, D, page, lens):
                         Ki=flat["K_pages"][None], Vi=flat["V_pages"][None],
                         sK=flat["sK_pages"][None, ..., 0], sV=flat["sV_pages"][None, ..., 0]), n)
         assert_attn_close(o, ref[0], f"paged D{D} page{page} len{n}")
+
+
+@pytest.mark.parametrize("D,H,page,longest", [(64, 32, 64, 600), (64, 64, 16, 1025),
+                                              (128, 64, 64, 1300)])
+def test_paged_plans_of_few_waves_match_float64(gpu, D, H, page, longest):
+    # enough (b,h) for the GPU: the plan's one to four waves per (b,h), not eight
+    lens = [longest, 1, 63, 64, 65, 0, longest - 1, longest // 2] * 4
+    B = len(lens)
+    assert 1 <= capi.decode_num_splits(B * H, longest, D) <= 4
+    c = workloads.paged_case(B, H, D, page, lens, seed=D + H, device=gpu)
+    out = capi.decode_attention_paged(c["Qi"], c["K_pages"], c["V_pages"], c["sQ"],
+                                      c["sK_pages"], c["sV_pages"], c["block_tables"],
+                                      c["context_lens"], c["max_context"])
+    torch.cuda.synchronize()
+    for b in list(range(8)) + [B - 2]:
+        o, n = out[b].float().cpu().numpy(), lens[b]
+        if n == 0:
+            assert np.all(o == 0)
+            continue
+        t = c["block_tables"][b, :-(-n // page)].long()
+        flat = {k: c[k][t].transpose(0, 1).reshape(H, len(t) * page, -1)[:, :n]
+                for k in ("K_pages", "V_pages", "sK_pages", "sV_pages")}
+        ref = _ref(dict(Qi=c["Qi"][b:b + 1], sQ=c["sQ"].reshape(B, H)[b:b + 1],
+                        Ki=flat["K_pages"][None], Vi=flat["V_pages"][None],
+                        sK=flat["sK_pages"][None, ..., 0], sV=flat["sV_pages"][None, ..., 0]), n)
+        assert_attn_close(o, ref[0], f"paged D{D} H{H} page{page} len{n}")
