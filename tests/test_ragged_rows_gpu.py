@@ -29,6 +29,29 @@ def test_quantize_rows(gpu, dtype, cols):
     np.testing.assert_array_equal(s.cpu().numpy(), rs)
 
 
+@pytest.mark.parametrize("cols,dtype", [(24, torch.float16), (512, torch.float16),
+                                        (768, torch.float16), (100, torch.float32)])
+@pytest.mark.parametrize("groups", [1, 4095, 4096, 4097, 16385, 32769])
+def test_quantize_row_groups(gpu, cols, dtype, groups):
+    # waves of one row group (as many rows as fill 64 lanes) up to 4 x 1024 waves, of up to
+    # four groups beyond, some of them past the end
+    chunks = cols * dtype.itemsize // 16
+    per = 64 >> min(6, (chunks - 1).bit_length())
+    rows = groups * per - (per > 1)
+    x = (torch.randn(rows, cols, device=gpu, generator=torch.Generator(gpu).manual_seed(rows))
+         * 3).to(dtype)
+    q, s = capi.quantize_per_token(x)
+    torch.cuda.synchronize()
+    at = sorted({i for n in (0, rows // 4, rows // 2, rows - 33) for i in range(n, n + 33)
+                 if 0 <= i < rows})
+    rq, rs = O.quantize_per_token(x[at].float().cpu().numpy())
+    np.testing.assert_array_equal(q[at].cpu().numpy(), rq)
+    np.testing.assert_array_equal(s[at].cpu().numpy(), rs)
+    # every row: codes times scale within half a step, on the GPU
+    d = (q.float() * s.unsqueeze(-1) - x.float()).abs().amax(-1)
+    assert bool((d <= s * (0.5 + 1e-4)).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("cols", COLS)
 @pytest.mark.parametrize("rows,shift", [(67, 0), (1100, 0), (3, 1)])
