@@ -72,7 +72,8 @@ constexpr long long kMaxBlocks = 1LL << 20;
 constexpr long long kVecBlocks = 8192;
 
 // LayerNorm keeps gamma and beta in registers over a wave's rows: a grid of 4
-// blocks per CU, so that many rows share one read of them.
+// blocks per CU, so that many rows share one read of them.  Without either the
+// rows spread over more blocks (fp32 30000 x 512 16.9 -> 14.8 us, 100000 x 256 36.3 -> 29.0).
 constexpr long long kLnBlocks = 1024;
 // Elements per lane of the longest row of layernorm_quant_row_kernel (768 columns).
 // One wave per row loses from 1280 columns on, where a block per row loads more in
@@ -468,7 +469,8 @@ extern "C" int int8k_layernorm_quantize_per_token(const void* x, int dtype, cons
     if (fills && rows < (1LL << 31) && aligned_to(x, 16) && aligned_to(q, w) &&
         (!y_out || aligned_to(y_out, 16))) {
         const long long waves = ceil_div(rows, 64 >> sh.lg);
-        const unsigned blocks = (unsigned)std::min(ceil_div(waves, 4), kLnBlocks);
+        const unsigned blocks =
+            (unsigned)std::min(ceil_div(waves, 4), gamma || beta ? kLnBlocks : kVecBlocks);
         const int affine_vec =
             (!gamma || aligned_to(gamma, 16)) && (!beta || aligned_to(beta, 16));
         with_dtype(dtype, [&](auto dt) {
