@@ -176,6 +176,8 @@ DecodeTuning tuning_for(int D) {
 
 constexpr int kNumCus = 256;
 
+constexpr long long kChunkAlias = 512 << 10;  // bytes (see plan_groups)
+
 // Most blocks per (b,h) of an automatic plan: 8, or one for each CU.
 inline long long most_groups(int BH, long long iters) {
     return std::min(ceil_div(iters, kGroupWaves), std::max(8LL, (long long)kNumCus / BH));
@@ -194,6 +196,10 @@ inline long long most_groups(int BH, long long iters) {
 // within 3% of it (B2 H8 D128 60013 rows: 53.2 / 44.1 / 46.0 us at 8 / 16 / 32
 // blocks; B1 H32 D64 128K: 103 / 87 / 88 us at 4 / 8 / 16): a partial extra round
 // leaves CUs idle, and fewer blocks than CUs read at a CU's ~55 GB/s each.
+// Chunks of whole multiples of 512 KB cost an eighth more: their waves read slower than
+// those of other lengths, probably in step on the same HBM channels (B8 H32 D128 on one
+// block: 6.7 TB/s at 32000 and 33001 rows, 6.2 at 32768, and 6.6 on two blocks: 343 -> 322
+// us; B2 H32 131072 rows on 4 and 8 blocks 350 -> 321, B4 H32 65536 on 2 and 4 350 -> 320).
 GroupPlan plan_groups(int BH, int S, int D, int slots, long long most) {
     const int R = rows_per_iter(D, slots);
     const long long iters = ceil_div(S, R);
@@ -203,7 +209,8 @@ GroupPlan plan_groups(int BH, int S, int D, int slots, long long most) {
         const long long pw = ceil_div(iters, nb * kGroupWaves);
         const long long bl = ceil_div(iters, pw * kGroupWaves);
         const long long rounds = ceil_div(BH * bl, kNumCus);
-        const long long cost = 2 * rounds * (pw + 2) + (bl > 1 ? (D == 128 ? 4 : 8) : 0);
+        long long cost = 2 * rounds * (pw + 2) + (bl > 1 ? (D == 128 ? 4 : 8) : 0);
+        if (pw * R * D % kChunkAlias == 0) cost += cost / 8;
         if (best < 0 || cost < best) best = cost, per_wave = pw, blocks = bl;
     }
     const int waves = (int)std::min<long long>(kGroupWaves, ceil_div(iters, per_wave));
