@@ -253,7 +253,10 @@ __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
 #pragma unroll
             for (int e = 0; e < W; ++e) sum += real(i) ? v[e] : 0.f;
         }
-        const float mean = row_reduce(sum, lg, add) * inv_cols;
+        float mean = row_reduce(sum, lg, add) * inv_cols;
+        // rounded here: the compiler fused the product into x - mean of the variance alone in
+        // some instances, which left the error of 1 / cols in every deviation
+        asm("" : "+v"(mean));
 #pragma unroll
         for (int i = 0; i < NC; ++i) reload_barrier(w[i]);
         float var = 0.f;

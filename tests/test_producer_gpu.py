@@ -101,3 +101,21 @@ def test_quantize_heads_feeds_attention(ext, gpu):
     out = ext.int8_attention_forward(qi, ki, vi, sq, sk, sv, True)
     torch.cuda.synchronize()
     assert out.shape == (B, H, S, Dh) and torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("cols", [256, 768, 1024, 1280, 1536, 1792, 2304, 2816, 3072, 3584, 4096])
+def test_mean_is_rounded_before_it_is_subtracted(gpu, cols):
+    # 1 + h, 1 - h in turn: the fp32 sums over a lane's columns and over the row are exact, and
+    # sum * (1 / cols) rounds to 1, so the deviations are h, the variance h^2 and y = +-1.  With
+    # that product fused into x - mean the error of 1 / cols (2^-29 and more) stays in every
+    # deviation of the variance and moves y by 2^-24 and more.
+    h = 2.0 ** -17
+    inv = np.float32(1) / np.float32(cols)
+    assert np.float32(cols) * inv == 1
+    sign = torch.ones(3, cols)
+    sign[:, 1::2] = -1
+    q, s, y = capi.layernorm_quantize_per_token((1 + h * sign).to(gpu), None, None, 0.0,
+                                                want_y=True)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(y.cpu().numpy(), sign.numpy())
+    np.testing.assert_array_equal(q.cpu().numpy(), 127 * sign.numpy())
