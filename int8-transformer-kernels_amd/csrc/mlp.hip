@@ -1193,10 +1193,11 @@ constexpr int kMidMaxBigTiles = 128;
 //    skinny / streaming: T = 16 17.9 / 16.1, T = 64 20.8 / 19.8, T = 128 22.9 / 22.1; K =
 //    3072: T = 16 16.3 / 15.4, T = 64 18.2 / 19.1), but for a per-tensor output, which takes
 //    a pass more behind partials (K = 3072, T = 16 16.9 / 18.0; K = 4096 18.3 / 18.4);
-//  - weights as stored are transposed for it above 128 rows, to 5/4 2^28 multiply-adds
+//  - weights as stored are transposed for it above 128 rows and below 2^29 multiply-adds
 //    (transposes + skinny / streaming / 128 x 128 tiles: 512 -> 512, T = 512 17.4 / 21.4 /
-//    19.0; 1024 -> 1024, T = 256 19.8 / 22.5 / 21.1, T = 384 23.8 / 23.5 / 23.5; 512 -> 2048,
-//    T = 320 23.3 / 25.7 on tiles), in whole transposing tiles (1024 -> 96, T = 320 32.9
+//    19.0; 1024 -> 1024, T = 256 19.8 / 22.5 / 21.1, T = 384 23.8 / 23.5 / 23.5, T = 512
+//    24.7 / - / 24.1; 512 -> 2048, T = 333 23.0 / - / 26.2, T = 500 24.9 / - / 26.7, T = 512
+//    25.7 / - / 24.9), in whole transposing tiles (1024 -> 96, T = 320 32.9
 //    against 18.3 on 128 x 128 tiles);
 //  - up to 128 rows the weights' read is the time and the streaming kernel takes it:
 //    4096 -> 16384, T = 32: 62 (skinny) -> 48, as stored 109 (transposes + skinny) ->
@@ -1208,7 +1209,7 @@ constexpr int kMidMaxBigTiles = 128;
 //    45.6; T = 512, 1024 -> 4096 43 (skinny) -> 30; T = 512, 4096 -> 16384 172 -> 107.
 constexpr int kStreamRows = 128, kStreamRowsSmall = 32, kFewRows = 512;
 constexpr long long kStreamSmallWeights = 3LL << 20, kSkinnyWeights = 1LL << 22;
-constexpr long long kSkinnyMacs = 1LL << 30, kSkinnyCopyMacs = 5LL << 26;
+constexpr long long kSkinnyMacs = 1LL << 30, kSkinnyCopyMacs = (1LL << 29) - 1;
 
 enum class Route { kStream, kSkinny, kMid, kTiled };
 

@@ -2,10 +2,11 @@
 
 Rows around the 32- and 64-row blocks of the streaming kernel and the 128-row tiles, K and N
 off the 128 grid (the API asks for multiples of 16), K ranges that leave the last wave or split
-short or empty, small weights on the skinny kernel (as stored: through transposed copies), the widest row of the fused epilogue (32768 columns) and one past it, both
-weight layouts, bias, scalar scales and the per-tensor output.  The integer sums are exact, so
-the codes are within one of the oracle's and at most 2% of them differ (an fp32 epilogue in
-another order moves a code only on a rounding tie), as in test_mlp_gpu.py.
+short or empty, small weights on the skinny kernel (as stored: through transposed copies), the
+widest row of the fused epilogue (32768 columns) and one past it, both weight layouts, bias,
+scalar scales and the per-tensor output.  The integer sums are exact, so the codes are within
+one of the oracle's and at most 2% of them differ (an fp32 epilogue in another order moves a
+code only on a rounding tie), as in test_mlp_gpu.py.
 """
 import numpy as np
 import pytest
@@ -71,10 +72,10 @@ def test_mid_tiles_and_splits(gpu, T, dm, dff):
 
 
 @pytest.mark.parametrize("T,dm,dff", [
-    # both GEMMs, packed; as stored through transposed copies above 128 rows to 2^28
+    # both GEMMs, packed; as stored through transposed copies above 128 rows, below 2^29
     # multiply-adds: the range's ends, GEMM2 alone (K = 1040 is off the kernel's grid), row tails
     (1, 512, 512), (33, 512, 1024), (128, 512, 512), (129, 512, 512), (257, 512, 1024),
-    (1280, 512, 512), (1281, 512, 512), (200, 1024, 1024), (640, 512, 1024), (140, 1024, 96),
+    (1280, 512, 512), (2047, 512, 512), (2048, 512, 512), (511, 512, 2048), (200, 1024, 1024), (640, 512, 1024), (140, 1024, 96),
     (16, 1024, 3072), (64, 1024, 3072), (140, 640, 512),
 ])
 def test_skinny_with_copies(gpu, T, dm, dff):
