@@ -31,9 +31,10 @@
 // gemm_i8_stream_kernel streams them in either layout over all CUs, the K range
 // split over waves and blocks; rows_epilogue_kernel<EPI> then sums the exact int32
 // partials of a row, applies the epilogue and requantizes it.  Small GEMMs run
-// gemm_i8_skinny_kernel (32 x 32 tiles, packed weights or transposed copies).  Between those and 128 big tiles,
-// gemm_i8_mid_kernel<EPI> runs 128 x 128 tiles, two blocks per CU, with the fp16
-// epilogue or, where the grid leaves CUs idle, split over K into the same partials.
+// gemm_i8_skinny_kernel (32 x 32 tiles, packed weights or transposed copies).
+// Between those and 128 big tiles, gemm_i8_mid_kernel<EPI> runs 128 x 128 tiles, two
+// blocks per CU, with the fp16 epilogue or, where the grid leaves CUs idle, split over
+// K into the same partials.
 // gemm_route and mid_plan choose.  The integer sums and the epilogue's expressions
 // are the same on every path: fp32 values, rounded to fp16 as such (f16_of_f32 where the
 // compiler would round the last product once, v_fma_mixlo_f16).
@@ -839,10 +840,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_i8_a16_kernel(
 // is the read of the weights (4096 -> 16384 as stored, 32 rows: 17.5 us per GEMM of 64
 // MiB, 3.8 TB/s, of which ~5 us are the first loads, the merge and the stores).  A wave
 // owns 128 columns over its own range of K and streams 128 x 128-byte weight tiles
-// through its own piece of LDS: 16 loads of 16 bytes per lane in flight, each covering whole 128-byte runs (8 weight rows
-// per instruction) for both layouts, the next tile's loads issued before the
-// current one's MFMAs, no block barrier in the loop.  Fragments come from LDS as
-// in the tiled kernels: 16-byte reads of [N][K] rows, or transposing reads of
+// through its own piece of LDS: 16 loads of 16 bytes per lane in flight, each
+// covering whole 128-byte runs (8 weight rows per instruction) for both layouts, the
+// next tile's loads issued before the current one's MFMAs, no block barrier in the
+// loop.  Fragments come from LDS as in the tiled kernels: 16-byte reads of [N][K] rows, or transposing reads of
 // [K][N] rows (BKN), so weights as stored need no transpose.  A's fragments are
 // read from global memory (L2) into registers one step ahead.  The waves of a
 // block meet in LDS, and the block writes exact int32 partials P[split][M][N],

@@ -75,9 +75,12 @@ constexpr long long kVecBlocks = 8192;
 // blocks per CU, so that many rows share one read of them.  Without either the
 // rows spread over more blocks (fp32 30000 x 512 16.9 -> 14.8 us, 100000 x 256 36.3 -> 29.0).
 constexpr long long kLnBlocks = 1024;
-// Elements per lane of the longest row of layernorm_quant_row_kernel (768 columns).
-// One wave per row loses from 1280 columns on, where a block per row loads more in
-// parallel: 4000 rows fp16, block -> wave: 24.2 -> 26.1 us at 1280, 31.0 -> 42.1 at 1600.
+// Elements per lane of the longest row of layernorm_quant_row_kernel (768 columns).  The
+// whole range below gains on a block per row, with gamma and beta: 4000 rows fp16, block ->
+// wave: 320 columns 11.4 -> 6.1 us, 520 15.0 -> 6.7, 768 16.4 -> 7.3; 7 rows 5.1 -> 3.3 and
+// 6.3 -> 3.5.  Rows up to 1280 would too, on an instance of 20 elements (776 18.4 -> 9.6,
+// 960 19.5 -> 9.8, 1280 23.5 -> 10.4), which costs the shorter rows a third if they share it
+// (768 columns 9.4 us): there is none yet.
 constexpr int kRowElems = 12;
 
 template <typename Op>
@@ -324,8 +327,8 @@ __global__ __launch_bounds__(256) void layernorm_quant_vec_kernel(
 // 64 columns (NE of them).  The sums keep the order of layernorm_quant_kernel, whose
 // thread t + 64 w is this lane's column group w modulo 4, so both give the same
 // bytes: a code on a rounding tie follows the last bit of mean and rstd.  One read of
-// x instead of five.  Against a block per row, launches included: 100000 x 80 fp16
-// 155 -> 46 us, 4000 x 768 bf16 15.3 -> 13.5 us (gamma and beta then read after the sums).
+// x instead of five.  Against a block per row: 100000 x 80 fp16 155 -> 46 us, 4000 x 768
+// 16.4 -> 7.3 (bound by the latency of the row's loads and reductions; kRowElems).
 template <int DT, int NE>
 __global__ __launch_bounds__(256) void layernorm_quant_row_kernel(
     const void* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
@@ -346,8 +349,8 @@ __global__ __launch_bounds__(256) void layernorm_quant_row_kernel(
         float v[NE];
 #pragma unroll
         for (int k = 0; k < NE; ++k) v[k] = load_any(x, base + min(lane + 64 * k, cols - 1), DT);
-        // gamma and beta in flight beside x: behind the sums each was a round trip to L2 of its
-        // own (4000 x 768 bf16 with the block's other quantizers: 33.1 -> 28.8 us)
+        // gamma and beta in flight beside x: behind the sums each was a round trip to L2 of
+        // its own (4.3 us of 4000 x 768 bf16)
         float eg[NE], eb[NE];
 #pragma unroll
         for (int k = 0; k < NE; ++k) {
@@ -378,7 +381,7 @@ __global__ __launch_bounds__(256) void layernorm_quant_row_kernel(
         }
         const float sc =
             fmaxf(row_reduce(m, 6, [](float a, float b) { return fmaxf(a, b); }), 1e-8f) / 127.f;
-        const float inv = 1.f / sc;  // one division per row, not per element: 28.8 -> 28.1 us there
+        const float inv = 1.f / sc;  // one division per row, not per element (0.7 us there)
 #pragma unroll
         for (int k = 0; k < NE; ++k) {
             const int c = lane + 64 * k;
